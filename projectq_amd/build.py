@@ -42,7 +42,24 @@ FLAGS = [
     "-Wno-unused-command-line-argument",
 ]
 
-SOURCES = ["kernels.hip", "mlp.hip", "compare.hip", "noalloc.hip", "mfma.hip", "batch_energy.hip", "engine.cpp", "planner.cpp", "batch.cpp", "capi.cpp"]
+# longest first: the tile kernels compile for minutes
+SOURCES = [
+    "tile_c64_rb5.hip",
+    "tile_c128_rb5.hip",
+    "tile_pf.hip",
+    "tile_c64_rb4.hip",
+    "tile_c128_rb4.hip",
+    "kernels.hip",
+    "mlp.hip",
+    "compare.hip",
+    "noalloc.hip",
+    "mfma.hip",
+    "batch_energy.hip",
+    "engine.cpp",
+    "planner.cpp",
+    "batch.cpp",
+    "capi.cpp",
+]
 
 
 def _compile(src):

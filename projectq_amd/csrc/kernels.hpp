@@ -1,4 +1,4 @@
-// Launchers of the HIP kernels (kernels.hip).  All take the simulator's stream; none
+// Launchers of the HIP kernels (kernels.hip, tile_*.hip).  All take the simulator's stream; none
 // synchronises.  Index conventions: amplitude index bit p belongs to the qubit at position p.
 #pragma once
 
