@@ -50,4 +50,8 @@ struct Amp<float> {
 template <typename R>
 using amp_t = typename Amp<R>::type;
 
+namespace dev {
+constexpr int kBlock = 256;  // threads per workgroup (4 wave64)
+}  // namespace dev
+
 }  // namespace qs

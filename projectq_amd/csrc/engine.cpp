@@ -101,7 +101,6 @@ Engine::Engine(uint32_t seed, int precision, int fusion_mode, int planner, unsig
   }
   QS_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
   QS_HIP(hipMalloc(&d_partials_, sizeof(double) * 2 * dev::kReduceGrid));
-  QS_HIP(hipMalloc(&d_result_, sizeof(double) * 4));
   QS_HIP(hipHostMalloc((void **)&h_result_, sizeof(double) * 4, hipHostMallocDefault));
   QS_HIP(hipMalloc(&d_flags_, sizeof(int) * 4));
   QS_HIP(hipHostMalloc((void **)&h_flags_, sizeof(int) * 4, hipHostMallocDefault));
@@ -134,7 +133,6 @@ Engine::~Engine() {
   (void)hipFree(psi_);
   release_scratch();
   (void)hipFree(d_partials_);
-  (void)hipFree(d_result_);
   (void)hipHostFree(h_result_);
   (void)hipFree(d_flags_);
   (void)hipHostFree(h_flags_);
@@ -191,9 +189,9 @@ const void *Engine::upload(const void *host, size_t bytes) {
 
 void Engine::sync() { QS_HIP(hipStreamSynchronize(stream_)); }
 
+// The sums go straight to the pinned result (one launch, no copy).
 double Engine::finish(int n_partials, int width, double *second) {
-  dev::finish_sum(d_partials_, n_partials, width, d_result_, stream_);
-  QS_HIP(hipMemcpyAsync(h_result_, d_result_, sizeof(double) * width, hipMemcpyDeviceToHost, stream_));
+  dev::finish_sum(d_partials_, n_partials, width, h_result_, stream_);
   sync();
   if (second) *second = h_result_[1];
   return h_result_[0];

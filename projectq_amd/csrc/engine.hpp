@@ -213,7 +213,7 @@ class Engine {
   std::mt19937 rng_;
   std::uniform_real_distribution<double> uni_{0.0, 1.0};
   hipStream_t stream_ = nullptr;
-  double *d_partials_ = nullptr, *d_result_ = nullptr, *h_result_ = nullptr;
+  double *d_partials_ = nullptr, *h_result_ = nullptr;
   int *d_flags_ = nullptr, *h_flags_ = nullptr;
   unsigned long long *d_key_ = nullptr, *h_key_ = nullptr;
   double *d_chunks_ = nullptr, *h_chunks_ = nullptr;

