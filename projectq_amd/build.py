@@ -50,6 +50,7 @@ SOURCES = [
     "tile_c64_rb4.hip",
     "tile_c128_rb4.hip",
     "kernels.hip",
+    "math.hip",
     "mlp.hip",
     "compare.hip",
     "noalloc.hip",
@@ -57,6 +58,7 @@ SOURCES = [
     "batch_energy.hip",
     "engine.cpp",
     "planner.cpp",
+    "math_map.cpp",
     "batch.cpp",
     "capi.cpp",
 ]

@@ -5,6 +5,7 @@
 #include <complex>
 
 #include "common.hpp"
+#include "math_map.hpp"
 
 namespace qs {
 namespace dev {
@@ -150,6 +151,9 @@ void scale_masked(amp_t<R> *psi, uint64_t n_amps, uint64_t cmask, double c_re, d
 template <typename R>
 void math_permute(const amp_t<R> *src, amp_t<R> *dst, uint64_t n_amps, const MathArgs &args,
                   const int32_t *table, int *err, hipStream_t s);
+// the same for the calls plan_math_gather covers (math_map.hpp): every destination reads its sources
+template <typename R>
+void math_gather(const amp_t<R> *src, amp_t<R> *dst, uint64_t n_amps, const MathGather &G, hipStream_t s);
 // bitmap (n_amps bits, zeroed by caller) marks dest(i); collide |= 1 on a repeated target
 void math_injective(uint64_t n_amps, const MathArgs &args, const int32_t *table,
                     uint32_t *bitmap, int *collide, int *err, hipStream_t s);
