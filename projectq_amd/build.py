@@ -51,6 +51,7 @@ SOURCES = [
     "tile_c128_rb4.hip",
     "kernels.hip",
     "math.hip",
+    "energy.hip",
     "mlp.hip",
     "compare.hip",
     "noalloc.hip",
@@ -59,6 +60,7 @@ SOURCES = [
     "engine.cpp",
     "planner.cpp",
     "math_map.cpp",
+    "energy_plan.cpp",
     "batch.cpp",
     "capi.cpp",
 ]

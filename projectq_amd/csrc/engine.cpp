@@ -4,6 +4,7 @@
 // cheat() and get_amplitude().
 #include "engine.hpp"
 
+#include "energy.hpp"
 #include "mfma_layout.hpp"
 
 #include <algorithm>
@@ -101,7 +102,7 @@ Engine::Engine(uint32_t seed, int precision, int fusion_mode, int planner, unsig
   }
   QS_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
   QS_HIP(hipMalloc(&d_partials_, sizeof(double) * 2 * dev::kReduceGrid));
-  QS_HIP(hipHostMalloc((void **)&h_result_, sizeof(double) * 4, hipHostMallocDefault));
+  QS_HIP(hipHostMalloc((void **)&h_result_, sizeof(double) * kResults, hipHostMallocDefault));
   QS_HIP(hipMalloc(&d_flags_, sizeof(int) * 4));
   QS_HIP(hipHostMalloc((void **)&h_flags_, sizeof(int) * 4, hipHostMallocDefault));
   QS_HIP(hipMalloc(&d_key_, sizeof(unsigned long long)));
@@ -1145,52 +1146,39 @@ void Engine::pauli_encode(const PauliString &t, const std::vector<unsigned> &ids
   encode_pauli(ops, x, z, omega);
 }
 
-// simulator.hpp:292-322: sum_t c_t Re<psi|P_t|psi>.  A state that fits in the last-level cache
-// is read once for all strings (one FP64 accumulator per thread: the coefficients and phases
-// are folded into each string); a larger state is read once per string so every pass streams.
+// simulator.hpp:292-322: sum_t c_t Re<psi|P_t|psi>, up to 128 strings a launch (energy.hip).
 double Engine::get_expectation_value(const std::vector<PauliString> &terms,
                                      const std::vector<double> &coeffs,
                                      const std::vector<unsigned> &ids) {
   run();
   check_known(ids, "get_expectation_value");
-  std::vector<dev::PauliTerm> pt(terms.size());
-  std::vector<cplx> omega(terms.size());
-  for (size_t t = 0; t < terms.size(); ++t) pauli_encode(terms[t], ids, &pt[t].x, &pt[t].z, &omega[t]);
-  const bool cached = amps() * amp_bytes() <= (uint64_t(64) << 20);
-  if (cached && !pt.empty()) {
-    for (size_t t = 0; t < pt.size(); ++t) {
-      if (!dev::pauli_hermitian(pt[t].x, pt[t].z, omega[t])) {
-        pt[t] = dev::PauliTerm{0, 0, 0.0, 0.0};  // Re<psi|P|psi> = 0 for an anti-Hermitian string
-        continue;
-      }
-      const cplx c = coeffs[t] * omega[t];
-      pt[t].c_re = c.real();
-      pt[t].c_im = c.imag();
-    }
-    const dev::PauliTerm *d_terms = (const dev::PauliTerm *)upload(pt.data(), pt.size() * sizeof(dev::PauliTerm));
-    dispatch([&](auto tag) {
-      using R = decltype(tag);
-      dev::pauli_energy<R>((const amp_t<R> *)psi_, amps(), d_terms, (int)pt.size(), d_partials_, stream_);
-    });
-    return finish(dev::kReduceGrid, 1);
+  std::vector<EnergyTerm> et(terms.size());
+  for (size_t t = 0; t < terms.size(); ++t) {
+    pauli_encode(terms[t], ids, &et[t].x, &et[t].z, &et[t].omega);
+    et[t].c = coeffs[t];
   }
   double total = 0.0;
-  for (size_t t = 0; t < terms.size(); ++t) {
-    if (!dev::pauli_hermitian(pt[t].x, pt[t].z, omega[t])) continue;  // Re<psi|P|psi> = 0
-    double delta;
-    if (pt[t].x == 0 && pt[t].z == 0) {
-      delta = omega[t].real() * masked_norm(0, 0);
-    } else {
-      dispatch([&](auto tag) {
-        using R = decltype(tag);
-        dev::pauli_expect<R>((const amp_t<R> *)psi_, amps(), pt[t].x, pt[t].z, d_partials_, stream_);
-      });
-      double si;
-      double sr = finish(dev::kReduceGrid, 2, &si);
-      delta = (omega[t] * cplx(sr, si)).real();
-    }
-    total += coeffs[t] * delta;
+  int results = 0;
+  auto collect = [&] {
+    sync();
+    for (int k = 0; k < results; ++k) total += h_result_[k];
+    results = 0;
+  };
+  EnergyPlan plan;
+  char records[kEnergyRecordBytes];
+  for (size_t t0 = 0; t0 < et.size(); t0 += kEnergyMaxStrings) {
+    const int m = (int)std::min<size_t>(kEnergyMaxStrings, et.size() - t0);
+    plan_energy(et.data() + t0, m, n_, c64_, plan);
+    const EnergyRecords rec = pack_energy(plan, records);
+    const char *d = rec.bytes ? (const char *)upload(records, rec.bytes) : nullptr;
+    if (results == kResults) collect();
+    double *out = h_result_ + results++;
+    dispatch([&](auto tag) {
+      using R = decltype(tag);
+      dev::energy<R>((const amp_t<R> *)psi_, n_, plan, d, rec, d_partials_, out, stream_);
+    });
   }
+  collect();
   return total;
 }
 

@@ -214,6 +214,7 @@ class Engine {
   std::uniform_real_distribution<double> uni_{0.0, 1.0};
   hipStream_t stream_ = nullptr;
   double *d_partials_ = nullptr, *h_result_ = nullptr;
+  static constexpr int kResults = 64;  // doubles in h_result_
   int *d_flags_ = nullptr, *h_flags_ = nullptr;
   unsigned long long *d_key_ = nullptr, *h_key_ = nullptr;
   double *d_chunks_ = nullptr, *h_chunks_ = nullptr;

@@ -381,102 +381,6 @@ __global__ __launch_bounds__(kBlock) void k_permute_tiles(const amp_t<R> *__rest
 }
 
 // ------------------------------------------------------------------------------ Pauli strings
-// Pauli strings in expectation values are Hermitian (the caller drops the others, whose real part
-// is zero): for x != 0 the amplitudes i and j = i ^ x contribute complex-conjugate terms to
-// <psi|omega X^x Z^z|psi>, so each pair is visited once, from the i with bit h (the highest bit of
-// x) clear, and counted twice.  That reads every amplitude once per string instead of twice.
-
-// partials[2b + {0,1}] <- block sums of f (-1)^popcount(j & z) conj(psi_i) psi_j, j = i ^ x, over the
-// i with bit h clear, f = 2 (x != 0); over every i with f = 1 (x = 0).  omega times the total has
-// the real part of <psi|omega X^x Z^z|psi>.
-template <typename R>
-__global__ __launch_bounds__(kBlock) void k_pauli_expect(const amp_t<R> *__restrict__ psi,
-                                                         uint64_t n, uint64_t x, uint64_t z,
-                                                         double *partials) {
-  __shared__ double lds[kBlock / 64];
-  Kahan sr, si;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  if (x == 0) {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-      const amp_t<R> a = psi[i];
-      const double v = (double)re(a) * re(a) + (double)im(a) * im(a);
-      sr.add((__popcll(i & z) & 1) ? -v : v);
-    }
-  } else {
-    const int hb = 63 - __clzll(x);
-    const uint64_t lo = (uint64_t(1) << hb) - 1;
-    for (uint64_t g = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; g < (n >> 1); g += stride) {
-      const uint64_t i = ((g & ~lo) << 1) | (g & lo);
-      const uint64_t j = i ^ x;
-      const amp_t<R> a = psi[i], b = psi[j];
-      const double f = (__popcll(j & z) & 1) ? -2.0 : 2.0;
-      sr.add(f * ((double)re(a) * re(b) + (double)im(a) * im(b)));
-      si.add(f * ((double)re(a) * im(b) - (double)im(a) * re(b)));
-    }
-  }
-  double tr = block_sum(sr.value(), lds);
-  double ti = block_sum(si.value(), lds);
-  if (threadIdx.x == 0) {
-    partials[2 * blockIdx.x] = tr;
-    partials[2 * blockIdx.x + 1] = ti;
-  }
-}
-
-// All strings in one pass over a state that fits the caches: partials[b] <- block sums of
-// Re(conj(psi_i) u_i), u_i = sum_t f_t c_t (-1)^popcount(j_t & z_t) psi_{j_t}, j_t = i ^ x_t, where a
-// string with x_t != 0 counts only at the i with bit h_t clear, with f_t = 2 (f_t = 1 for x_t = 0).
-// Partner loads are issued kInFlight strings at a time.
-template <typename R>
-__global__ __launch_bounds__(kBlock) void k_pauli_energy(const amp_t<R> *__restrict__ psi, uint64_t n,
-                                                         const PauliTerm *__restrict__ terms,
-                                                         int n_terms, double *partials) {
-  constexpr int kInFlight = 8;
-  __shared__ double lds[kBlock / 64];
-  Kahan acc;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const amp_t<R> a = psi[i];
-    double ur1 = 0.0, ui1 = 0.0, ur2 = 0.0, ui2 = 0.0;  // strings with x = 0, paired strings
-    auto term = [&](const PauliTerm &pt, const amp_t<R> &b) {
-      double br = re(b), bi = im(b);
-      if (__popcll((i ^ pt.x) & pt.z) & 1) {
-        br = -br;
-        bi = -bi;
-      }
-      const double vr = br * pt.c_re - bi * pt.c_im, vi = br * pt.c_im + bi * pt.c_re;
-      if (pt.x) {
-        ur2 += vr;
-        ui2 += vi;
-      } else {
-        ur1 += vr;
-        ui1 += vi;
-      }
-    };
-    int t = 0;
-    for (; t + kInFlight <= n_terms; t += kInFlight) {
-      amp_t<R> b[kInFlight];
-      bool on[kInFlight];
-#pragma unroll
-      for (int u = 0; u < kInFlight; ++u) {
-        const uint64_t x = terms[t + u].x;
-        on[u] = x == 0 || !((i >> (63 - __clzll(x))) & 1);
-        if (on[u]) b[u] = psi[i ^ x];
-      }
-#pragma unroll
-      for (int u = 0; u < kInFlight; ++u)
-        if (on[u]) term(terms[t + u], b[u]);
-    }
-    for (; t < n_terms; ++t) {
-      const PauliTerm &pt = terms[t];
-      if (pt.x && ((i >> (63 - __clzll(pt.x))) & 1)) continue;
-      term(pt, psi[i ^ pt.x]);
-    }
-    acc.add((double)re(a) * (ur1 + 2.0 * ur2) + (double)im(a) * (ui1 + 2.0 * ui2));  // Re(conj(a) * u)
-  }
-  double t = block_sum(acc.value(), lds);
-  if (threadIdx.x == 0) partials[blockIdx.x] = t;
-}
-
 template <typename R, bool EVOLVE>
 __global__ __launch_bounds__(kBlock) void k_pauli_sum(const amp_t<R> *__restrict__ src,
                                                       amp_t<R> *__restrict__ dst,
@@ -873,22 +777,6 @@ void permute_tiles(const amp_t<R> *src, amp_t<R> *dst, uint64_t n_amps, const Pe
 }
 
 template <typename R>
-void pauli_expect(const amp_t<R> *psi, uint64_t n, uint64_t x, uint64_t z, double *partials,
-                  hipStream_t s) {
-  hipLaunchKernelGGL(k_pauli_expect<R>, dim3(kReduceGrid), dim3(kBlock), 0, s, psi, n, x, z,
-                     partials);
-  QS_HIP(hipGetLastError());
-}
-
-template <typename R>
-void pauli_energy(const amp_t<R> *psi, uint64_t n, const PauliTerm *terms, int n_terms, double *partials,
-                  hipStream_t s) {
-  hipLaunchKernelGGL(k_pauli_energy<R>, dim3(kReduceGrid), dim3(kBlock), 0, s, psi, n, terms, n_terms,
-                     partials);
-  QS_HIP(hipGetLastError());
-}
-
-template <typename R>
 void pauli_sum(const amp_t<R> *src, amp_t<R> *dst, amp_t<R> *out, uint64_t n,
                const PauliTerm *terms, int n_terms, double f_re, double f_im, bool evolve,
                uint64_t cmask, double *partials, hipStream_t s) {
@@ -1003,10 +891,6 @@ template void convert_amps<float, double>(const amp_t<float> *, amp_t<double> *,
   template void drop_bit<R>(const amp_t<R> *, amp_t<R> *, uint64_t, int, int, hipStream_t);       \
   template void swap_bits<R>(amp_t<R> *, uint64_t, int, int, hipStream_t);                          \
   template void permute_tiles<R>(const amp_t<R> *, amp_t<R> *, uint64_t, const PermTile &, hipStream_t); \
-  template void pauli_expect<R>(const amp_t<R> *, uint64_t, uint64_t, uint64_t, double *,         \
-                                hipStream_t);                                                     \
-  template void pauli_energy<R>(const amp_t<R> *, uint64_t, const PauliTerm *, int, double *,      \
-                                hipStream_t);                                                     \
   template void pauli_sum<R>(const amp_t<R> *, amp_t<R> *, amp_t<R> *, uint64_t,                  \
                              const PauliTerm *, int, double, double, bool, uint64_t, double *,    \
                              hipStream_t);                                                        \

@@ -123,17 +123,6 @@ void swap_bits(amp_t<R> *psi, uint64_t n_amps, int a, int b, hipStream_t s);
 template <typename R>
 void permute_tiles(const amp_t<R> *src, amp_t<R> *dst, uint64_t n_amps, const PermTile &P, hipStream_t s);
 
-// Both expectation kernels take Hermitian strings only, omega X^x Z^z with omega^2 =
-// (-1)^popcount(x & z) (pauli_hermitian); the caller drops the others (their real part is zero).
-// partials[2*b + {0,1}] <- block sums whose total S satisfies Re(omega S) = Re<psi|omega X^x Z^z|psi>
-template <typename R>
-void pauli_expect(const amp_t<R> *psi, uint64_t n_amps, uint64_t x, uint64_t z,
-                  double *partials, hipStream_t s);
-// partials[b] <- block sums of sum_t Re<psi|c_t X^x_t Z^z_t|psi> (all terms in one pass; c_t
-// already carries the string's phase omega_t)
-template <typename R>
-void pauli_energy(const amp_t<R> *psi, uint64_t n_amps, const PauliTerm *terms, int n_terms,
-                  double *partials, hipStream_t s);
 // dst_i <- f * sum_t c_t (-1)^popcount((i^x_t)&z_t) src_{i^x_t}; with `evolve` also
 // out_i += dst_i and nrm partial sums of |dst_i|^2 on entries with (i & cmask) == cmask
 template <typename R>

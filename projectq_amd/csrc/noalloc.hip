@@ -14,7 +14,7 @@
 #include <complex>
 #include <mutex>
 
-#include "kernels.hpp"
+#include "energy.hpp"
 #include "planner.hpp"
 
 namespace qs {
@@ -22,13 +22,13 @@ namespace qs {
 namespace {
 
 // scratch layout (byte offsets, 256-byte aligned)
-constexpr size_t kTermsOff = 0;                                                         // PauliTerm[kNoAllocMaxTerms]
-constexpr size_t kPartialsOff = kTermsOff + sizeof(dev::PauliTerm) * kNoAllocMaxTerms;  // double[2 * kReduceGrid]
-constexpr size_t kResultsOff = kPartialsOff + sizeof(double) * 2 * dev::kReduceGrid;    // double[2 * kNoAllocMaxTerms]
-constexpr size_t kScratchBytes = kResultsOff + sizeof(double) * 2 * kNoAllocMaxTerms;
-static_assert(sizeof(dev::PauliTerm) == 32, "PauliTerm record size");
+constexpr size_t kRecordsOff = 0;                                                            // one plan's records
+constexpr size_t kPartialsOff = kRecordsOff + ((kEnergyRecordBytes + 255) & ~size_t(255));  // double[kEnergyPartials]
+constexpr size_t kResultsOff = kPartialsOff + sizeof(double) * dev::kEnergyPartials;        // double[plans]
+constexpr size_t kPlans = kNoAllocMaxTerms / kEnergyMaxStrings;
+constexpr size_t kScratchBytes = kResultsOff + sizeof(double) * kPlans;
 static_assert(kPartialsOff % 256 == 0 && kResultsOff % 256 == 0, "scratch regions stay 256-byte aligned");
-static_assert(kScratchBytes == kNoAllocScratchBytes, "scratch size as declared in noalloc.hpp");
+static_assert(kScratchBytes <= kNoAllocScratchBytes, "scratch size as declared in noalloc.hpp");
 
 }  // namespace
 
@@ -56,11 +56,9 @@ char *scratch_on_current_device() {
   return g_scratch[dev];
 }
 
-constexpr size_t kChunk = 128;  // strings encoded per host chunk (stack storage)
-
 // String t as  omega * X^x Z^z  (the engine's encoding), with its local indices mapped.
 void encode(size_t t, const uint32_t *term_idx, const uint8_t *term_ops, const size_t *term_offsets,
-            const uint32_t *positions, size_t n_positions, dev::PauliTerm *pt, std::complex<double> *omega) {
+            const uint32_t *positions, size_t n_positions, EnergyTerm *out) {
   PauliEncoder e;
   for (size_t j = term_offsets[t]; j < term_offsets[t + 1]; ++j) {
     if (term_idx[j] >= n_positions) throw ValueError("qubit_operator acts on more qubits than contained in the qureg.");
@@ -68,9 +66,9 @@ void encode(size_t t, const uint32_t *term_idx, const uint8_t *term_ops, const s
     if (op != 'X' && op != 'Y' && op != 'Z') throw ValueError("Pauli operator must be X, Y or Z");
     e.add(positions[term_idx[j]], op);
   }
-  pt->x = e.x;
-  pt->z = e.z;
-  *omega = e.omega;
+  out->x = e.x;
+  out->z = e.z;
+  out->omega = e.omega;
 }
 
 }  // namespace
@@ -86,82 +84,40 @@ double expectation_noalloc(const void *state, unsigned n_qubits, bool c64, const
     if (positions[l] >= n_qubits) throw ValueError("expectation_noalloc: a qubit position lies outside the state");
   // validate every string before any device work
   for (size_t t = 0; t < n_terms; ++t) {
-    dev::PauliTerm pt;
-    std::complex<double> w;
-    encode(t, term_idx, term_ops, term_offsets, positions, n_positions, &pt, &w);
+    EnergyTerm e;
+    encode(t, term_idx, term_ops, term_offsets, positions, n_positions, &e);
   }
   if (n_terms == 0) return 0.0;
-  const uint64_t n_amps = uint64_t(1) << n_qubits;
   char *base = scratch_on_current_device();
-  dev::PauliTerm *d_terms = reinterpret_cast<dev::PauliTerm *>(base + kTermsOff);
   double *d_partials = reinterpret_cast<double *>(base + kPartialsOff);
   double *d_results = reinterpret_cast<double *>(base + kResultsOff);
   const hipStream_t s = nullptr;  // the null stream; the call returns when its work is done
   QS_HIP(hipStreamSynchronize(s));
-  dev::PauliTerm pt[kChunk];
-  std::complex<double> omega[kChunk];
-  // the engine's choice: one pass for all strings while the state fits the last-level cache, one
-  // streaming pass per string above it
-  const bool cached = n_amps * (c64 ? 8u : 16u) <= (uint64_t(64) << 20);
-  if (cached) {
-    for (size_t t0 = 0; t0 < n_terms; t0 += kChunk) {
-      const size_t m = std::min(kChunk, n_terms - t0);
-      for (size_t i = 0; i < m; ++i) {
-        encode(t0 + i, term_idx, term_ops, term_offsets, positions, n_positions, &pt[i], &omega[i]);
-        if (!dev::pauli_hermitian(pt[i].x, pt[i].z, omega[i])) {
-          pt[i] = dev::PauliTerm{0, 0, 0.0, 0.0};  // Re<psi|P|psi> = 0 for an anti-Hermitian string
-          continue;
-        }
-        const std::complex<double> c = coeffs[t0 + i] * omega[i];
-        pt[i].c_re = c.real();
-        pt[i].c_im = c.imag();
-      }
-      QS_HIP(hipMemcpy(d_terms + t0, pt, m * sizeof(dev::PauliTerm), hipMemcpyHostToDevice));
+  EnergyTerm terms[kEnergyMaxStrings];
+  EnergyPlan plan;
+  char records[kEnergyRecordBytes];
+  size_t plans = 0;
+  for (size_t t0 = 0; t0 < n_terms; t0 += kEnergyMaxStrings, ++plans) {
+    const size_t m = std::min<size_t>(kEnergyMaxStrings, n_terms - t0);
+    for (size_t i = 0; i < m; ++i) {
+      encode(t0 + i, term_idx, term_ops, term_offsets, positions, n_positions, &terms[i]);
+      terms[i].c = coeffs[t0 + i];
     }
+    plan_energy(terms, (int)m, n_qubits, c64, plan);
+    const EnergyRecords rec = pack_energy(plan, records);
+    // in stream order: the previous plan's kernels have read their records
+    if (rec.bytes) QS_HIP(hipMemcpy(base + kRecordsOff, records, rec.bytes, hipMemcpyHostToDevice));
     if (c64)
-      dev::pauli_energy<float>(static_cast<const float2 *>(state), n_amps, d_terms, (int)n_terms, d_partials, s);
+      dev::energy<float>(static_cast<const float2 *>(state), n_qubits, plan, base + kRecordsOff, rec, d_partials,
+                         d_results + plans, s);
     else
-      dev::pauli_energy<double>(static_cast<const double2 *>(state), n_amps, d_terms, (int)n_terms, d_partials, s);
-    dev::finish_sum(d_partials, dev::kReduceGrid, 1, d_results, s);
-    double out = 0.0;
-    QS_HIP(hipMemcpy(&out, d_results, sizeof(double), hipMemcpyDeviceToHost));
-    return out;
+      dev::energy<double>(static_cast<const double2 *>(state), n_qubits, plan, base + kRecordsOff, rec, d_partials,
+                          d_results + plans, s);
   }
-  const BitInsert none{};
+  double res[kPlans];
+  QS_HIP(hipMemcpy(res, d_results, plans * sizeof(double), hipMemcpyDeviceToHost));
   double total = 0.0;
-  for (size_t t0 = 0; t0 < n_terms; t0 += kChunk) {
-    const size_t m = std::min(kChunk, n_terms - t0);
-    for (size_t i = 0; i < m; ++i) {
-      encode(t0 + i, term_idx, term_ops, term_offsets, positions, n_positions, &pt[i], &omega[i]);
-      double *out = d_results + 2 * (t0 + i);
-      if (!dev::pauli_hermitian(pt[i].x, pt[i].z, omega[i])) continue;  // contributes 0, read back unused
-      if (pt[i].x == 0 && pt[i].z == 0) {
-        if (c64)
-          dev::norm_masked<float>(static_cast<const float2 *>(state), n_amps, none, 0, d_partials, s);
-        else
-          dev::norm_masked<double>(static_cast<const double2 *>(state), n_amps, none, 0, d_partials, s);
-        dev::finish_sum(d_partials, dev::kReduceGrid, 1, out, s);
-      } else {
-        if (c64)
-          dev::pauli_expect<float>(static_cast<const float2 *>(state), n_amps, pt[i].x, pt[i].z, d_partials, s);
-        else
-          dev::pauli_expect<double>(static_cast<const double2 *>(state), n_amps, pt[i].x, pt[i].z, d_partials, s);
-        dev::finish_sum(d_partials, dev::kReduceGrid, 2, out, s);
-      }
-    }
-    double res[2 * kChunk];
-    QS_HIP(hipMemcpy(res, d_results + 2 * t0, 2 * m * sizeof(double), hipMemcpyDeviceToHost));
-    for (size_t i = 0; i < m; ++i) {
-      double delta;
-      if (!dev::pauli_hermitian(pt[i].x, pt[i].z, omega[i]))
-        delta = 0.0;
-      else if (pt[i].x == 0 && pt[i].z == 0)
-        delta = omega[i].real() * res[2 * i];
-      else
-        delta = (omega[i] * std::complex<double>(res[2 * i], res[2 * i + 1])).real();
-      total += coeffs[t0 + i] * delta;
-    }
-  }
+  for (size_t k = 0; k < plans; ++k) total += res[k];
   return total;
 }
 
