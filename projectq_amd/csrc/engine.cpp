@@ -863,17 +863,20 @@ void Engine::exec_block(const Block &b) {
   }
   dispatch([&](auto tag) {
     using R = decltype(tag);
-    std::vector<amp_t<R>> m(D * D);
-    for (size_t i = 0; i < D * D; ++i) {
-      m[i].x = (R)b.m[i].real();
-      m[i].y = (R)b.m[i].imag();
+    const amp_t<R> *dm = nullptr;
+    if (k == 5) {
+      std::vector<amp_t<R>> m(D * D);
+      for (size_t i = 0; i < D * D; ++i) {
+        m[i].x = (R)b.m[i].real();
+        m[i].y = (R)b.m[i].imag();
+      }
+      dm = (const amp_t<R> *)upload(m.data(), m.size() * sizeof(amp_t<R>));
     }
-    const amp_t<R> *dm = (const amp_t<R> *)upload(m.data(), m.size() * sizeof(amp_t<R>));
     PassFeatures f{};
     if (recording_) f = block_features(b);
     hipEvent_t e0, e1;
     begin_pass(&e0, &e1);
-    dev::apply_block<R>((amp_t<R> *)psi_, n_groups, ins, cmask, tpos.data(), k, dm, stream_);
+    dev::apply_block<R>((amp_t<R> *)psi_, n_groups, ins, cmask, tpos.data(), k, b.m.data(), dm, stream_);
     end_pass(e0, e1, recording_ ? &f : nullptr);
   });
   // algorithmic traffic: every touched amplitude is read once and written once

@@ -67,10 +67,11 @@ void batch_energy_finish(const EnergyJob *jobs, int n_jobs, const double *partia
 
 // dense gate block: psi[base + off(r)] = sum_c M[r][c] psi[base + off(c)] for every base with
 // target bits 0 and control bits 1.  tpos[l] is the position of matrix bit l; ins lists the
-// sorted target+control positions; n_groups = 2^(n - k - #controls).
+// sorted target+control positions; n_groups = 2^(n - k - #controls).  The host matrix `mat` is read
+// before the call returns; k = 5 takes it from device memory instead (`d_mat`).
 template <typename R>
 void apply_block(amp_t<R> *psi, uint64_t n_groups, const BitInsert &ins, uint64_t cmask,
-                 const uint32_t *tpos, int k, const amp_t<R> *d_mat, hipStream_t s);
+                 const uint32_t *tpos, int k, const std::complex<double> *mat, const amp_t<R> *d_mat, hipStream_t s);
 
 // the same dense block for a complex64 state on the matrix cores (k = 3, 4, 5): d_table is the
 // per-lane A-operand table of mfma::operand_table (mfma_layout.hpp)
