@@ -112,6 +112,7 @@ class Engine {
   void ensure_capacity(uint64_t need_amps);
   void *scratch(int which);  // full-capacity scratch buffer 0 or 1 (lazy)
   void release_scratch();
+  char *reserve(size_t bytes, char **host);
   const void *upload(const void *host, size_t bytes);
   double finish(int n_partials, int width, double *second = nullptr);
   void sync();
@@ -172,7 +173,15 @@ class Engine {
   // windows without 2-qubit gates; PROJECTQ_AMD_CZ=0 keeps them as X ops
   bool cnot_cz_ = true;
   void apply_relabel(const std::vector<std::pair<uint32_t, uint32_t>> &swaps);
-  void exec_tile_program(const TileProgram &prog, unsigned rb);
+  struct DeviceProgram {  // a TileProgram's records in device memory
+    const dev::TileStage *stages;
+    const dev::RegOp *rops;
+    const dev::TileOp *tops;
+    const void *mats;
+    bool two_qubit_ops;
+  };
+  size_t upload_programs(const std::vector<TileProgram> &progs, size_t first, std::vector<DeviceProgram> *out);
+  void exec_tile_program(const TileProgram &prog, const DeviceProgram &d, unsigned rb);
   PassFeatures block_features(const Block &b) const;
   void begin_pass(hipEvent_t *e0, hipEvent_t *e1);
   void end_pass(hipEvent_t e0, hipEvent_t e1, const PassFeatures *f);
