@@ -2,7 +2,7 @@
 #include "planner.hpp"
 
 #include <algorithm>
-#include <map>
+#include <atomic>
 #include <set>
 #include <stdexcept>
 
@@ -11,13 +11,13 @@ namespace qs {
 std::vector<PGate> merge_single_qubit_runs(const std::vector<PGate> &gates) {
   std::vector<PGate> out;
   out.reserve(gates.size());
-  std::map<uint32_t, int> last;  // position -> index in `out` of the last gate touching it
+  int last[64];  // position -> index in `out` of the last gate touching it
+  std::fill(last, last + 64, -1);
   for (const PGate &g : gates) {
     const bool single = g.tpos.size() == 1 && g.cmask == 0;
     if (single) {
-      auto it = last.find(g.tpos[0]);
-      if (it != last.end()) {
-        PGate &prev = out[it->second];
+      if (last[g.tpos[0]] >= 0) {
+        PGate &prev = out[last[g.tpos[0]]];
         if (prev.tpos.size() == 1 && prev.cmask == 0) {
           // prev <- g * prev (g acts after prev)
           std::vector<std::complex<double>> m(4);
@@ -30,9 +30,7 @@ std::vector<PGate> merge_single_qubit_runs(const std::vector<PGate> &gates) {
     }
     out.push_back(g);
     const int idx = (int)out.size() - 1;
-    uint64_t touch = g.tmask() | g.cmask;
-    for (uint32_t p = 0; p < 64; ++p)
-      if ((touch >> p) & 1) last[p] = idx;
+    for (uint64_t touch = g.tmask() | g.cmask; touch; touch &= touch - 1) last[__builtin_ctzll(touch)] = idx;
   }
   return out;
 }
@@ -49,19 +47,16 @@ std::vector<PGate> cnot_to_cz(const std::vector<PGate> &gates) {
     return i >= 0 && i < n && gates[i].tpos.size() == 1 && gates[i].tpos[0] == p && gates[i].cmask == 0;
   };
   // gates touching each position, in order
-  std::map<uint32_t, std::vector<int>> seq;
-  for (int i = 0; i < n; ++i) {
-    const uint64_t touch = gates[i].tmask() | gates[i].cmask;
-    for (uint32_t p = 0; p < 64; ++p)
-      if ((touch >> p) & 1) seq[p].push_back(i);
-  }
+  std::vector<int> seq[64];
+  for (int i = 0; i < n; ++i)
+    for (uint64_t touch = gates[i].tmask() | gates[i].cmask; touch; touch &= touch - 1)
+      seq[__builtin_ctzll(touch)].push_back(i);
   // runs of CNOTs on one target with nothing else touching it in between: X_1 .. X_k = H Z_1 .. Z_k H,
   // so a run between uncontrolled 1-qubit gates on the target takes one H before its first CNOT
   // and one after its last
   std::vector<char> h_before(n, 0), h_after(n, 0), as_cz(n, 0);
-  for (auto &kv : seq) {
-    const uint32_t t = kv.first;
-    const std::vector<int> &s = kv.second;
+  for (uint32_t t = 0; t < 64; ++t) {
+    const std::vector<int> &s = seq[t];
     for (size_t a = 0; a < s.size();) {
       if (!is_cnot(s[a]) || gates[s[a]].tpos[0] != t) {
         ++a;
@@ -159,19 +154,20 @@ std::vector<PPass> schedule_tiles(const std::vector<PGate> &gates, const TileSha
     for (int i = 0; i < G; ++i) {
       const bool diag = diagonal_gate(gates[i]);
       const uint64_t tm = diag ? 0 : gates[i].tmask(), cm = gates[i].cmask | (diag ? gates[i].tmask() : 0);
-      std::set<int> ps;
-      for (uint32_t p = 0; p < 64; ++p) {
-        if (!(((tm | cm) >> p) & 1)) continue;
-        if (writer[p] >= 0) ps.insert(writer[p]);
+      std::vector<int> &ps = preds[i];
+      for (uint64_t m = tm | cm; m; m &= m - 1) {
+        const uint32_t p = (uint32_t)__builtin_ctzll(m);
+        if (writer[p] >= 0) ps.push_back(writer[p]);
         if ((tm >> p) & 1) {
-          ps.insert(readers[p].begin(), readers[p].end());
+          ps.insert(ps.end(), readers[p].begin(), readers[p].end());
           readers[p].clear();
           writer[p] = i;
         } else {
           readers[p].push_back(i);
         }
       }
-      preds[i].assign(ps.begin(), ps.end());
+      std::sort(ps.begin(), ps.end());
+      ps.erase(std::unique(ps.begin(), ps.end()), ps.end());
     }
   }
   std::vector<char> done(G, 0);
@@ -284,11 +280,7 @@ namespace {
 
 using cplx = std::complex<double>;
 
-uint32_t popcount32(uint32_t x) {
-  uint32_t c = 0;
-  for (; x; x &= x - 1) ++c;
-  return c;
-}
+uint32_t popcount32(uint32_t x) { return (uint32_t)__builtin_popcount(x); }
 
 // a gate of the pass in tile-local terms
 struct LocalGate {
@@ -344,6 +336,22 @@ void emit_lds_op(const LocalGate &g, unsigned t, TileProgram &prog) {
   prog.stages.push_back(st);
 }
 
+// stage_conflict_degree of the register bits `mask`, remembered: planning asks for the same few
+// thousand sets over and over, from several threads (0: not known yet; every thread computes the same
+// value).
+uint32_t conflict_degree(uint32_t mask, uint32_t t, bool c64) {
+  static std::atomic<uint8_t> known[2][dev::kTileMaxBits + 1][1u << dev::kTileMaxBits];
+  const uint32_t lane_bits = c64 ? 5u : 4u;
+  if (t > (uint32_t)dev::kTileMaxBits || mask >> dev::kTileMaxBits) return dev::stage_conflict_degree(mask, t, c64, lane_bits);
+  std::atomic<uint8_t> &e = known[c64][t][mask];
+  uint32_t v = e.load(std::memory_order_relaxed);
+  if (v == 0) {
+    v = dev::stage_conflict_degree(mask, t, c64, lane_bits);
+    e.store((uint8_t)v, std::memory_order_relaxed);
+  }
+  return v;
+}
+
 // Register bits of a stage: the op targets `need` plus padding up to rb bits.  The padding is the
 // choice with the fewest LDS bank conflicts (stage_conflict_degree over the lanes one LDS cycle
 // serves: 32 lanes of 8-byte accesses for complex64, 16 lanes of 16-byte accesses for
@@ -359,7 +367,6 @@ uint32_t pad_stage_bits(uint32_t need, unsigned t, unsigned rb, bool c64) {
   for (uint32_t p = 0; p < t; ++p)
     if (!((need >> p) & 1)) free_bits.push_back(p);
   const uint32_t k = rb - have;
-  const uint32_t lane_bits = c64 ? 5u : 4u;
   uint32_t best = 0, best_cost = ~0u;
   // enumerate k-subsets of free_bits in lexicographic order (lowest bits first)
   std::vector<uint32_t> idx(k);
@@ -367,7 +374,7 @@ uint32_t pad_stage_bits(uint32_t need, unsigned t, unsigned rb, bool c64) {
   while (true) {
     uint32_t bits = need;
     for (uint32_t i : idx) bits |= 1u << free_bits[i];
-    const uint32_t cost = dev::stage_conflict_degree(bits, t, c64, lane_bits);
+    const uint32_t cost = conflict_degree(bits, t, c64);
     if (cost < best_cost) {
       best_cost = cost;
       best = bits;
@@ -469,19 +476,20 @@ void partition_stages(const std::vector<LocalGate> &lgs, const std::vector<char>
     std::vector<int> writer(32, -1);
     std::vector<std::vector<int>> readers(32);
     for (int i = 0; i < n; ++i) {
-      std::set<int> ps;
-      for (uint32_t b = 0; b < 32; ++b) {
-        if (!(((wr[i] | rd[i]) >> b) & 1)) continue;
-        if (writer[b] >= 0) ps.insert(writer[b]);
+      std::vector<int> &ps = preds[i];
+      for (uint32_t m = wr[i] | rd[i]; m; m &= m - 1) {
+        const uint32_t b = (uint32_t)__builtin_ctz(m);
+        if (writer[b] >= 0) ps.push_back(writer[b]);
         if ((wr[i] >> b) & 1) {
-          ps.insert(readers[b].begin(), readers[b].end());
+          ps.insert(ps.end(), readers[b].begin(), readers[b].end());
           readers[b].clear();
           writer[b] = i;
         } else {
           readers[b].push_back(i);
         }
       }
-      preds[i].assign(ps.begin(), ps.end());
+      std::sort(ps.begin(), ps.end());
+      ps.erase(std::unique(ps.begin(), ps.end()), ps.end());
     }
   }
   std::vector<char> done(n, 0);
@@ -507,34 +515,41 @@ void partition_stages(const std::vector<LocalGate> &lgs, const std::vector<char>
         cand |= tm[i];
       }
       cand &= ~tm[f];
-      const uint32_t lane_bits = c64 ? 5u : 4u;
       const uint32_t free_slots = rb - (uint32_t)popcount32(tm[f]);
       uint32_t bits;
       if ((uint32_t)popcount32(cand) <= free_slots) {
         bits = pad_stage_bits(tm[f] | cand, t, rb, c64);
       } else {
-        // gates a stage with these bits would take, simulated over the window
-        std::vector<char> sim(n);
-        auto absorbed = [&](uint32_t b) {
-          for (int i : window) sim[i] = done[i];
-          int got = 0;
-          for (bool progress = true; progress;) {
-            progress = false;
-            for (int i : window) {
-              if (sim[i] || (tm[i] & ~b) || popcount32(lgs[i].lc & b) > 1) continue;
-              bool ok = true;
-              for (int p : preds[i])
-                if (!(p >= f ? sim[p] : done[p])) {
-                  ok = false;
-                  break;
-                }
-              if (!ok) continue;
-              sim[i] = 1;
-              ++got;
-              progress = true;
-            }
+        // gates a stage with these bits would take, simulated over the window (at most 48 gates: one
+        // word).  Predecessors come first, so one sweep in order finds them all.
+        const int nw = (int)window.size();
+        uint64_t needs[kWindow], on_bit[32] = {}, crowded = 0, stuck = 0;
+        for (int k = 0; k < nw; ++k) {
+          const int i = window[k];
+          needs[k] = 0;
+          for (int p : preds[i]) {
+            if (p < f) continue;  // placed
+            const auto it = std::lower_bound(window.begin(), window.end(), p);
+            if (it == window.end() || *it != p) stuck |= uint64_t(1) << k;  // not among the gates simulated
+            else needs[k] |= uint64_t(1) << (it - window.begin());
           }
-          return got;
+          for (uint32_t m = tm[i]; m; m &= m - 1) on_bit[__builtin_ctz(m)] |= uint64_t(1) << k;
+          if (lgs[i].lc & (lgs[i].lc - 1)) crowded |= uint64_t(1) << k;
+        }
+        const uint64_t all = nw == 64 ? ~uint64_t(0) : (uint64_t(1) << nw) - 1;
+        auto absorbed = [&](uint32_t b) {
+          uint64_t fits = all & ~stuck;
+          for (uint32_t m = cand & ~b; m; m &= m - 1) fits &= ~on_bit[__builtin_ctz(m)];
+          for (uint64_t m = crowded & fits; m; m &= m - 1) {
+            const int k = __builtin_ctzll(m);
+            if (popcount32(lgs[window[k]].lc & b) > 1) fits &= ~(uint64_t(1) << k);
+          }
+          uint64_t got = 0;
+          for (uint64_t m = fits; m; m &= m - 1) {
+            const int k = __builtin_ctzll(m);
+            if (!(needs[k] & ~got)) got |= uint64_t(1) << k;
+          }
+          return __builtin_popcountll(got);
         };
         std::vector<uint32_t> cbits;
         for (uint32_t b = 0; b < t; ++b)
@@ -548,7 +563,7 @@ void partition_stages(const std::vector<LocalGate> &lgs, const std::vector<char>
           uint32_t b = tm[f];
           for (uint32_t i : idx) b |= 1u << cbits[i];
           const int got = absorbed(b);
-          const uint32_t conf = dev::stage_conflict_degree(b, t, c64, lane_bits);
+          const uint32_t conf = conflict_degree(b, t, c64);
           if (got > best_got || (got == best_got && conf < best_conf)) {
             best_got = got;
             best_conf = conf;
