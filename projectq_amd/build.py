@@ -52,6 +52,7 @@ SOURCES = [
     "kernels.hip",
     "math.hip",
     "energy.hip",
+    "measure.hip",
     "mlp.hip",
     "compare.hip",
     "noalloc.hip",

@@ -107,6 +107,8 @@ Engine::Engine(uint32_t seed, int precision, int fusion_mode, int planner, unsig
   QS_HIP(hipHostMalloc((void **)&h_flags_, sizeof(int) * 4, hipHostMallocDefault));
   QS_HIP(hipMalloc(&d_key_, sizeof(unsigned long long)));
   QS_HIP(hipHostMalloc((void **)&h_key_, sizeof(unsigned long long), hipHostMallocDefault));
+  QS_HIP(hipMalloc(&d_measure_, sizeof(dev::Measurement)));
+  QS_HIP(hipEventCreateWithFlags(&picked_, hipEventDisableTiming));
   QS_HIP(hipMalloc(&d_arena_, kArenaBytes));
   QS_HIP(hipHostMalloc((void **)&h_arena_, kArenaBytes, hipHostMallocDefault));
   // initial state |> = [1]  (simulator.hpp:48-51)
@@ -139,8 +141,9 @@ Engine::~Engine() {
   (void)hipHostFree(h_flags_);
   (void)hipFree(d_key_);
   (void)hipHostFree(h_key_);
-  (void)hipFree(d_chunks_);
-  (void)hipHostFree(h_chunks_);
+  (void)hipFree(d_sums_);
+  (void)hipFree(d_measure_);
+  if (picked_) (void)hipEventDestroy(picked_);
   (void)hipFree(d_arena_);
   (void)hipHostFree(h_arena_);
   if (stream_) (void)hipStreamDestroy(stream_);
@@ -241,19 +244,25 @@ void Engine::allocate_qubit(unsigned id) {
   pos_[id] = n_++;
 }
 
+// Whether an amplitude above tol has the bit of qubit `id` clear (bit 0 of the answer) and set (bit 1).
+int Engine::sides(unsigned id, double tol) {
+  const bool known = tol >= 0.0;  // the amplitudes known to be zero are not above it
+  const BitInsert sub = make_insert(bits_of(known ? zmask_ : 0));
+  dispatch([&](auto tag) {
+    using R = decltype(tag);
+    dev::classical<R>((const amp_t<R> *)psi_, amps() >> sub.count, sub, known ? zval_ : 0, (int)pos_[id], tol, d_flags_, h_flags_,
+                      stream_);
+  });
+  sync();
+  return *h_flags_;
+}
+
 // simulator.hpp:93-108
 bool Engine::is_classical(unsigned id, double tol) {
   run();
   check_known({id}, "is_classical");
-  QS_HIP(hipMemsetAsync(d_flags_, 0, sizeof(int) * 2, stream_));
-  int p = (int)pos_[id];
-  dispatch([&](auto tag) {
-    using R = decltype(tag);
-    dev::classical_flags<R>((const amp_t<R> *)psi_, amps(), p, tol, d_flags_, stream_);
-  });
-  QS_HIP(hipMemcpyAsync(h_flags_, d_flags_, sizeof(int) * 2, hipMemcpyDeviceToHost, stream_));
-  sync();
-  return (h_flags_[0] ^ h_flags_[1]) == 1;
+  const int s = sides(id, tol);
+  return s == 1 || s == 2;
 }
 
 // simulator.hpp:76-91: the first pair (bit clear, bit set) in index order holding an entry
@@ -278,10 +287,11 @@ bool Engine::get_classical_value(unsigned id, double tol) {
 void Engine::deallocate_qubit(unsigned id) {
   canonicalize();
   check_known({id}, "deallocate_qubit");
-  if (!is_classical(id, 1e-12))
+  const int side = sides(id, 1e-12);
+  if (side != 1 && side != 2)
     throw RuntimeError(
         "Error: Qubit has not been measured / uncomputed! There is most likely a bug in your code.");
-  const bool value = get_classical_value(id, 1e-12);
+  const bool value = side == 2;  // every amplitude above the tolerance has this value
   const unsigned p = pos_[id];
   const uint64_t half = amps() / 2;
   if (p == n_ - 1) {  // top bit: the kept half is already contiguous
@@ -296,7 +306,6 @@ void Engine::deallocate_qubit(unsigned id) {
     });
     std::swap(psi_, buf_[0]);
   }
-  sync();
   for (auto &kv : pos_)
     if (kv.second > p) kv.second--;
   pos_.erase(id);
@@ -313,77 +322,33 @@ void Engine::deallocate_qubit(unsigned id) {
 }
 
 // ------------------------------------------------------------------------------ measurement
-// simulator.hpp:145-186.  One uniform draw; the serial cumulative scan of the reference is
-// replaced by chunk sums (one read pass), a host prefix over the chunks and an in-chunk scan,
-// which lands on the same index unless the draw is within rounding of a boundary.
+// simulator.hpp:145-186.  One uniform draw; the serial cumulative scan of the reference is replaced by
+// chunk sums (one read pass), a prefix over the chunks and an in-chunk scan, which lands on the same
+// index unless the draw is within rounding of a boundary.
 std::vector<uint8_t> Engine::measure_qubits(const std::vector<unsigned> &ids) {
   canonicalize();  // the pick scans the reference's index order
   check_known(ids, "measure_qubits");
-  const double rnd = uni_(rng_);
-  const uint64_t N = amps();
+  pointer_out_ = false;  // a handed-out state pointer is valid up to the next measurement
   // the scan runs over the subspace outside which every amplitude is zero: the same amplitudes in
   // the same index order, without the zeros
-  const BitInsert sub = make_insert(bits_of(zmask_));
-  const uint64_t n_sub = N >> sub.count;
-  uint64_t pick;
-  if (!(rnd > 0.0)) {
-    pick = ~uint64_t(0);  // the reference's loop never runs and `pick--` wraps
-  } else {
-    const int lg = (int)std::min<unsigned>(n_ - sub.count, 12);
-    const uint64_t len = uint64_t(1) << lg, chunks = n_sub >> lg;
-    if (chunks > chunks_cap_) {
-      (void)hipFree(d_chunks_);
-      (void)hipHostFree(h_chunks_);
-      d_chunks_ = h_chunks_ = nullptr;
-      chunks_cap_ = 0;
-      QS_HIP(hipMalloc(&d_chunks_, chunks * sizeof(double)));
-      QS_HIP(hipHostMalloc((void **)&h_chunks_, chunks * sizeof(double), hipHostMallocDefault));
-      chunks_cap_ = chunks;
-    }
-    dispatch([&](auto tag) {
-      using R = decltype(tag);
-      dev::chunk_norms<R>((const amp_t<R> *)psi_, n_sub, sub, zval_, lg, d_chunks_, stream_);
-    });
-    QS_HIP(hipMemcpyAsync(h_chunks_, d_chunks_, chunks * sizeof(double), hipMemcpyDeviceToHost, stream_));
-    sync();
-    double run_sum = 0.0;
-    uint64_t c = 0;
-    for (; c < chunks; ++c) {
-      if (run_sum + h_chunks_[c] >= rnd) break;
-      run_sum += h_chunks_[c];
-    }
-    if (c == chunks) {
-      pick = N - 1;  // the draw exceeds the total norm: the scan runs off the end
-    } else {
-      *h_key_ = ~0ull;
-      QS_HIP(hipMemcpyAsync(d_key_, h_key_, sizeof(unsigned long long), hipMemcpyHostToDevice, stream_));
-      dispatch([&](auto tag) {
-        using R = decltype(tag);
-        dev::chunk_pick<R>((const amp_t<R> *)psi_, sub, zval_, c * len, len, run_sum, rnd, d_key_, stream_);
-      });
-      QS_HIP(hipMemcpyAsync(h_key_, d_key_, sizeof(unsigned long long), hipMemcpyDeviceToHost, stream_));
-      sync();
-      const uint64_t compact = (*h_key_ == ~0ull) ? (c + 1) * len - 1 : (uint64_t)*h_key_;
-      pick = insert_zeros_host(compact, sub) | zval_;
-    }
-  }
-  std::vector<uint8_t> res(ids.size());
-  uint64_t mask = 0, val = 0;
-  for (size_t i = 0; i < ids.size(); ++i) {
-    unsigned p = pos_[ids[i]];
-    res[i] = (uint8_t)((pick >> p) & 1);
-    mask |= uint64_t(1) << p;
-    val |= uint64_t(res[i]) << p;
-  }
-  // outcome bits that contradict fixed bits select only zero amplitudes (the reference's edge
-  // cases of a draw of 0 or beyond the total)
-  const double kept = ((val ^ zval_) & mask & zmask_) ? 0.0 : masked_norm(mask | zmask_, val | (zval_ & ~mask));
-  double scale = 1.0 / std::sqrt(kept);
+  dev::MeasureArgs a{};
+  a.rnd = uni_(rng_);
+  a.n_amps = amps();
+  a.sub = make_insert(bits_of(zmask_));
+  a.n_sub = a.n_amps >> a.sub.count;
+  a.sval = zval_;
+  a.zmask = zmask_;
+  a.mask = mask_of(ids);
+  if (a.n_sub > dev::kMeasureSmall && !d_sums_) QS_HIP(hipMalloc(&d_sums_, 2 * dev::kMeasureChunks * sizeof(double)));
   dispatch([&](auto tag) {
     using R = decltype(tag);
-    dev::collapse<R>((amp_t<R> *)psi_, n_sub, sub, zval_, mask, val, scale, stream_);
+    dev::measure<R>((amp_t<R> *)psi_, a, d_measure_, h_key_, d_sums_, d_partials_, picked_, stream_);
   });
-  subspace_fix(mask, val);
+  QS_HIP(hipEventSynchronize(picked_));  // the outcome; the collapse may still run
+  const uint64_t pick = *h_key_;
+  std::vector<uint8_t> res(ids.size());
+  for (size_t i = 0; i < ids.size(); ++i) res[i] = (uint8_t)((pick >> pos_[ids[i]]) & 1);
+  subspace_fix(a.mask, pick & a.mask);
   norm_changed();
   return res;
 }

@@ -16,6 +16,7 @@
 #include "common.hpp"
 #include "fusion.hpp"
 #include "kernels.hpp"
+#include "measure.hpp"
 #include "mlp.hpp"
 #include "planner.hpp"
 
@@ -124,6 +125,7 @@ class Engine {
                           const std::vector<unsigned> &ctrl) const;
   void math_apply(dev::MathArgs args, const int32_t *d_table, bool known_bijective);
   double masked_norm(uint64_t mask, uint64_t val);
+  int sides(unsigned id, double tol);
   void flush_window();
   // complex64 norm guard: FP32-rounded gate matrices are unitary only to ~1e-8 (the FP32 H scales
   // the norm by 1 - 3.4e-8), so over thousands of gates the state's norm drifts from its exact
@@ -150,7 +152,7 @@ class Engine {
   // operation that can move amplitudes anywhere, or a handed-out device pointer, frees all bits.
   uint64_t zmask_ = 0, zval_ = 0;
   bool pointer_out_ = false;  // device_state handed the state out; it may be written until the
-                              // next call that applies gates, allocates or frees qubits
+                              // next call that applies gates, allocates or frees qubits, or measures
   void subspace_unknown() { zmask_ = zval_ = 0; }
   void subspace_fix(uint64_t mask, uint64_t val) {
     if (pointer_out_) return;
@@ -226,8 +228,9 @@ class Engine {
   static constexpr int kResults = 64;  // doubles in h_result_
   int *d_flags_ = nullptr, *h_flags_ = nullptr;
   unsigned long long *d_key_ = nullptr, *h_key_ = nullptr;
-  double *d_chunks_ = nullptr, *h_chunks_ = nullptr;
-  size_t chunks_cap_ = 0;
+  dev::Measurement *d_measure_ = nullptr;
+  double *d_sums_ = nullptr;  // chunk sums of a measurement
+  hipEvent_t picked_ = nullptr;
   bool profiling_ = false;
   uint64_t stat_passes_ = 0, stat_timed_ = 0;
   double stat_bytes_ = 0.0, stat_ms_ = 0.0;

@@ -193,9 +193,9 @@ __global__ __launch_bounds__(kBlock) void k_finish_sum(const double *__restrict_
   if (threadIdx.x == 0) out[j] = t;
 }
 
-// The measurement kernels run over a subspace: compact index c is the amplitude
+// The collapse runs over a subspace: compact index c is the amplitude
 // insert_zeros(c, sub) | sval, so the bits listed in `sub` are fixed to their values in sval (the
-// caller knows every amplitude outside is zero).  With sub.count = 0 they cover the whole state.
+// caller knows every amplitude outside is zero).  With sub.count = 0 it covers the whole state.
 template <typename R>
 __global__ __launch_bounds__(kBlock) void k_collapse(amp_t<R> *__restrict__ psi, uint64_t n_sub, BitInsert sub,
                                                      uint64_t sval, uint64_t mask, uint64_t val, double scale) {
@@ -206,81 +206,6 @@ __global__ __launch_bounds__(kBlock) void k_collapse(amp_t<R> *__restrict__ psi,
     if ((i & mask) != val) a = make_amp<R>(0.0, 0.0);
     else a = make_amp<R>(re(a) * scale, im(a) * scale);
     psi[i] = a;
-  }
-}
-
-template <typename R>
-__global__ __launch_bounds__(kBlock) void k_chunk_norms(const amp_t<R> *__restrict__ psi, BitInsert sub,
-                                                        uint64_t sval, int chunk_log2, double *sums) {
-  __shared__ double lds[kBlock / 64];
-  const uint64_t base = (uint64_t)blockIdx.x << chunk_log2;
-  const uint64_t len = uint64_t(1) << chunk_log2;
-  double acc = 0.0;
-  for (uint64_t j = threadIdx.x; j < len; j += blockDim.x) {
-    amp_t<R> a = psi[insert_zeros(base + j, sub) | sval];
-    double x = re(a), y = im(a);
-    acc = fma(x, x, fma(y, y, acc));
-  }
-  double t = block_sum(acc, lds);
-  if (threadIdx.x == 0) sums[blockIdx.x] = t;
-}
-
-// One workgroup: thread t owns the contiguous slice [t*per, (t+1)*per) of the chunk (compact
-// indices of the subspace); the picked compact index goes to *pick.
-template <typename R>
-__global__ __launch_bounds__(kBlock) void k_chunk_pick(const amp_t<R> *__restrict__ psi, BitInsert sub,
-                                                       uint64_t sval, uint64_t start, uint64_t len, double base,
-                                                       double rnd, unsigned long long *pick) {
-  __shared__ double part[kBlock];
-  const uint64_t per = (len + kBlock - 1) / kBlock;
-  const uint64_t lo = min<uint64_t>(len, threadIdx.x * per), hi = min<uint64_t>(len, lo + per);
-  double mine = 0.0;
-  for (uint64_t j = lo; j < hi; ++j) {
-    amp_t<R> a = psi[insert_zeros(start + j, sub) | sval];
-    double x = re(a), y = im(a);
-    mine += x * x + y * y;
-  }
-  part[threadIdx.x] = mine;
-  __syncthreads();
-  if (threadIdx.x == 0) {  // exclusive prefix in slice order
-    double run = base;
-    for (int t = 0; t < kBlock; ++t) {
-      double v = part[t];
-      part[t] = run;
-      run += v;
-    }
-  }
-  __syncthreads();
-  double run = part[threadIdx.x];
-  for (uint64_t j = lo; j < hi; ++j) {
-    amp_t<R> a = psi[insert_zeros(start + j, sub) | sval];
-    double x = re(a), y = im(a);
-    run += x * x + y * y;
-    if (run >= rnd) {
-      atomicMin(pick, (unsigned long long)(start + j));
-      break;
-    }
-  }
-}
-
-template <typename R>
-__global__ __launch_bounds__(kBlock) void k_classical_flags(const amp_t<R> *__restrict__ psi,
-                                                            uint64_t n, int p, double tol,
-                                                            int *flags) {
-  int lo = 0, hi = 0;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    amp_t<R> a = psi[i];
-    double x = re(a), y = im(a);
-    int big = (x * x + y * y) > tol;
-    if ((i >> p) & 1) hi |= big;
-    else lo |= big;
-  }
-  lo = __syncthreads_or(lo);
-  hi = __syncthreads_or(hi);
-  if (threadIdx.x == 0) {
-    if (lo) atomicOr(&flags[0], 1);
-    if (hi) atomicOr(&flags[1], 1);
   }
 }
 
@@ -747,29 +672,6 @@ void collapse(amp_t<R> *psi, uint64_t n_sub, const BitInsert &sub, uint64_t sval
 }
 
 template <typename R>
-void chunk_norms(const amp_t<R> *psi, uint64_t n_sub, const BitInsert &sub, uint64_t sval, int chunk_log2,
-                 double *sums, hipStream_t s) {
-  uint64_t chunks = n_sub >> chunk_log2;
-  hipLaunchKernelGGL(k_chunk_norms<R>, dim3((unsigned)chunks), dim3(kBlock), 0, s, psi, sub, sval, chunk_log2,
-                     sums);
-  QS_HIP(hipGetLastError());
-}
-
-template <typename R>
-void chunk_pick(const amp_t<R> *psi, const BitInsert &sub, uint64_t sval, uint64_t start, uint64_t len, double base,
-                double rnd, unsigned long long *pick, hipStream_t s) {
-  hipLaunchKernelGGL(k_chunk_pick<R>, dim3(1), dim3(kBlock), 0, s, psi, sub, sval, start, len, base, rnd, pick);
-  QS_HIP(hipGetLastError());
-}
-
-template <typename R>
-void classical_flags(const amp_t<R> *psi, uint64_t n, int p, double tol, int *flags, hipStream_t s) {
-  hipLaunchKernelGGL(k_classical_flags<R>, dim3(grid_for(n)), dim3(kBlock), 0, s, psi, n, p, tol,
-                     flags);
-  QS_HIP(hipGetLastError());
-}
-
-template <typename R>
 void first_pair(const amp_t<R> *psi, uint64_t n_pairs, int p, double tol, unsigned long long *key,
                 hipStream_t s) {
   hipLaunchKernelGGL(k_first_pair<R>, dim3(grid_for(n_pairs)), dim3(kBlock), 0, s, psi, n_pairs, p,
@@ -908,11 +810,6 @@ template void convert_amps<float, double>(const amp_t<float> *, amp_t<double> *,
                                hipStream_t);                                                      \
   template void collapse<R>(amp_t<R> *, uint64_t, const BitInsert &, uint64_t, uint64_t, uint64_t, double,    \
                             hipStream_t);                                                         \
-  template void chunk_norms<R>(const amp_t<R> *, uint64_t, const BitInsert &, uint64_t, int, double *,        \
-                               hipStream_t);                                                      \
-  template void chunk_pick<R>(const amp_t<R> *, const BitInsert &, uint64_t, uint64_t, uint64_t, double,      \
-                              double, unsigned long long *, hipStream_t);                         \
-  template void classical_flags<R>(const amp_t<R> *, uint64_t, int, double, int *, hipStream_t);  \
   template void first_pair<R>(const amp_t<R> *, uint64_t, int, double, unsigned long long *,      \
                               hipStream_t);                                                       \
   template void drop_bit<R>(const amp_t<R> *, amp_t<R> *, uint64_t, int, int, hipStream_t);       \

@@ -1,0 +1,340 @@
+// Measurement on the device: the pick of the reference's serial scan (simulator.hpp:145-186), the
+// projection and the renormalisation, with one wait of the host (for the outcome) per measurement.
+//
+// All(Measure) measures qubit by qubit, and each measurement halves what the next one reads, so
+// most of them are short and their cost was latency: three host round trips and three copies each.
+// 27 qubits complex64, 8 probabilities and All(Measure): 22.3 ms before, 5.7 ms now; measuring and
+// freeing 10 qubits with the rest of a variational step: 1.93 and 1.22 ms.
+// Large subspaces are read once for the chunk sums (split by the measured bit, so that the norm of
+// the outcome needs no second read) and written once by the collapse, which does not load what it
+// clears; up to 4096 amplitudes one workgroup does everything.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "kernels.hpp"
+#include "measure.hpp"
+
+namespace qs {
+namespace dev {
+namespace {
+
+__device__ __forceinline__ uint64_t insert_zeros(uint64_t g, const BitInsert &ins) {
+  for (uint32_t i = 0; i < ins.count; ++i) {
+    const uint32_t p = ins.pos[i];
+    g = ((g >> p) << (p + 1)) | (g & ((uint64_t(1) << p) - 1));
+  }
+  return g;
+}
+template <typename A>
+__device__ __forceinline__ double norm2(const A &a) {
+  const double x = a.x, y = a.y;
+  return fma(x, x, y * y);
+}
+
+// Sum over a workgroup of NT threads, valid in every thread.
+template <int NT>
+__device__ __forceinline__ double sum_all(double v, double *lds) {
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double t = 0.0;
+  for (int w = 0; w < NT / 64; ++w) t += lds[w];
+  __syncthreads();
+  return t;
+}
+// Exclusive prefix sum in thread order; *total is the sum.
+template <int NT>
+__device__ __forceinline__ double prefix(double v, double *lds, double *total) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double incl = v;
+  for (int off = 1; off < 64; off <<= 1) {
+    const double o = __shfl_up(incl, off, 64);
+    if (lane >= off) incl += o;
+  }
+  if (lane == 63) lds[wave] = incl;
+  __syncthreads();
+  double before = 0.0, all = 0.0;
+  for (int w = 0; w < NT / 64; ++w) {
+    if (w < wave) before += lds[w];
+    all += lds[w];
+  }
+  __syncthreads();
+  *total = all;
+  const double excl = __shfl_up(incl, 1, 64);
+  return before + (lane ? excl : 0.0);
+}
+
+// The outcome of a pick contradicts the fixed bits only in the reference's edge cases (a draw of 0 or
+// beyond the total): no amplitude is left then.
+__device__ __forceinline__ bool contradicts(const MeasureArgs &a, uint64_t pick) {
+  return ((pick ^ a.sval) & a.mask & a.zmask) != 0;
+}
+
+// The in-order scan of `len` compact indices from `start` by a workgroup of NT threads: the first index
+// at which base + running norm reaches the draw, ~0 if none.  *total: base + their norm.
+template <typename R, int NT>
+__device__ __forceinline__ unsigned long long scan_pick(const amp_t<R> *psi, const MeasureArgs &a, uint64_t start,
+                                                        uint64_t len, double base, double *lds, unsigned long long *found,
+                                                        double *total) {
+  const uint64_t per = (len + NT - 1) / NT;
+  const uint64_t lo = min<uint64_t>(len, threadIdx.x * per), hi = min<uint64_t>(len, lo + per);
+  double mine = 0.0;
+  for (uint64_t j = lo; j < hi; ++j) mine += norm2(psi[insert_zeros(start + j, a.sub) | a.sval]);
+  if (threadIdx.x == 0) *found = ~0ull;
+  double sum;
+  double run = base + prefix<NT>(mine, lds, &sum);  // its barriers order *found before the scan
+  *total = base + sum;
+  for (uint64_t j = lo; j < hi; ++j) {
+    run += norm2(psi[insert_zeros(start + j, a.sub) | a.sval]);
+    if (run >= a.rnd) {
+      atomicMin(found, (unsigned long long)(start + j));
+      break;
+    }
+  }
+  __syncthreads();
+  return *found;
+}
+
+template <typename R>
+__global__ __launch_bounds__(kBlock) void k_measure_small(amp_t<R> *__restrict__ psi, MeasureArgs a,
+                                                          unsigned long long *__restrict__ host_pick) {
+  __shared__ double lds[kBlock / 64];
+  __shared__ unsigned long long found;
+  uint64_t pick = ~uint64_t(0);
+  if (a.rnd > 0.0) {
+    double total;
+    const unsigned long long c = scan_pick<R, kBlock>(psi, a, 0, a.n_sub, 0.0, lds, &found, &total);
+    if (c != ~0ull) pick = insert_zeros(c, a.sub) | a.sval;
+    else pick = total >= a.rnd ? insert_zeros(a.n_sub - 1, a.sub) | a.sval : a.n_amps - 1;
+  }
+  if (threadIdx.x == 0) *host_pick = pick;
+  const uint64_t val = pick & a.mask;
+  double kept = 0.0;
+  if (!contradicts(a, pick))
+    for (uint64_t c = threadIdx.x; c < a.n_sub; c += kBlock) {
+      const uint64_t i = insert_zeros(c, a.sub) | a.sval;
+      if ((i & a.mask) == val) kept += norm2(psi[i]);
+    }
+  const double scale = 1.0 / sqrt(sum_all<kBlock>(kept, lds));
+  for (uint64_t c = threadIdx.x; c < a.n_sub; c += kBlock) {
+    const uint64_t i = insert_zeros(c, a.sub) | a.sval;
+    amp_t<R> v;
+    v.x = v.y = 0;
+    if ((i & a.mask) == val) {
+      v = psi[i];
+      v.x = (R)((double)v.x * scale);
+      v.y = (R)((double)v.y * scale);
+    }
+    psi[i] = v;
+  }
+}
+
+// sums[2c], sums[2c + 1] <- norms of chunk c (2^lg compact indices) with the measured bit clear and set
+// (of a mask of several bits: all of them set, or not)
+template <typename R>
+__global__ __launch_bounds__(kBlock) void k_measure_chunks(const amp_t<R> *__restrict__ psi, MeasureArgs a, int lg,
+                                                           double *__restrict__ sums) {
+  __shared__ double lds[kBlock / 64];
+  const uint64_t base = (uint64_t)blockIdx.x << lg, len = uint64_t(1) << lg;
+  double clear = 0.0, set = 0.0;
+  for (uint64_t j = threadIdx.x; j < len; j += kBlock) {
+    const uint64_t i = insert_zeros(base + j, a.sub) | a.sval;
+    const double v = norm2(psi[i]);
+    if ((i & a.mask) == a.mask) set += v;
+    else clear += v;
+  }
+  clear = sum_all<kBlock>(clear, lds);
+  set = sum_all<kBlock>(set, lds);
+  if (threadIdx.x == 0) {
+    sums[2 * blockIdx.x] = clear;
+    sums[2 * blockIdx.x + 1] = set;
+  }
+}
+
+// One workgroup: the chunk that reaches the draw, the pick inside it, and for one measured qubit the
+// norm of its outcome.
+constexpr int kPickThreads = 1024;
+template <typename R>
+__global__ __launch_bounds__(kPickThreads) void k_measure_pick(const amp_t<R> *__restrict__ psi, MeasureArgs a, int lg,
+                                                               uint32_t chunks, const double *__restrict__ sums, int single,
+                                                               Measurement *__restrict__ m,
+                                                               unsigned long long *__restrict__ host_pick) {
+  __shared__ double lds[kPickThreads / 64];
+  __shared__ unsigned long long found;
+  __shared__ double before;
+  uint64_t pick = ~uint64_t(0);
+  if (a.rnd > 0.0) {
+    const uint32_t per = (chunks + kPickThreads - 1) / kPickThreads;
+    const uint32_t lo = min(chunks, threadIdx.x * per), hi = min(chunks, lo + per);
+    double mine = 0.0;
+    for (uint32_t c = lo; c < hi; ++c) mine += sums[2 * c] + sums[2 * c + 1];
+    if (threadIdx.x == 0) found = ~0ull;
+    double total;
+    const double start = prefix<kPickThreads>(mine, lds, &total);
+    double run = start;
+    for (uint32_t c = lo; c < hi; ++c) {
+      run += sums[2 * c] + sums[2 * c + 1];
+      if (run >= a.rnd) {
+        atomicMin(&found, (unsigned long long)c);
+        break;
+      }
+    }
+    __syncthreads();
+    const unsigned long long chunk = found;
+    if (chunk == ~0ull) {
+      pick = a.n_amps - 1;  // the draw exceeds the total norm: the scan runs off the end
+    } else {
+      if (chunk >= lo && chunk < hi) {
+        double r = start;
+        for (uint32_t c = lo; c < chunk; ++c) r += sums[2 * c] + sums[2 * c + 1];
+        before = r;
+      }
+      __syncthreads();
+      const uint64_t len = uint64_t(1) << lg;
+      const unsigned long long c =
+          scan_pick<R, kPickThreads>(psi, a, chunk * len, len, before, lds, &found, &total);
+      pick = insert_zeros(c != ~0ull ? (uint64_t)c : (chunk + 1) * len - 1, a.sub) | a.sval;
+    }
+  }
+  double kept = 0.0;
+  if (single && !contradicts(a, pick)) {
+    const uint32_t set = (pick & a.mask) ? 1 : 0;
+    for (uint32_t c = threadIdx.x; c < chunks; c += kPickThreads) kept += sums[2 * c + set];
+  }
+  kept = sum_all<kPickThreads>(kept, lds);
+  if (threadIdx.x == 0) {
+    m->pick = pick;
+    m->scale = 1.0 / sqrt(kept);
+    *host_pick = pick;
+  }
+}
+
+// Several measured qubits: the norm of the outcome over the subspace, then its scale.
+template <typename R>
+__global__ __launch_bounds__(kBlock) void k_measure_kept(const amp_t<R> *__restrict__ psi, MeasureArgs a,
+                                                         const Measurement *__restrict__ m, double *__restrict__ partials) {
+  __shared__ double lds[kBlock / 64];
+  const uint64_t pick = m->pick, val = pick & a.mask;
+  double kept = 0.0;
+  if (!contradicts(a, pick))
+    for (uint64_t c = (uint64_t)blockIdx.x * kBlock + threadIdx.x; c < a.n_sub; c += (uint64_t)gridDim.x * kBlock) {
+      const uint64_t i = insert_zeros(c, a.sub) | a.sval;
+      if ((i & a.mask) == val) kept += norm2(psi[i]);
+    }
+  kept = sum_all<kBlock>(kept, lds);
+  if (threadIdx.x == 0) partials[blockIdx.x] = kept;
+}
+__global__ __launch_bounds__(kBlock) void k_measure_scale(const double *__restrict__ partials, Measurement *__restrict__ m) {
+  __shared__ double lds[kBlock / 64];
+  double kept = 0.0;
+  for (int b = threadIdx.x; b < kReduceGrid; b += kBlock) kept += partials[b];
+  kept = sum_all<kBlock>(kept, lds);
+  if (threadIdx.x == 0) m->scale = 1.0 / sqrt(kept);
+}
+
+template <typename R>
+__global__ __launch_bounds__(kBlock) void k_measure_collapse(amp_t<R> *__restrict__ psi, MeasureArgs a,
+                                                             const Measurement *__restrict__ m) {
+  const uint64_t val = m->pick & a.mask;
+  const double scale = m->scale;
+  for (uint64_t c = (uint64_t)blockIdx.x * kBlock + threadIdx.x; c < a.n_sub; c += (uint64_t)gridDim.x * kBlock) {
+    const uint64_t i = insert_zeros(c, a.sub) | a.sval;
+    amp_t<R> v;
+    v.x = v.y = 0;
+    if ((i & a.mask) == val) {
+      v = psi[i];
+      v.x = (R)((double)v.x * scale);
+      v.y = (R)((double)v.y * scale);
+    }
+    psi[i] = v;
+  }
+}
+
+// SMALL: one workgroup, which writes the answer itself.
+template <typename R, bool SMALL>
+__global__ __launch_bounds__(kBlock) void k_classical(const amp_t<R> *__restrict__ psi, uint64_t n_sub, BitInsert sub,
+                                                      uint64_t sval, int p, double tol, int *__restrict__ count,
+                                                      int *__restrict__ flags) {
+  int lo = 0, hi = 0;
+  for (uint64_t c = (uint64_t)blockIdx.x * kBlock + threadIdx.x; c < n_sub; c += (uint64_t)gridDim.x * kBlock) {
+    const uint64_t i = insert_zeros(c, sub) | sval;
+    const amp_t<R> v = psi[i];
+    const double x = v.x, y = v.y;
+    const int big = (x * x + y * y) > tol;
+    if ((i >> p) & 1) hi |= big;
+    else lo |= big;
+  }
+  lo = __syncthreads_or(lo);
+  hi = __syncthreads_or(hi);
+  if (threadIdx.x == 0) {
+    if (SMALL) {
+      *flags = (lo ? 1 : 0) | (hi ? 2 : 0);
+    } else {
+      if (lo) atomicOr(&count[0], 1);
+      if (hi) atomicOr(&count[1], 1);
+    }
+  }
+}
+__global__ void k_classical_clear(int *count) { count[threadIdx.x] = 0; }
+__global__ void k_classical_flags(const int *__restrict__ count, int *__restrict__ flags) {
+  *flags = (count[0] ? 1 : 0) | (count[1] ? 2 : 0);
+}
+
+unsigned grid_of(uint64_t work) { return (unsigned)std::min<uint64_t>(16384, std::max<uint64_t>(1, (work + kBlock - 1) / kBlock)); }
+
+}  // namespace
+
+template <typename R>
+void measure(amp_t<R> *psi, const MeasureArgs &a, Measurement *m, unsigned long long *pick, double *sums, double *partials,
+             hipEvent_t picked, hipStream_t s) {
+  if (a.n_sub <= kMeasureSmall) {
+    hipLaunchKernelGGL(k_measure_small<R>, dim3(1), dim3(kBlock), 0, s, psi, a, pick);
+    QS_HIP(hipGetLastError());
+    QS_HIP(hipEventRecord(picked, s));
+    return;
+  }
+  int lg = 12;
+  while ((a.n_sub >> lg) > kMeasureChunks) ++lg;
+  const uint32_t chunks = (uint32_t)(a.n_sub >> lg);
+  const int single = a.mask != 0 && (a.mask & (a.mask - 1)) == 0;
+  hipLaunchKernelGGL(k_measure_chunks<R>, dim3(chunks), dim3(kBlock), 0, s, psi, a, lg, sums);
+  QS_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_measure_pick<R>, dim3(1), dim3(kPickThreads), 0, s, psi, a, lg, chunks, sums, single, m, pick);
+  QS_HIP(hipGetLastError());
+  QS_HIP(hipEventRecord(picked, s));
+  if (!single) {
+    hipLaunchKernelGGL(k_measure_kept<R>, dim3(kReduceGrid), dim3(kBlock), 0, s, psi, a, m, partials);
+    QS_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_measure_scale, dim3(1), dim3(kBlock), 0, s, partials, m);
+    QS_HIP(hipGetLastError());
+  }
+  hipLaunchKernelGGL(k_measure_collapse<R>, dim3(grid_of(a.n_sub)), dim3(kBlock), 0, s, psi, a, m);
+  QS_HIP(hipGetLastError());
+}
+
+template <typename R>
+void classical(const amp_t<R> *psi, uint64_t n_sub, const BitInsert &sub, uint64_t sval, int p, double tol, int *count,
+               int *flags, hipStream_t s) {
+  if (n_sub <= 4 * kMeasureSmall) {
+    hipLaunchKernelGGL((k_classical<R, true>), dim3(1), dim3(kBlock), 0, s, psi, n_sub, sub, sval, p, tol, count, flags);
+    QS_HIP(hipGetLastError());
+    return;
+  }
+  hipLaunchKernelGGL(k_classical_clear, dim3(1), dim3(2), 0, s, count);
+  QS_HIP(hipGetLastError());
+  hipLaunchKernelGGL((k_classical<R, false>), dim3(grid_of(n_sub)), dim3(kBlock), 0, s, psi, n_sub, sub, sval, p, tol, count, flags);
+  QS_HIP(hipGetLastError());
+  hipLaunchKernelGGL(k_classical_flags, dim3(1), dim3(1), 0, s, count, flags);
+  QS_HIP(hipGetLastError());
+}
+
+#define QS_INSTANTIATE_MEASURE(R)                                                                                       \
+  template void measure<R>(amp_t<R> *, const MeasureArgs &, Measurement *, unsigned long long *, double *, double *,   \
+                           hipEvent_t, hipStream_t);                                                                    \
+  template void classical<R>(const amp_t<R> *, uint64_t, const BitInsert &, uint64_t, int, double, int *, int *, hipStream_t);
+QS_INSTANTIATE_MEASURE(double)
+QS_INSTANTIATE_MEASURE(float)
+
+}  // namespace dev
+}  // namespace qs

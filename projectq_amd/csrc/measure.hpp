@@ -1,0 +1,43 @@
+// Launchers of the measurement kernels (measure.hip).
+#pragma once
+
+#include "common.hpp"
+
+namespace qs {
+namespace dev {
+
+// What one measurement leaves on the device for its collapse: the picked index and the factor of the
+// amplitudes that stay.
+struct Measurement {
+  unsigned long long pick;
+  double scale;
+};
+
+// Chunks of a measurement's first pass, at most.
+constexpr uint32_t kMeasureChunks = 32768;
+// Subspaces up to this size are measured by one workgroup in one launch.
+constexpr uint64_t kMeasureSmall = 4096;
+
+struct MeasureArgs {
+  uint64_t n_amps, n_sub;  // amplitudes of the state, and of the subspace outside which they are zero
+  BitInsert sub;           // the subspace's fixed bits
+  uint64_t sval, zmask;    // their values, and their mask
+  uint64_t mask;           // index bits of the measured qubits
+  double rnd;              // the draw; 0: the reference's loop never runs and the pick is all ones
+};
+
+// Pick (the first index whose running norm reaches the draw), projection and renormalisation.  m: one
+// record in device memory; pick: pinned, written before `picked` is recorded; sums: 2 kMeasureChunks
+// doubles; partials: kReduceGrid doubles.
+template <typename R>
+void measure(amp_t<R> *psi, const MeasureArgs &a, Measurement *m, unsigned long long *pick, double *sums, double *partials,
+             hipEvent_t picked, hipStream_t s);
+
+// *flags (pinned) <- bit 0: an amplitude > tol with index bit p clear, bit 1: one with it set, over the
+// subspace.  count: two ints of device memory.
+template <typename R>
+void classical(const amp_t<R> *psi, uint64_t n_sub, const BitInsert &sub, uint64_t sval, int p, double tol, int *count,
+               int *flags, hipStream_t s);
+
+}  // namespace dev
+}  // namespace qs
