@@ -122,7 +122,7 @@ int qs_get_expectation_value(qs_simulator *sim, const uint32_t *term_idx, const 
  * amplitudes at `device_state` on the current GPU (complex128 for QS_C128, complex64 for QS_C64,
  * e.g. from qs_device_state); local index l of a string is the qubit at bit position
  * positions[l].  Allocates no device or host memory: the strings, partial sums and per-string
- * results use a fixed 49 KiB device array per GPU (held until the process ends).  At most 4096
+ * results use a fixed 51 KiB device array per GPU (held until the process ends).  At most 4096
  * strings per call (QS_ERR_VALUE beyond).  Synchronous on the null stream; calls that overlap on
  * one GPU share that array and race. */
 int qs_expectation_value_noalloc(const void *device_state, uint32_t n_qubits, int precision,

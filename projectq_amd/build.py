@@ -52,6 +52,7 @@ SOURCES = [
     "kernels.hip",
     "math.hip",
     "energy.hip",
+    "pauli_sum.hip",
     "measure.hip",
     "mlp.hip",
     "compare.hip",

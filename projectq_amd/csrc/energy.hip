@@ -16,7 +16,8 @@
 // What bounds it: FP64 issue (a conversion, two FMAs of the pair and one per string) while a few
 // passes of 5 TB/s reads hide behind it.  Tile: 32 KiB, so four or five workgroups share a CU and
 // one loads while the others compute; 256-byte segments, the shortest that stream at the full rate.
-// 28 qubits complex64, 40 random strings: 22.4 ms string by string, 3.7 ms from tiles (6 passes).
+// 28 qubits complex64, 40 random strings: 22.4 ms string by string, 3.7 ms from tiles (6 passes), 3.0 ms
+// with one kernel arm per kind and the next group's record loaded ahead.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -56,40 +57,50 @@ __device__ __forceinline__ double workgroup_total(const Compensated &a, double *
   return t;
 }
 
-// v[j] <- Re or Im of conj(a_j) b_j over the j without bit HB (HB = 0: every j), b_j the partner,
-// and one weighted sum per string.
-template <typename R, int NJ, int HB>
+// One group of kind IM: v[j] <- Re or Im of conj(a_j) b_j over the j without bit HB (HB = 0: every j), b_j
+// the partner, and one weighted sum per string.
+template <typename R, int NJ, int HB, bool IM>
 __device__ __forceinline__ void energy_group(const amp_t<R> *__restrict__ tile, const double *__restrict__ ar,
-                                             const double *__restrict__ ai, uint32_t mask, const EnergyString *st,
-                                             uint32_t n_re, uint32_t n_im, uint64_t base, Compensated &acc) {
+                                             const double *__restrict__ ai, const EnergyGroup &g,
+                                             const EnergyString *__restrict__ strings, uint64_t base, Compensated &acc) {
   const uint32_t tid = threadIdx.x;
-  const uint32_t lo = tid ^ (mask & 255u), mj = mask & ~255u;
-#pragma unroll 1
-  for (int kind = 0; kind < 2; ++kind) {
-    const uint32_t count = kind ? n_im : n_re;
-    if (count == 0) continue;
-    double v[NJ];
+  const uint32_t lo = tid ^ (g.mask & 255u), mj = g.mask & ~255u;
+  double v[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    if (HB && (j & HB)) continue;
+    const amp_t<R> b = tile[lo | (((uint32_t)j << 8) ^ mj)];
+    const double br = b.x, bi = b.y;
+    v[j] = IM ? fma(ar[j], bi, -ai[j] * br) : fma(ar[j], br, ai[j] * bi);
+  }
+  auto string = [&](const EnergyString &st) {
+    const double w = flip(st.w, (uint32_t)__popcll(base & st.z) & 1u);
+    const uint32_t zj = st.zloc >> 8;
+    double sum = 0.0;
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
       if (HB && (j & HB)) continue;
-      const amp_t<R> b = tile[lo | (((uint32_t)j << 8) ^ mj)];
-      const double br = b.x, bi = b.y;
-      v[j] = kind ? fma(ar[j], bi, -ai[j] * br) : fma(ar[j], br, ai[j] * bi);
+      sum = fma(flip(w, (uint32_t)__popc((uint32_t)j & zj) & 1u), v[j], sum);
     }
-    for (uint32_t s = 0; s < count; ++s, ++st) {
-      const uint32_t zl = st->zloc;
-      const uint32_t odd = (uint32_t)__popcll(base & st->z) & 1u;
-      const double w = flip(st->w, odd);
-      const uint32_t zj = zl >> 8;
-      double sum = 0.0;
-#pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        if (HB && (j & HB)) continue;
-        sum = fma(flip(w, (uint32_t)__popc((uint32_t)j & zj) & 1u), v[j], sum);
-      }
-      acc.add(flip(sum, (uint32_t)__popc(tid & zl) & 1u));
-    }
-  }
+    acc.add(flip(sum, (uint32_t)__popc(tid & st.zloc) & 1u));
+  };
+  string(g.head);
+#pragma unroll 2
+  for (uint32_t s = 0; s < g.more; ++s) string(strings[g.next + s]);
+}
+
+template <typename R, int LJ, bool IM>
+__device__ __forceinline__ void energy_kind(const amp_t<R> *__restrict__ tile, const double *__restrict__ ar,
+                                            const double *__restrict__ ai, const EnergyGroup &g,
+                                            const EnergyString *__restrict__ strings, uint64_t base, Compensated &acc) {
+  constexpr int NJ = 1 << LJ;
+  const uint32_t mj = g.mask >> 8;
+  const int hb = mj ? 31 - __clz(mj) : -1;  // uniform
+  if (hb < 0) energy_group<R, NJ, 0, IM>(tile, ar, ai, g, strings, base, acc);
+  if constexpr (LJ > 0) if (hb == 0) energy_group<R, NJ, 1, IM>(tile, ar, ai, g, strings, base, acc);
+  if constexpr (LJ > 1) if (hb == 1) energy_group<R, NJ, 2, IM>(tile, ar, ai, g, strings, base, acc);
+  if constexpr (LJ > 2) if (hb == 2) energy_group<R, NJ, 4, IM>(tile, ar, ai, g, strings, base, acc);
+  if constexpr (LJ > 3) if (hb == 3) energy_group<R, NJ, 8, IM>(tile, ar, ai, g, strings, base, acc);
 }
 
 // LJ = log2 of the amplitudes per thread.  Workgroup b works on pass b / per_pass, on the tiles
@@ -143,19 +154,14 @@ __global__ __launch_bounds__(kEnergyThreads) void k_energy(const amp_t<R> *__res
       ai[j] = (double)a[j].y;
     }
     __syncthreads();
+    // the next group's record loads while this one computes
+    const EnergyGroup *gp = groups + pass.first_group;
+    EnergyGroup cur = *gp;
     for (uint32_t g = 0; g < pass.n_groups; ++g) {
-      const EnergyGroup &gr = groups[pass.first_group + g];
-      const EnergyString *st = strings + gr.first;
-      const uint32_t m = gr.mask, mj = m >> 8;
-      if (mj == 0) {
-        energy_group<R, NJ, 0>(tile, ar, ai, m, st, gr.n_re, gr.n_im, base, acc);
-      } else {
-        const int hb = 31 - __clz(mj);
-        if constexpr (LJ > 0) if (hb == 0) energy_group<R, NJ, 1>(tile, ar, ai, m, st, gr.n_re, gr.n_im, base, acc);
-        if constexpr (LJ > 1) if (hb == 1) energy_group<R, NJ, 2>(tile, ar, ai, m, st, gr.n_re, gr.n_im, base, acc);
-        if constexpr (LJ > 2) if (hb == 2) energy_group<R, NJ, 4>(tile, ar, ai, m, st, gr.n_re, gr.n_im, base, acc);
-        if constexpr (LJ > 3) if (hb == 3) energy_group<R, NJ, 8>(tile, ar, ai, m, st, gr.n_re, gr.n_im, base, acc);
-      }
+      const EnergyGroup next = *++gp;
+      if (cur.kind) energy_kind<R, LJ, true>(tile, ar, ai, cur, strings, base, acc);
+      else energy_kind<R, LJ, false>(tile, ar, ai, cur, strings, base, acc);
+      cur = next;
     }
   }
   const double total = workgroup_total<kEnergyThreads>(acc, sums);

@@ -46,14 +46,39 @@ struct Span {
 
 }  // namespace
 
+namespace {
+
+// The tile of an n-qubit state: at most 2^tmax amplitudes, 256 contiguous bytes.  Small states take
+// the tile that holds them.
+void tile_of(unsigned n, bool c64, uint32_t tmax, uint32_t *t, uint32_t *L, uint32_t *h) {
+  const uint32_t lmin = c64 ? 5u : 4u;
+  *t = std::max(8u, std::min(tmax, n));
+  *L = n <= *t ? *t : lmin;
+  *h = *t - *L;
+}
+
+// fills the span up to h generators with the lowest positions it lacks; its pivots, ascending
+void complete(Span &span, uint64_t *gen, uint32_t L, uint32_t h, uint8_t *pivot) {
+  for (uint32_t p = L; span.n < (int)h; ++p) {
+    uint32_t combo;
+    const uint64_t rest = span.reduce(uint64_t(1) << p, &combo);
+    if (!rest) continue;
+    gen[span.n] = uint64_t(1) << p;
+    span.add(rest, combo);
+  }
+  for (uint32_t b = 0; b < h; ++b) {
+    const uint8_t p = (uint8_t)top_bit(span.row[b]);
+    uint32_t at = b;
+    for (; at > 0 && pivot[at - 1] > p; --at) pivot[at] = pivot[at - 1];
+    pivot[at] = p;
+  }
+}
+
+}  // namespace
+
 void plan_energy(const EnergyTerm *terms, int count, unsigned n, bool c64, EnergyPlan &plan) {
-  // Tile: 32 KiB of LDS, 256 threads with 16 (complex64) or 8 (complex128) amplitudes each; 256
-  // contiguous bytes.  Small states take the tile that holds them.
-  const uint32_t tmax = c64 ? 12u : 11u, lmin = c64 ? 5u : 4u;
-  plan.t = std::max(8u, std::min(tmax, n));
-  plan.L = std::min(lmin, n);
-  if (n <= plan.t) plan.L = plan.t;
-  plan.h = plan.t - plan.L;
+  tile_of(n, c64, c64 ? 12u : 11u, &plan.t, &plan.L, &plan.h);
+  // 32 KiB of LDS, 256 threads with 16 (complex64) or 8 (complex128) amplitudes each
   plan.n_passes = plan.n_groups = plan.n_strings = 0;
 
   // order by x, real kinds first
@@ -123,19 +148,7 @@ void plan_energy(const EnergyTerm *terms, int count, unsigned n, bool c64, Energ
     // visits each pair once; a string whose x lies in the others alone would visit both members.  So
     // each of the others carries one of the first ones: gen_k ^ gen_{k mod top_h}.
     const int from_strings = span.n;
-    for (uint32_t p = plan.L; span.n < (int)plan.h; ++p) {
-      uint32_t combo;
-      const uint64_t rest = span.reduce(uint64_t(1) << p, &combo);
-      if (!rest) continue;
-      gen[span.n] = uint64_t(1) << p;
-      span.add(rest, combo);
-    }
-    for (uint32_t b = 0; b < plan.h; ++b) {
-      uint8_t p = (uint8_t)top_bit(span.row[b]);
-      uint32_t at = b;
-      for (; at > 0 && pass.pivot[at - 1] > p; --at) pass.pivot[at] = pass.pivot[at - 1];
-      pass.pivot[at] = p;
-    }
+    complete(span, gen, plan.L, plan.h, pass.pivot);
     uint32_t local[kEnergyMaxGens];  // tile-local mask of generator b as a string has it
     for (uint32_t b = 0; b < plan.h; ++b) {
       const uint32_t bit = b < top_h ? plan.L + lanes_h + b : plan.L + (b - top_h);
@@ -149,27 +162,27 @@ void plan_energy(const EnergyTerm *terms, int count, unsigned n, bool c64, Energ
     }
     for (int q = 0; q < k; ++q) {
       const Group &src = g[taken[q]];
-      EnergyGroup &dst = plan.groups[plan.n_groups++];
       const EnergyTerm &lead = terms[order[src.first]];
-      dst.mask = (uint32_t)(lead.x & low);
+      uint32_t mask = (uint32_t)(lead.x & low);
       for (uint32_t b = 0; b < plan.h; ++b)
-        if ((alpha[q] >> b) & 1) dst.mask ^= local[b];
-      dst.first = plan.n_strings;
-      dst.n_re = (uint32_t)src.n_re;
-      dst.n_im = (uint32_t)src.n_im;
-      const bool once = (dst.mask >> kEnergyLaneBits) != 0;  // each pair visited once: twice the weight
-      for (int s = src.first; s < src.first + src.n_re + src.n_im; ++s) {
+        if ((alpha[q] >> b) & 1) mask ^= local[b];
+      const bool once = (mask >> kEnergyLaneBits) != 0;  // each pair visited once: twice the weight
+      auto string = [&](int s) {
         const EnergyTerm &e = terms[order[s]];
-        EnergyString &o = plan.strings[plan.n_strings++];
         // Re(omega (pr + i pi)): omega = +-1 takes +-pr, omega = +-i takes -+pi
         const bool im = parity(e.x & e.z);
         double w = e.c * (im ? -e.omega.imag() : e.omega.real());
-        if (parity(e.x & e.z)) w = -w;  // popcount(j & z) = popcount(i & z) + popcount(x & z)
-        o.w = once ? 2.0 * w : w;
-        o.z = e.z;
-        o.zloc = (uint32_t)(e.z & low);
+        if (im) w = -w;  // popcount(j & z) = popcount(i & z) + popcount(x & z)
+        EnergyString o{e.z, once ? 2.0 * w : w, (uint32_t)(e.z & low), 0};
         for (uint32_t b = 0; b < plan.h; ++b) o.zloc |= parity(pass.gen[b] & e.z) << (plan.L + b);
-        o.pad = 0;
+        return o;
+      };
+      for (uint32_t kind = 0, s = (uint32_t)src.first; kind < 2; ++kind) {
+        const uint32_t count = (uint32_t)(kind ? src.n_im : src.n_re);
+        if (count == 0) continue;
+        plan.groups[plan.n_groups++] = EnergyGroup{string((int)s), mask, kind, plan.n_strings, count - 1};
+        for (uint32_t i = 1; i < count; ++i) plan.strings[plan.n_strings++] = string((int)(s + i));
+        s += count;
       }
     }
     pass.n_groups = plan.n_groups - pass.first_group;
@@ -179,12 +192,86 @@ void plan_energy(const EnergyTerm *terms, int count, unsigned n, bool c64, Energ
 EnergyRecords pack_energy(const EnergyPlan &plan, char *out) {
   EnergyRecords r;
   r.groups = plan.n_passes * sizeof(EnergyPass);
-  r.strings = r.groups + plan.n_groups * sizeof(EnergyGroup);
+  r.strings = r.groups + (plan.n_groups + 1) * sizeof(EnergyGroup);
   r.bytes = r.strings + plan.n_strings * sizeof(EnergyString);
   std::memcpy(out, plan.passes, r.groups);
-  std::memcpy(out + r.groups, plan.groups, r.strings - r.groups);
+  std::memcpy(out + r.groups, plan.groups, plan.n_groups * sizeof(EnergyGroup));
+  std::memset(out + r.strings - sizeof(EnergyGroup), 0, sizeof(EnergyGroup));
   std::memcpy(out + r.strings, plan.strings, r.bytes - r.strings);
   return r;
+}
+
+void plan_sum(const std::vector<SumTerm> &terms, unsigned n, bool c64, SumPlan &plan) {
+  tile_of(n, c64, kSumTileBits, &plan.t, &plan.L, &plan.h);
+  plan.groups.clear();
+  plan.strings.clear();
+  const uint64_t low = (uint64_t(1) << plan.L) - 1;
+  // highest x first: the generators take the far partners, and those left to memory are near, in
+  // the L2 of the workgroup's XCD
+  std::vector<uint32_t> order(terms.size());
+  for (size_t i = 0; i < order.size(); ++i) order[i] = (uint32_t)i;
+  std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return terms[a].x > terms[b].x; });
+  Span span;
+  std::vector<uint32_t> alpha;
+  for (size_t i = 0; i < order.size();) {
+    const uint64_t x = terms[order[i]].x;
+    size_t e = i;
+    while (e < order.size() && terms[order[e]].x == x) ++e;
+    SumGroup g{};
+    g.x = x;
+    bool any = false;
+    uint32_t combo = 0;
+    for (uint32_t kind = 0; kind < 2; ++kind) {
+      g.kind = kind;
+      g.next = (uint32_t)plan.strings.size();
+      g.more = 0;
+      bool head = false;
+      for (size_t s = i; s < e; ++s) {
+        const SumTerm &t = terms[order[s]];
+        double w = kind ? t.c.imag() : t.c.real();
+        if (w == 0.0) continue;
+        if (parity(x & t.z)) w = -w;  // popcount(j & z) = popcount(i & z) + popcount(x & z)
+        const EnergyString o{t.z, w, 0, 0};
+        if (head) {
+          plan.strings.push_back(o);
+          ++g.more;
+        } else {
+          g.head = o;
+          head = true;
+        }
+      }
+      if (!head) continue;
+      if (!any) {
+        any = true;
+        const uint64_t rest = span.reduce(x & ~low, &combo);
+        g.inside = 1;
+        if (rest) {
+          if (span.n < (int)plan.h) {
+            plan.gen[span.n] = x & ~low;
+            span.add(rest, combo);
+            combo = 1u << (span.n - 1);
+          } else {
+            g.inside = 0;
+          }
+        }
+      }
+      alpha.push_back(combo);
+      plan.groups.push_back(g);
+    }
+    i = e;
+  }
+  complete(span, plan.gen, plan.L, plan.h, plan.pivot);
+  auto place = [&](EnergyString &o) {
+    o.zloc = (uint32_t)(o.z & low);
+    for (uint32_t b = 0; b < plan.h; ++b) o.zloc |= parity(plan.gen[b] & o.z) << (plan.L + b);
+  };
+  for (size_t k = 0; k < plan.groups.size(); ++k) {
+    SumGroup &g = plan.groups[k];
+    if (g.inside) g.mask = (uint32_t)(g.x & low) | alpha[k] << plan.L;
+    place(g.head);
+  }
+  for (EnergyString &o : plan.strings) place(o);
+  plan.groups.push_back(SumGroup{});
 }
 
 }  // namespace qs

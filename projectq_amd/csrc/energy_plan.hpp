@@ -6,6 +6,7 @@
 #include <complex>
 #include <cstddef>
 #include <cstdint>
+#include <vector>
 
 #include "layout.hpp"
 
@@ -25,10 +26,12 @@ struct EnergyString {
   uint32_t zloc, pad;
 };
 
-// Strings with the same x: tile-local XOR mask `mask`; strings [first, first + n_re) are of kind 0
-// and the n_im after them of kind 1.
+// Strings with the same x and the same kind: tile-local XOR mask `mask`.  The first string is in the
+// record (most x have one string, and a kernel then waits for one scalar load, not two); the others
+// are strings [next, next + more).
 struct EnergyGroup {
-  uint32_t mask, first, n_re, n_im;
+  EnergyString head;
+  uint32_t mask, kind, next, more;
 };
 
 // A pass over the state in tiles of 2^t amplitudes: the low L index bits (contiguous) and the span
@@ -45,13 +48,13 @@ struct EnergyPlan {
   uint32_t t, L, h;             // tile bits, contiguous bits, generators (t = L + h)
   uint32_t n_passes, n_groups, n_strings;
   EnergyPass passes[kEnergyMaxStrings];
-  EnergyGroup groups[kEnergyMaxStrings];
+  EnergyGroup groups[kEnergyMaxStrings + 1];  // one spare: kernels load one group ahead
   EnergyString strings[kEnergyMaxStrings];
 };
 
 // The used records of a plan, packed for one upload: passes, then groups, then strings.
 constexpr size_t kEnergyRecordBytes =
-    size_t(kEnergyMaxStrings) * (sizeof(EnergyPass) + sizeof(EnergyGroup) + sizeof(EnergyString));
+    size_t(kEnergyMaxStrings) * (sizeof(EnergyPass) + sizeof(EnergyString)) + (kEnergyMaxStrings + 1) * sizeof(EnergyGroup);
 struct EnergyRecords {
   size_t groups, strings, bytes;  // byte offsets, and the size
 };
@@ -67,5 +70,31 @@ struct EnergyTerm {
 // Plans `count` <= kEnergyMaxStrings terms on a state of n qubits.  Terms that are not Hermitian
 // are left out: the real part of their expectation value is zero.
 void plan_energy(const EnergyTerm *terms, int count, unsigned n, bool c64, EnergyPlan &plan);
+
+// ---- sum_t c_t P_t applied to a state (qubit operators and the terms of a time evolution) ----------
+
+// Strings with the same x and kind, the first in the record as in EnergyGroup: each contributes
+// w (-1)^{popcount(i & z)} psi_{i ^ x}, kind 1 times the imaginary unit (the sign (-1)^{popcount(x & z)} is
+// folded into w).  The partner is in the tile, at tile-local index ^ mask (inside), or read from memory.
+struct SumGroup {
+  EnergyString head;
+  uint64_t x;
+  uint32_t mask, kind, inside, next, more, pad;
+};
+
+constexpr uint32_t kSumTileBits = 10;
+struct SumPlan {
+  uint32_t t, L, h;  // the tile, as in EnergyPlan
+  uint64_t gen[kEnergyMaxGens];
+  uint8_t pivot[kEnergyMaxGens];
+  std::vector<SumGroup> groups;  // and one spare: kernels load one group ahead
+  std::vector<EnergyString> strings;
+};
+// c may be complex; the strings need not be Hermitian.
+struct SumTerm {
+  uint64_t x, z;
+  std::complex<double> c;  // with the string's phase
+};
+void plan_sum(const std::vector<SumTerm> &terms, unsigned n, bool c64, SumPlan &plan);
 
 }  // namespace qs

@@ -5,6 +5,7 @@
 #include "engine.hpp"
 
 #include "energy.hpp"
+#include "pauli_sum.hpp"
 #include "mfma_layout.hpp"
 
 #include <algorithm>
@@ -1197,27 +1198,58 @@ double Engine::get_expectation_value(const std::vector<PauliString> &terms,
   return total;
 }
 
+// The records of a Pauli sum in device memory: in the upload arena, or where they would crowd it in
+// memory of their own, which `own` frees after its stream has run out.
+struct Engine::SumUpload {
+  Engine &e;
+  dev::SumRecords rec{nullptr, nullptr};
+  void *own = nullptr;
+  SumUpload(Engine &engine, const SumPlan &plan) : e(engine) {
+    const size_t groups = plan.groups.size() * sizeof(SumGroup), strings = plan.strings.size() * sizeof(EnergyString);
+    if (groups + strings == 0) return;
+    std::vector<char> host(groups + strings);
+    std::memcpy(host.data(), plan.groups.data(), groups);
+    std::memcpy(host.data() + groups, plan.strings.data(), strings);
+    const char *d;
+    if (host.size() <= kArenaBytes / 4) {
+      d = (const char *)e.upload(host.data(), host.size());
+    } else {
+      QS_HIP(hipMalloc(&own, host.size()));
+      const hipError_t err = hipMemcpy(own, host.data(), host.size(), hipMemcpyHostToDevice);
+      if (err != hipSuccess) (void)hipFree(own);
+      QS_HIP(err);
+      d = (const char *)own;
+    }
+    rec.groups = (const SumGroup *)d;
+    rec.strings = (const EnergyString *)(d + groups);
+  }
+  ~SumUpload() {
+    if (!own) return;
+    (void)hipStreamSynchronize(e.stream_);
+    (void)hipFree(own);
+  }
+};
+
 // simulator.hpp:324-350: psi <- sum_t c_t P_t psi in one out-of-place pass.
 void Engine::apply_qubit_operator(const std::vector<PauliString> &terms, const std::vector<cplx> &coeffs,
                                   const std::vector<unsigned> &ids) {
   subspace_unknown();  // amplitudes may move anywhere
   run();
   check_known(ids, "apply_qubit_operator");
-  std::vector<dev::PauliTerm> pt(terms.size());
+  std::vector<SumTerm> st(terms.size());
   for (size_t t = 0; t < terms.size(); ++t) {
     cplx w;
-    pauli_encode(terms[t], ids, &pt[t].x, &pt[t].z, &w);
-    cplx c = coeffs[t] * w;
-    pt[t].c_re = c.real();
-    pt[t].c_im = c.imag();
+    pauli_encode(terms[t], ids, &st[t].x, &st[t].z, &w);
+    st[t].c = coeffs[t] * w;
   }
-  const dev::PauliTerm *d_terms =
-      pt.empty() ? nullptr : (const dev::PauliTerm *)upload(pt.data(), pt.size() * sizeof(dev::PauliTerm));
+  SumPlan plan;
+  plan_sum(st, n_, c64_, plan);
+  SumUpload up(*this, plan);
   void *dst = scratch(0);
   dispatch([&](auto tag) {
     using R = decltype(tag);
-    dev::pauli_sum<R>((const amp_t<R> *)psi_, (amp_t<R> *)dst, nullptr, amps(), d_terms, (int)pt.size(), 1.0,
-                      0.0, false, 0, d_partials_, stream_);
+    dev::pauli_sum<R>((const amp_t<R> *)psi_, (amp_t<R> *)dst, nullptr, n_, plan, up.rec, 1.0, false, 1.0, 0, nullptr,
+                      d_partials_, stream_);
   });
   std::swap(psi_, buf_[0]);
   norm_changed();
@@ -1225,7 +1257,11 @@ void Engine::apply_qubit_operator(const std::vector<PauliString> &terms, const s
 }
 
 // simulator.hpp:386-438: scaled, truncated Taylor series of exp(-i H t) on the controlled
-// subspace; each Taylor term is one pass that also accumulates the output and the update norm.
+// subspace; each Taylor term is one pass that also accumulates the output and the update norm.  The
+// device decides when a step's series ends; the host queues as many terms as the step before took and
+// then looks.  A step reads its state from psi_ and builds the next one in buf_[0] (the first term
+// writes state + term); the terms go back and forth between buf_[1] and psi_, whose amplitudes only
+// the first term needs.
 void Engine::emulate_time_evolution(const std::vector<PauliString> &terms, const std::vector<double> &coeffs,
                                     double time, const std::vector<unsigned> &ids,
                                     const std::vector<unsigned> &ctrl) {
@@ -1235,48 +1271,55 @@ void Engine::emulate_time_evolution(const std::vector<PauliString> &terms, const
   check_known(ctrl, "emulate_time_evolution");
   const cplx I(0.0, 1.0);
   double tr = 0.0, op_nrm = 0.0;
-  std::vector<dev::PauliTerm> pt;
+  std::vector<SumTerm> st;
   for (size_t t = 0; t < terms.size(); ++t) {
     if (terms[t].ops.empty()) {
       tr += coeffs[t];
       continue;
     }
-    dev::PauliTerm p;
+    SumTerm p;
     cplx w;
     pauli_encode(terms[t], ids, &p.x, &p.z, &w);
-    cplx c = coeffs[t] * w;
-    p.c_re = c.real();
-    p.c_im = c.imag();
-    pt.push_back(p);
+    p.c = coeffs[t] * w;
+    st.push_back(p);
     op_nrm += std::abs(coeffs[t]);
   }
   const unsigned steps = (unsigned)(std::abs(time) * op_nrm + 1.);
   const cplx correction = std::exp(-time * I * tr / (double)steps);
-  const uint64_t cmask = mask_of(ctrl), N = amps();
-  const dev::PauliTerm *d_terms =
-      pt.empty() ? nullptr : (const dev::PauliTerm *)upload(pt.data(), pt.size() * sizeof(dev::PauliTerm));
-  void *out = scratch(0);
-  scratch(1);  // buf_[1] ping-pongs with psi_ as the Taylor term; psi_, buf_[0], buf_[1] stay distinct
-  QS_HIP(hipMemcpyAsync(out, psi_, N * amp_bytes(), hipMemcpyDeviceToDevice, stream_));
-  for (unsigned s = 0; s < steps; ++s) {
-    double change = 1.0;
-    for (unsigned k = 0; change > 1.e-12; ++k) {
-      const cplx f = (-time * I) / double(steps * (k + 1));
-      dispatch([&](auto tag) {
-        using R = decltype(tag);
-        dev::pauli_sum<R>((const amp_t<R> *)psi_, (amp_t<R> *)buf_[1], (amp_t<R> *)out, N, d_terms,
-                          (int)pt.size(), f.real(), f.imag(), true, cmask, d_partials_, stream_);
-      });
-      change = std::sqrt(finish(dev::kReduceGrid, 1));
-      std::swap(psi_, buf_[1]);
-    }
-    dispatch([&](auto tag) {
-      using R = decltype(tag);
-      dev::scale_masked<R>((amp_t<R> *)out, N, cmask, correction.real(), correction.imag(), stream_);
-    });
-    QS_HIP(hipMemcpyAsync(psi_, out, N * amp_bytes(), hipMemcpyDeviceToDevice, stream_));
+  const uint64_t cmask = mask_of(ctrl);
+  SumPlan plan;
+  plan_sum(st, n_, c64_, plan);
+  SumUpload up(*this, plan);
+  scratch(0);
+  scratch(1);
+  dev::EvolveState *state = (dev::EvolveState *)d_flags_, *seen = (dev::EvolveState *)h_flags_;
+  // the series ends at the latest where the product of the factors' bounds does
+  const double theta = std::abs(time) * op_nrm / steps;
+  unsigned guess = 1;
+  for (double bound = theta; bound > 1.e-12 && guess < 64; bound *= theta / ++guess) {
   }
-  sync();
+  guess = std::max(1u, guess * 3 / 4);
+  for (unsigned s = 0; s < steps; ++s) {
+    dev::evolve_reset(state, stream_);
+    unsigned k = 0;
+    seen->done = 0;
+    for (unsigned last = guess; !seen->done; last = k + 3) {
+      for (; k < last; ++k) {
+        const cplx f = (-time * I) / double(steps * (k + 1));
+        const bool first = k == 0;
+        void *src = (k & 1) ? buf_[1] : psi_, *dst = (k & 1) ? psi_ : buf_[1];
+        dispatch([&](auto tag) {
+          using R = decltype(tag);
+          dev::pauli_sum<R>((const amp_t<R> *)src, (amp_t<R> *)dst, (amp_t<R> *)buf_[0], n_, plan, up.rec,
+                            first ? f * correction : f, first, correction, cmask, state, d_partials_, stream_);
+        });
+        dev::evolve_check(d_partials_, n_, plan, state, seen, stream_);
+      }
+      sync();
+    }
+    guess = (unsigned)seen->terms;
+    std::swap(psi_, buf_[0]);
+  }
   norm_changed();
   subspace_unknown();
 }

@@ -126,6 +126,7 @@ class Engine {
   void math_apply(dev::MathArgs args, const int32_t *d_table, bool known_bijective);
   double masked_norm(uint64_t mask, uint64_t val);
   int sides(unsigned id, double tol);
+  struct SumUpload;
   void flush_window();
   // complex64 norm guard: FP32-rounded gate matrices are unitary only to ~1e-8 (the FP32 H scales
   // the norm by 1 - 3.4e-8), so over thousands of gates the state's norm drifts from its exact

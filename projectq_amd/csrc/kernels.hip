@@ -319,49 +319,6 @@ __global__ __launch_bounds__(kBlock) void k_permute_tiles(const amp_t<R> *__rest
   }
 }
 
-// ------------------------------------------------------------------------------ Pauli strings
-template <typename R, bool EVOLVE>
-__global__ __launch_bounds__(kBlock) void k_pauli_sum(const amp_t<R> *__restrict__ src,
-                                                      amp_t<R> *__restrict__ dst,
-                                                      amp_t<R> *__restrict__ out, uint64_t n,
-                                                      const PauliTerm *__restrict__ terms,
-                                                      int n_terms, double f_re, double f_im,
-                                                      uint64_t cmask, double *partials) {
-  __shared__ double lds[kBlock / 64];
-  double nrm = 0.0;
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    double ur = 0.0, ui = 0.0;
-    for (int t = 0; t < n_terms; ++t) {
-      const PauliTerm pt = terms[t];
-      const uint64_t j = i ^ pt.x;
-      amp_t<R> b = src[j];
-      double br = re(b), bi = im(b);
-      if (__popcll(j & pt.z) & 1) {
-        br = -br;
-        bi = -bi;
-      }
-      ur += br * pt.c_re - bi * pt.c_im;
-      ui += br * pt.c_im + bi * pt.c_re;
-    }
-    if (EVOLVE) {
-      double vr = ur * f_re - ui * f_im, vi = ur * f_im + ui * f_re;
-      ur = vr;
-      ui = vi;
-    }
-    dst[i] = make_amp<R>(ur, ui);
-    if (EVOLVE && (i & cmask) == cmask) {
-      amp_t<R> o = out[i];
-      out[i] = make_amp<R>(re(o) + ur, im(o) + ui);
-      nrm += ur * ur + ui * ui;
-    }
-  }
-  if (EVOLVE) {
-    double t = block_sum(nrm, lds);
-    if (threadIdx.x == 0) partials[blockIdx.x] = t;
-  }
-}
-
 template <typename R>
 __global__ __launch_bounds__(kBlock) void k_scale_masked(amp_t<R> *__restrict__ psi, uint64_t n,
                                                          uint64_t cmask, double cr, double ci) {
@@ -706,19 +663,6 @@ void permute_tiles(const amp_t<R> *src, amp_t<R> *dst, uint64_t n_amps, const Pe
 }
 
 template <typename R>
-void pauli_sum(const amp_t<R> *src, amp_t<R> *dst, amp_t<R> *out, uint64_t n,
-               const PauliTerm *terms, int n_terms, double f_re, double f_im, bool evolve,
-               uint64_t cmask, double *partials, hipStream_t s) {
-  if (evolve)
-    hipLaunchKernelGGL((k_pauli_sum<R, true>), dim3(kReduceGrid), dim3(kBlock), 0, s, src, dst, out,
-                       n, terms, n_terms, f_re, f_im, cmask, partials);
-  else
-    hipLaunchKernelGGL((k_pauli_sum<R, false>), dim3(grid_for(n)), dim3(kBlock), 0, s, src, dst, out,
-                       n, terms, n_terms, f_re, f_im, cmask, partials);
-  QS_HIP(hipGetLastError());
-}
-
-template <typename R>
 void scale_masked(amp_t<R> *psi, uint64_t n, uint64_t cmask, double cr, double ci, hipStream_t s) {
   hipLaunchKernelGGL(k_scale_masked<R>, dim3(grid_for(n)), dim3(kBlock), 0, s, psi, n, cmask, cr, ci);
   QS_HIP(hipGetLastError());
@@ -815,9 +759,6 @@ template void convert_amps<float, double>(const amp_t<float> *, amp_t<double> *,
   template void drop_bit<R>(const amp_t<R> *, amp_t<R> *, uint64_t, int, int, hipStream_t);       \
   template void swap_bits<R>(amp_t<R> *, uint64_t, int, int, hipStream_t);                          \
   template void permute_tiles<R>(const amp_t<R> *, amp_t<R> *, uint64_t, const PermTile &, hipStream_t); \
-  template void pauli_sum<R>(const amp_t<R> *, amp_t<R> *, amp_t<R> *, uint64_t,                  \
-                             const PauliTerm *, int, double, double, bool, uint64_t, double *,    \
-                             hipStream_t);                                                        \
   template void scale_masked<R>(amp_t<R> *, uint64_t, uint64_t, double, double, hipStream_t);     \
   template void math_permute<R>(const amp_t<R> *, amp_t<R> *, uint64_t, const MathArgs &,         \
                                 const int32_t *, int *, hipStream_t);                             \

@@ -110,12 +110,6 @@ void swap_bits(amp_t<R> *psi, uint64_t n_amps, int a, int b, hipStream_t s);
 template <typename R>
 void permute_tiles(const amp_t<R> *src, amp_t<R> *dst, uint64_t n_amps, const PermTile &P, hipStream_t s);
 
-// dst_i <- f * sum_t c_t (-1)^popcount((i^x_t)&z_t) src_{i^x_t}; with `evolve` also
-// out_i += dst_i and nrm partial sums of |dst_i|^2 on entries with (i & cmask) == cmask
-template <typename R>
-void pauli_sum(const amp_t<R> *src, amp_t<R> *dst, amp_t<R> *out, uint64_t n_amps,
-               const PauliTerm *terms, int n_terms, double f_re, double f_im, bool evolve,
-               uint64_t cmask, double *partials, hipStream_t s);
 // psi_i *= c where (i & cmask) == cmask
 template <typename R>
 void scale_masked(amp_t<R> *psi, uint64_t n_amps, uint64_t cmask, double c_re, double c_im,

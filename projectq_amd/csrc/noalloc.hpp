@@ -9,7 +9,7 @@ namespace qs {
 // Pauli strings per call; the scratch array holds the records and partial sums of one plan (128
 // strings) and every plan's result.
 constexpr size_t kNoAllocMaxTerms = 4096;
-constexpr size_t kNoAllocScratchBytes = 49 << 10;
+constexpr size_t kNoAllocScratchBytes = 51 << 10;
 
 // sum_t coeffs[t] * Re<psi|P_t|psi> for the state of 2^n_qubits amplitudes at `state` (this GPU's
 // memory; complex64 if c64, else complex128).  String t owns ops [term_offsets[t],

@@ -46,12 +46,12 @@ extern "C" int energy_emu(const double *psi, unsigned n, int c64, const unsigned
         const EnergyGroup &gr = plan.groups[g];
         const uint32_t above = gr.mask >> kEnergyLaneBits;
         const uint32_t skip = above ? (1u << (31 - __builtin_clz(above))) << kEnergyLaneBits : 0;
-        for (uint32_t s = 0; s < gr.n_re + gr.n_im; ++s) {
-          const EnergyString &st = plan.strings[gr.first + s];
+        for (uint32_t s = 0; s <= gr.more; ++s) {
+          const EnergyString &st = s ? plan.strings[gr.next + s - 1] : gr.head;
           for (uint32_t l = 0; l < size; ++l) {
             if (l & skip) continue;
             const uint32_t m = l ^ gr.mask;
-            const double v = s < gr.n_re ? re[l] * re[m] + im[l] * im[m] : re[l] * im[m] - im[l] * re[m];
+            const double v = gr.kind == 0 ? re[l] * re[m] + im[l] * im[m] : re[l] * im[m] - im[l] * re[m];
             total += (odd(base & st.z) ^ odd(l & st.zloc)) ? -st.w * v : st.w * v;
           }
         }
@@ -62,4 +62,58 @@ extern "C" int energy_emu(const double *psi, unsigned n, int c64, const unsigned
   }
   *out = total;
   return (int)plan.n_passes;
+}
+
+// sum_t c_t (-1)^{popcount(j & z_t)} psi_j, j = i ^ x_t, for every i, through the Pauli-sum plan
+// (projectq_amd/csrc/pauli_sum.hip).  Returns the number of groups read from memory, negative as above.
+extern "C" int sum_emu(const double *psi, unsigned n, int c64, const unsigned long long *x, const unsigned long long *z,
+                       const double *c, int count, double *out) {
+  std::vector<SumTerm> terms(count);
+  for (int t = 0; t < count; ++t) terms[t] = SumTerm{x[t], z[t], {c[2 * t], c[2 * t + 1]}};
+  SumPlan plan;
+  plan_sum(terms, n, c64 != 0, plan);
+  if (plan.t != plan.L + plan.h || plan.h > kEnergyMaxGens) return -2;
+  const uint64_t tiles = n > plan.t ? uint64_t(1) << (n - plan.t) : 1, N = uint64_t(1) << n;
+  const uint32_t size = 1u << plan.t;
+  std::vector<int> seen(N, 0);
+  auto index = [&](uint64_t base, uint32_t l) {
+    uint64_t i = base ^ (l & ((1u << plan.L) - 1));
+    for (uint32_t b = 0; b < plan.h; ++b)
+      if ((l >> (plan.L + b)) & 1) i ^= plan.gen[b];
+    return i;
+  };
+  int outside = 0;
+  plan.groups.pop_back();  // the spare
+  for (const SumGroup &g : plan.groups) outside += !g.inside;
+  for (uint64_t k = 0; k < tiles; ++k) {
+    uint64_t base = k << plan.L;
+    for (uint32_t b = 0; b < plan.h; ++b) {
+      const uint32_t q = plan.pivot[b];
+      base = ((base >> q) << (q + 1)) | (base & ((uint64_t(1) << q) - 1));
+    }
+    for (uint32_t l = 0; l < size; ++l) {
+      const uint64_t i = index(base, l);
+      if (i >= N) {
+        if (n >= 8) return -1;
+        continue;
+      }
+      ++seen[i];
+      std::complex<double> u = 0.0;
+      for (const SumGroup &g : plan.groups) {
+        const uint64_t j = g.inside ? index(base, l ^ g.mask) : i ^ g.x;
+        if (j != (i ^ g.x)) return -3;
+        const std::complex<double> b(psi[2 * j], psi[2 * j + 1]);
+        for (uint32_t s = 0; s <= g.more; ++s) {
+          const EnergyString &st = s ? plan.strings[g.next + s - 1] : g.head;
+          const double w = (odd(base & st.z) ^ odd(l & st.zloc)) ? -st.w : st.w;
+          u += g.kind == 0 ? w * b : std::complex<double>(0.0, w) * b;
+        }
+      }
+      out[2 * i] = u.real();
+      out[2 * i + 1] = u.imag();
+    }
+  }
+  for (int v : seen)
+    if (v != 1) return -1;
+  return outside;
 }
