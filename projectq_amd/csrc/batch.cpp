@@ -6,6 +6,7 @@
 #include <complex>
 #include <cstring>
 #include <limits>
+#include <memory>
 
 namespace qs {
 
@@ -106,13 +107,16 @@ void Batch::release() {
   launch_jobs_.clear();
   launch_blocks_.clear();
   launch_tmax_.clear();
-  void *bufs[] = {psi_, d_state_off_, d_stages_, d_rops_, d_tops_, d_mats_, d_ejobs_, d_eblock_, d_terms_, d_partials_, d_energies_};
+  void *bufs[] = {psi_, d_state_off_, d_stages_, d_rops_, d_tops_, d_mats_, d_epass_, d_eblock_, d_egroup_, d_estring_, d_eslot_, d_partials_, d_energies_};
   for (void *b : bufs) (void)hipFree(b);
   psi_ = d_state_off_ = nullptr;
   d_stages_ = d_rops_ = d_tops_ = d_mats_ = nullptr;
-  d_ejobs_ = nullptr;
+  d_epass_ = nullptr;
   d_eblock_ = nullptr;
-  d_terms_ = nullptr;
+  d_egroup_ = nullptr;
+  d_estring_ = nullptr;
+  d_eslot_ = nullptr;
+  energy_launches_.clear();
   d_partials_ = d_energies_ = nullptr;
 }
 
@@ -193,57 +197,89 @@ void Batch::build(const BatchShape &shape) {
     launch_blocks_.push_back(blocks);
     launch_tmax_.push_back(tmax);
   }
-  // ---- energies: one job per circuit, chunks of up to 4096 amplitudes per workgroup
-  std::vector<dev::EnergyJob> ejobs(circ_.size());
-  std::vector<dev::BatchTerm> terms;
-  uint32_t slots = 0;
+  // ---- energies: every circuit's strings in plans of up to 128, every pass of a plan over its tiles
+  std::vector<dev::BatchEnergyPass> epass;
+  std::vector<EnergyGroup> egroup;
+  std::vector<EnergyString> estring;
+  std::vector<uint32_t> eslot;
+  constexpr int kXcds = 8;
+  constexpr uint64_t kBatchWorkgroups = 8;  // per circuit at least: 100 strings in one workgroup take 40 us
+  constexpr uint32_t kSmallest = 8, kSizes = 5;  // tiles of 2^8 .. 2^12 amplitudes
+  // Workgroup w runs on XCD w mod 8.  Every circuit goes whole to one XCD (largest first, to the
+  // least loaded), so the later passes over its state hit that XCD's L2; the XCDs' workgroup lists are
+  // interleaved and padded with idle workgroups to equal length.
+  std::vector<std::vector<dev::BatchEnergyBlock>> per_xcd[kSizes];
+  for (auto &v : per_xcd) v.resize(kXcds);
+  std::vector<size_t> order(circ_.size());
+  std::vector<int> xcd_of(circ_.size());
+  for (size_t c = 0; c < order.size(); ++c) order[c] = c;
+  std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return circ_[a].n > circ_[b].n; });
+  std::vector<uint64_t> load(kXcds, 0);
+  for (size_t c : order) {
+    const int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+    load[x] += (uint64_t(1) << circ_[c].n) * std::max<size_t>(circ_[c].terms.size(), 1);
+    xcd_of[c] = x;
+  }
+  auto plan = std::make_unique<EnergyPlan>();
+  std::vector<EnergyTerm> terms;
+  std::vector<std::vector<dev::BatchEnergyBlock>> of_circuit(circ_.size());
+  std::vector<uint32_t> tile_bits(circ_.size(), kSmallest);
   for (size_t c = 0; c < circ_.size(); ++c) {
-    dev::EnergyJob &e = ejobs[c];
-    e.state_off = state_off[c];
-    e.n_amps = uint64_t(1) << circ_[c].n;
-    e.chunk = std::min<uint64_t>(e.n_amps, 4096);
-    e.first_block = slots;
-    e.n_blocks = (uint32_t)((e.n_amps + e.chunk - 1) / e.chunk);
-    slots += e.n_blocks;
-    e.term_off = (uint32_t)terms.size();
-    e.n_terms = (uint32_t)circ_[c].terms.size();
+    eslot.push_back(eslot.empty() ? 0u : eslot.back());
+    terms.clear();
     for (const dev::PauliTerm &t0 : circ_[c].terms) {
-      // the strings act on the circuit's final layout (relabelling moves qubits)
-      dev::PauliTerm t = t0;
-      t.x = t.z = 0;
+      // the strings act on the circuit's final layout (relabelling moves qubits); Hermitian, so the
+      // coefficient with its phase is real, or imaginary for an odd number of Y
+      EnergyTerm t{0, 0, 1.0, t0.c_re};
       for (uint32_t q = 0; q < circ_[c].n; ++q) {
         t.x |= ((t0.x >> q) & 1u) << final_pos[c][q];
         t.z |= ((t0.z >> q) & 1u) << final_pos[c][q];
       }
-      // (-1)^{popcount((i ^ x) & z)} = (-1)^{popcount(i & z)} (-1)^{popcount(x & z)}
-      double s = (__builtin_popcountll(t.x & t.z) & 1) ? -1.0 : 1.0;
-      // pairs (i, i ^ x): half the amplitudes, twice the weight
-      const uint32_t h = t.x ? 1u << (63 - __builtin_clzll(t.x)) : 0u;
-      if (t.x) s *= 2.0;
-      terms.push_back(dev::BatchTerm{(uint32_t)t.x, (uint32_t)t.z, h, 0u, s * t.c_re, s * t.c_im});
+      if (__builtin_popcountll(t.x & t.z) & 1) {
+        t.omega = std::complex<double>(0.0, 1.0);
+        t.c = t0.c_im;
+      }
+      terms.push_back(t);
     }
+    uint32_t slot = eslot.back();
+    for (size_t t0 = 0; t0 < terms.size(); t0 += kEnergyMaxStrings) {
+      const int m = (int)std::min<size_t>(kEnergyMaxStrings, terms.size() - t0);
+      plan_energy(terms.data() + t0, m, circ_[c].n, c64_, kBatchWorkgroups, *plan);
+      tile_bits[c] = plan->t;
+      const uint32_t tiles = circ_[c].n > plan->t ? 1u << (circ_[c].n - plan->t) : 1u;
+      for (uint32_t p = 0; p < plan->n_passes; ++p) {
+        dev::BatchEnergyPass bp{state_off[c], uint64_t(1) << circ_[c].n, plan->L, plan->h, plan->passes[p]};
+        bp.pass.first_group += (uint32_t)egroup.size();
+        const uint32_t each = std::max(1u, tiles / 1024);
+        for (uint32_t k = 0; k < tiles; k += each)
+          of_circuit[c].push_back(dev::BatchEnergyBlock{(uint32_t)epass.size(), k, std::min(each, tiles - k), slot++});
+        epass.push_back(bp);
+      }
+      for (uint32_t g = 0; g < plan->n_groups; ++g) {
+        EnergyGroup eg = plan->groups[g];
+        eg.next += (uint32_t)estring.size();
+        egroup.push_back(eg);
+      }
+      estring.insert(estring.end(), plan->strings, plan->strings + plan->n_strings);
+    }
+    eslot.back() = slot;
   }
-  // Workgroup w runs on XCD w mod 8.  Every circuit goes whole to one XCD (largest first, to the
-  // least loaded), so its partner reads stay in that XCD's L2; the XCDs' workgroup lists are
-  // interleaved and padded with idle workgroups to equal length.
-  constexpr int kXcds = 8;
-  std::vector<size_t> order(circ_.size());
-  for (size_t c = 0; c < order.size(); ++c) order[c] = c;
-  std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return circ_[a].n > circ_[b].n; });
-  std::vector<std::vector<dev::EnergyBlock>> per_xcd(kXcds);
-  std::vector<uint64_t> load(kXcds, 0);
+  eslot.insert(eslot.begin(), 0u);
+  egroup.push_back(EnergyGroup{});  // kernels load one group ahead
   for (size_t c : order) {
-    const int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-    load[x] += ejobs[c].n_amps * std::max<uint32_t>(ejobs[c].n_terms, 1);
-    for (uint32_t b = 0; b < ejobs[c].n_blocks; ++b) per_xcd[x].push_back(dev::EnergyBlock{(uint32_t)c, b});
+    auto &list = per_xcd[tile_bits[c] - kSmallest][xcd_of[c]];
+    list.insert(list.end(), of_circuit[c].begin(), of_circuit[c].end());
   }
-  size_t longest = 0;
-  for (auto &v : per_xcd) longest = std::max(longest, v.size());
-  std::vector<dev::EnergyBlock> eblock;
-  for (size_t k = 0; k < longest; ++k)
-    for (int x = 0; x < kXcds; ++x)
-      eblock.push_back(k < per_xcd[x].size() ? per_xcd[x][k] : dev::EnergyBlock{dev::kNoJob, 0});
-  e_blocks_ = (uint32_t)eblock.size();
+  std::vector<dev::BatchEnergyBlock> eblock;
+  for (uint32_t s = kSizes; s-- > 0;) {  // the largest first
+    size_t longest = 0;
+    for (auto &v : per_xcd[s]) longest = std::max(longest, v.size());
+    if (longest == 0) continue;
+    energy_launches_.push_back({kSmallest + s, (uint32_t)eblock.size(), (uint32_t)(longest * kXcds)});
+    for (size_t k = 0; k < longest; ++k)
+      for (int x = 0; x < kXcds; ++x)
+        eblock.push_back(k < per_xcd[s][x].size() ? per_xcd[s][x][k] : dev::BatchEnergyBlock{dev::kNoPass, 0, 0, 0});
+  }
   // ---- device buffers
   const size_t ab = c64_ ? 8 : 16;
   QS_HIP(hipMalloc(&psi_, total_amps_ * ab));
@@ -265,10 +301,12 @@ void Batch::build(const BatchShape &shape) {
     for (size_t i = 0; i < m.size(); ++i) m[i] = make_double2(mats[i].real(), mats[i].imag());
     d_mats_ = to_device(m);
   }
-  d_ejobs_ = to_device(ejobs);
+  d_epass_ = to_device(epass);
   d_eblock_ = to_device(eblock);
-  d_terms_ = to_device(terms);
-  QS_HIP(hipMalloc(&d_partials_, std::max<size_t>(slots, 1) * sizeof(double)));
+  d_egroup_ = to_device(egroup);
+  d_estring_ = to_device(estring);
+  d_eslot_ = to_device(eslot);
+  QS_HIP(hipMalloc(&d_partials_, std::max<size_t>(eslot.back(), 1) * sizeof(double)));
   QS_HIP(hipMalloc(&d_energies_, circ_.size() * sizeof(double)));
   // ---- capture one run into a graph
   QS_HIP(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
@@ -293,11 +331,13 @@ void Batch::enqueue() {
       dev::batch_tile_pass<R>(psi, d_jobs_[l], d_block_job_[l], launch_blocks_[l], launch_tmax_[l], (int)shape_.rb,
                               (const dev::TileStage *)d_stages_, (const dev::RegOp *)d_rops_,
                               (const dev::TileOp *)d_tops_, (const amp_t<R> *)d_mats_, two_qubit_ops_, stream_);
-    dev::batch_energy<R>(psi, d_ejobs_, d_eblock_, e_blocks_, d_terms_, d_partials_, stream_);
+    for (const EnergyLaunch &l : energy_launches_)
+      dev::batch_energy<R>(psi, l.t, d_epass_, d_eblock_ + l.first_block, l.n_blocks, d_egroup_, d_estring_, d_partials_,
+                           stream_);
   };
   if (c64_) go(float{});
   else go(double{});
-  dev::batch_energy_finish(d_ejobs_, (int)circ_.size(), d_partials_, d_energies_, stream_);
+  dev::batch_energy_finish(d_eslot_, (int)circ_.size(), d_partials_, d_energies_, stream_);
 }
 
 double Batch::run(bool graph, double *energies) {

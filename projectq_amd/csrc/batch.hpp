@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "energy.hpp"
 #include "kernels.hpp"
 #include "planner.hpp"
 
@@ -62,10 +63,15 @@ class Batch {
   std::vector<uint32_t *> d_block_job_;
   std::vector<std::vector<dev::BatchJob>> launch_jobs_;
   std::vector<uint32_t> launch_blocks_, launch_tmax_;
-  dev::EnergyJob *d_ejobs_ = nullptr;
-  dev::EnergyBlock *d_eblock_ = nullptr;
-  uint32_t e_blocks_ = 0;
-  dev::BatchTerm *d_terms_ = nullptr;
+  dev::BatchEnergyPass *d_epass_ = nullptr;
+  dev::BatchEnergyBlock *d_eblock_ = nullptr;
+  struct EnergyLaunch {
+    uint32_t t, first_block, n_blocks;
+  };
+  std::vector<EnergyLaunch> energy_launches_;  // one per tile size
+  EnergyGroup *d_egroup_ = nullptr;
+  EnergyString *d_estring_ = nullptr;
+  uint32_t *d_eslot_ = nullptr;  // first partial sum of every circuit, and the end
   double *d_partials_ = nullptr, *d_energies_ = nullptr, *h_energies_ = nullptr;
   hipGraph_t graph_ = nullptr;
   hipGraphExec_t exec_ = nullptr;

@@ -76,7 +76,7 @@ void complete(Span &span, uint64_t *gen, uint32_t L, uint32_t h, uint8_t *pivot)
 
 }  // namespace
 
-void plan_energy(const EnergyTerm *terms, int count, unsigned n, bool c64, EnergyPlan &plan) {
+void plan_energy(const EnergyTerm *terms, int count, unsigned n, bool c64, uint64_t workgroups, EnergyPlan &plan) {
   tile_of(n, c64, c64 ? 12u : 11u, &plan.t, &plan.L, &plan.h);
   // 32 KiB of LDS, 256 threads with 16 (complex64) or 8 (complex128) amplitudes each
   plan.n_passes = plan.n_groups = plan.n_strings = 0;
@@ -110,10 +110,9 @@ void plan_energy(const EnergyTerm *terms, int count, unsigned n, bool c64, Energ
     g[n_groups++] = Group{i, re, e - i - re, terms[order[i]].x & ~low};
     i = e;
   }
-  // At least about 1024 workgroups where the state has few tiles: the strings are spread over more
-  // passes (the state is in the caches then).
+  // fewer strings to a pass where the state has few tiles (it is in the caches then)
   const uint64_t tiles = n > plan.t ? uint64_t(1) << (n - plan.t) : 1;
-  const uint64_t want = (1024 + tiles - 1) / tiles;  // passes that fill the chip
+  const uint64_t want = std::max<uint64_t>(1, (workgroups + tiles - 1) / tiles);
   const int most = std::max<int>(1, (int)((uint64_t)(m + (int)want - 1) / want));
 
   const uint32_t lanes_h = kEnergyLaneBits > (int)plan.L ? std::min(kEnergyLaneBits - plan.L, plan.h) : 0;  // generators on thread bits

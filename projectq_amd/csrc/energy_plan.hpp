@@ -68,8 +68,10 @@ struct EnergyTerm {
 };
 
 // Plans `count` <= kEnergyMaxStrings terms on a state of n qubits.  Terms that are not Hermitian
-// are left out: the real part of their expectation value is zero.
-void plan_energy(const EnergyTerm *terms, int count, unsigned n, bool c64, EnergyPlan &plan);
+// are left out: the real part of their expectation value is zero.  workgroups: where the state has few
+// tiles, the strings are spread over more passes until about that many workgroups have work.
+void plan_energy(const EnergyTerm *terms, int count, unsigned n, bool c64, uint64_t workgroups, EnergyPlan &plan);
+constexpr uint64_t kEnergyWorkgroups = 1024;  // fills the chip: for a plan that runs alone
 
 // ---- sum_t c_t P_t applied to a state (qubit operators and the terms of a time evolution) ----------
 

@@ -1184,7 +1184,7 @@ double Engine::get_expectation_value(const std::vector<PauliString> &terms,
   char records[kEnergyRecordBytes];
   for (size_t t0 = 0; t0 < et.size(); t0 += kEnergyMaxStrings) {
     const int m = (int)std::min<size_t>(kEnergyMaxStrings, et.size() - t0);
-    plan_energy(et.data() + t0, m, n_, c64_, plan);
+    plan_energy(et.data() + t0, m, n_, c64_, kEnergyWorkgroups, plan);
     const EnergyRecords rec = pack_energy(plan, records);
     const char *d = rec.bytes ? (const char *)upload(records, rec.bytes) : nullptr;
     if (results == kResults) collect();

@@ -58,13 +58,6 @@ template <typename R>
 void batch_tile_pass(amp_t<R> *psi, const BatchJob *jobs, const uint32_t *block_job, uint32_t n_blocks,
                      uint32_t max_t, int rb, const TileStage *stages, const RegOp *rops, const TileOp *tops,
                      const amp_t<R> *mats, bool two_qubit_ops, hipStream_t s);
-// partials[b] for every energy workgroup, then energies[j] = sum of job j's partials in order
-template <typename R>
-void batch_energy(const amp_t<R> *psi, const EnergyJob *jobs, const EnergyBlock *blocks, uint32_t n_blocks,
-                  const BatchTerm *terms, double *partials, hipStream_t s);
-void batch_energy_finish(const EnergyJob *jobs, int n_jobs, const double *partials, double *energies,
-                         hipStream_t s);
-
 // dense gate block: psi[base + off(r)] = sum_c M[r][c] psi[base + off(c)] for every base with
 // target bits 0 and control bits 1.  tpos[l] is the position of matrix bit l; ins lists the
 // sorted target+control positions; n_groups = 2^(n - k - #controls).  The host matrix `mat` is read

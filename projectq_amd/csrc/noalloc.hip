@@ -103,7 +103,7 @@ double expectation_noalloc(const void *state, unsigned n_qubits, bool c64, const
       encode(t0 + i, term_idx, term_ops, term_offsets, positions, n_positions, &terms[i]);
       terms[i].c = coeffs[t0 + i];
     }
-    plan_energy(terms, (int)m, n_qubits, c64, plan);
+    plan_energy(terms, (int)m, n_qubits, c64, kEnergyWorkgroups, plan);
     const EnergyRecords rec = pack_energy(plan, records);
     // in stream order: the previous plan's kernels have read their records
     if (rec.bytes) QS_HIP(hipMemcpy(base + kRecordsOff, records, rec.bytes, hipMemcpyHostToDevice));

@@ -15,7 +15,7 @@ extern "C" int energy_emu(const double *psi, unsigned n, int c64, const unsigned
   std::vector<EnergyTerm> terms(count);
   for (int t = 0; t < count; ++t) terms[t] = EnergyTerm{x[t], z[t], {omega[2 * t], omega[2 * t + 1]}, c[t]};
   static EnergyPlan plan;
-  plan_energy(terms.data(), count, n, c64 != 0, plan);
+  plan_energy(terms.data(), count, n, c64 != 0, kEnergyWorkgroups, plan);
   if (plan.t != plan.L + plan.h || plan.h > kEnergyMaxGens || plan.n_passes > (uint32_t)kEnergyMaxStrings) return -2;
   const uint64_t tiles = n > plan.t ? uint64_t(1) << (n - plan.t) : 1, N = uint64_t(1) << n;
   const uint32_t size = 1u << plan.t;
