@@ -90,7 +90,10 @@ class Engine {
 
   // measurement hooks (C-ABI extensions)
   void synchronize();
-  void set_profiling(bool on) { profiling_ = on; }
+  void set_profiling(bool on) {
+    exec_blocks();
+    profiling_ = on;
+  }
   void get_stats(uint64_t *passes, double *bytes, double *gpu_ms, uint64_t *timed);
   void reset_stats();
   cplx overlap(Engine &other);
@@ -165,7 +168,7 @@ class Engine {
   unsigned tile_tmax_ = 13, tile_rb_ = 5;  // tile shape limits (PROJECTQ_AMD_TILE="t:rb" overrides)
   unsigned tile_bits(unsigned tmax) const;
   std::vector<Block> greedy_blocks(const std::vector<Gate> &gates) const;
-  std::vector<PGate> resolve(const std::vector<Gate> &gates) const;
+  std::vector<PGate> resolve(const std::vector<Gate> &gates, bool cnot_cz) const;
   std::vector<TileProgram> plan_tiles(const std::vector<PGate> &pg, unsigned tmax, unsigned rb, unsigned lmin,
                                       int rule, bool relabel, unsigned *t_used) const;
   int slot_rule_ = kSlotLookahead;  // rule of QS_PLANNER_TILE
@@ -184,6 +187,7 @@ class Engine {
     bool two_qubit_ops;
   };
   size_t upload_programs(const std::vector<TileProgram> &progs, size_t first, std::vector<DeviceProgram> *out);
+  void exec_programs(const std::vector<TileProgram> &progs, unsigned rb);
   void exec_tile_program(const TileProgram &prog, const DeviceProgram &d, unsigned rb);
   PassFeatures block_features(const Block &b) const;
   void begin_pass(hipEvent_t *e0, hipEvent_t *e1);
@@ -220,8 +224,14 @@ class Engine {
   // state in HBM); every call that hands the layout out restores it first (canonicalize).
   std::map<unsigned, unsigned> ref_pos_;
   void canonicalize();
-  GateQueue queue_;
-  std::vector<Gate> window_;
+  std::vector<Gate> window_;  // queued gates, both fusion modes
+  // block fusion: window_ is cut into the reference's blocks as gates arrive (ends_: the end of each
+  // block that is complete, open_: the qubits of the one that is not)
+  std::vector<size_t> ends_;
+  BlockQubits open_;
+  static constexpr size_t kMaxPending = 4096;  // gates of complete blocks that may wait
+  void close_block();
+  void exec_blocks();
   std::mt19937 rng_;
   std::uniform_real_distribution<double> uni_{0.0, 1.0};
   hipStream_t stream_ = nullptr;

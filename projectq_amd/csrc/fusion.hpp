@@ -22,6 +22,38 @@ struct Gate {
   std::vector<unsigned> ctrl;   // qubit ids that must be 1
 };
 
+// The qubits of a GateQueue without its matrices: enough to decide where a block ends.
+class BlockQubits {
+ public:
+  unsigned num_qubits() const { return (unsigned)qubits_.size(); }
+  void clear() {
+    qubits_.clear();
+    gctrl_.clear();
+    empty_ = true;
+  }
+  void insert(const Gate &g) {  // as GateQueue::insert
+    std::vector<unsigned> stale = gctrl_;
+    for (unsigned q : g.ids) add(&qubits_, q);
+    for (unsigned c : g.ctrl) {
+      if (has(gctrl_, c)) stale.erase(std::remove(stale.begin(), stale.end(), c), stale.end());
+      else add(empty_ ? &gctrl_ : &qubits_, c);
+    }
+    for (unsigned c : stale) {
+      gctrl_.erase(std::remove(gctrl_.begin(), gctrl_.end(), c), gctrl_.end());
+      add(&qubits_, c);
+    }
+    empty_ = false;
+  }
+
+ private:
+  static bool has(const std::vector<unsigned> &v, unsigned q) { return std::find(v.begin(), v.end(), q) != v.end(); }
+  static void add(std::vector<unsigned> *v, unsigned q) {
+    if (!has(*v, q)) v->push_back(q);
+  }
+  std::vector<unsigned> qubits_, gctrl_;
+  bool empty_ = true;
+};
+
 // A fused block ready for the device: matrix bit l <-> qubit id qubits[l] (ascending ids).
 struct Block {
   std::vector<cplx> m;
