@@ -47,6 +47,8 @@ SOURCES = [
     "tile_c64_rb5.hip",
     "tile_c128_rb5.hip",
     "tile_pf.hip",
+    "tile_c64_phase.hip",
+    "tile_c128_phase.hip",
     "tile_c64_rb4.hip",
     "tile_c128_rb4.hip",
     "kernels.hip",

@@ -533,7 +533,7 @@ std::vector<Block> Engine::greedy_blocks(const std::vector<Gate> &gates) const {
   return out;
 }
 
-std::vector<PGate> Engine::resolve(const std::vector<Gate> &gates, bool cnot_cz) const {
+Engine::Resolved Engine::resolve(const std::vector<Gate> &gates, bool cnot_cz) const {
   std::vector<PGate> pg;
   pg.reserve(gates.size());
   for (const Gate &g : gates) {
@@ -548,7 +548,15 @@ std::vector<PGate> Engine::resolve(const std::vector<Gate> &gates, bool cnot_cz)
   // makes the CZ cheap: in windows without 2-qubit gates (the only source of 2-qubit register ops)
   bool two_qubit_gates = false;
   for (const PGate &p : pg) two_qubit_gates = two_qubit_gates || p.tpos.size() == 2;
-  return merge_single_qubit_runs(cnot_cz && !two_qubit_gates ? cnot_to_cz(pg) : pg);
+  Resolved out;
+  out.gates = merge_single_qubit_runs(cnot_cz && !two_qubit_gates ? cnot_to_cz(pg) : pg);
+  if (!two_qubit_gates) {  // the kernels with phase ops hold no 2-qubit ones
+    out.phases = diagonals_to_phases(out.gates);
+    size_t n = 0;
+    for (const PGate &p : out.phases) n += p.tpos.empty();
+    if (n * kPhaseShare < out.phases.size()) out.phases.clear();
+  }
+  return out;
 }
 
 // Tile size: 2^t amplitudes of LDS per workgroup, at most n bits, and small enough that a state
@@ -558,10 +566,13 @@ unsigned Engine::tile_bits(unsigned tmax) const {
   return std::min(tmax, std::max(10u, n_ - 8));
 }
 
-std::vector<TileProgram> Engine::plan_tiles(const std::vector<PGate> &pg, unsigned tmax, unsigned rb,
+std::vector<TileProgram> Engine::plan_tiles(const Resolved &resolved, unsigned tmax, unsigned rb,
                                             unsigned lmin, int rule, bool relabel, unsigned *t_used) const {
   const unsigned t = tile_bits(tmax);
   *t_used = t;
+  // phase ops: full tiles only (2^11 complex128 or 2^12 complex64 amplitudes and more)
+  const bool phases = !resolved.phases.empty() && rb == 4 && t >= (c64_ ? 12u : 11u);
+  const std::vector<PGate> &pg = phases ? resolved.phases : resolved.gates;
   std::vector<PPass> passes = schedule_tiles(pg, TileShape{n_, t, lmin}, slot_chooser(rule), 256, 16.0, relabel);
   std::vector<TileProgram> progs(passes.size());
   for (size_t i = 0; i < passes.size(); ++i) build_tile_pass(pg, passes[i], t, rb, c64_, progs[i]);
@@ -709,7 +720,7 @@ void Engine::plan_window(const std::vector<Gate> &gates, std::vector<Block> *blo
     info->passes = (unsigned)blocks_out->size();
     return;
   }
-  const std::vector<PGate> pg = resolve(gates, cnot_cz_);
+  const Resolved pg = resolve(gates, cnot_cz_);
   if (planner_kind_ == 2) {
     unsigned t;
     *progs_out = plan_tiles(pg, tile_tmax_, tile_rb_, tile_lmin_, slot_rule_, relabel_mode_ == 1, &t);
@@ -840,10 +851,11 @@ size_t Engine::upload_programs(const std::vector<TileProgram> &progs, size_t fir
     d.stages = (const dev::TileStage *)put(p.stages);
     d.rops = (const dev::RegOp *)put(p.rops);
     d.tops = (const dev::TileOp *)put(p.tops);
-    d.two_qubit_ops = false;
+    d.forms = dev::kFormsOneQubit;
     for (const dev::RegOp &op : p.rops) {
       const uint32_t kind = (op.code >> 8) & 15u;
-      d.two_qubit_ops = d.two_qubit_ops || kind == dev::kOp2General || kind == dev::kOp2Diag;
+      if (kind == dev::kOp2General || kind == dev::kOp2Diag) d.forms = dev::kFormsAll;
+      if (kind >= dev::kOpPhases) d.forms = dev::kFormsPhases;
     }
     dispatch([&](auto tag) {
       using R = decltype(tag);
@@ -871,7 +883,7 @@ void Engine::exec_tile_program(const TileProgram &prog, const DeviceProgram &d, 
     hipEvent_t e0, e1;
     begin_pass(&e0, &e1);
     dev::tile_pass<R>((amp_t<R> *)psi_, n_tiles, prog.P, (int)rb, d.stages, d.rops, d.tops, (const amp_t<R> *)d.mats,
-                      d.two_qubit_ops, stream_);
+                      d.forms, stream_);
     end_pass(e0, e1, recording_ ? &f : nullptr);
   });
   count_pass(2.0 * (double)amp_bytes() * (double)amps());

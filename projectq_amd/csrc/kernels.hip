@@ -568,11 +568,11 @@ void apply_block(amp_t<R> *psi, uint64_t n_groups, const BitInsert &ins, uint64_
 
 template <typename R>
 void tile_pass(amp_t<R> *psi, uint64_t n_tiles, const TilePass &P, int rb, const TileStage *d_stages,
-               const RegOp *d_rops, const TileOp *d_tops, const amp_t<R> *d_mats, bool two_qubit_ops, hipStream_t s) {
+               const RegOp *d_rops, const TileOp *d_tops, const amp_t<R> *d_mats, TileForms forms, hipStream_t s) {
   if (P.h > (uint32_t)kTileMaxHigh || P.L < 1 || P.t > (uint32_t)kTileMaxBits)
     throw ValueError("tile pass: bad tile shape");
-  if (rb == 5) launch_tile_pass<R, 5>(psi, n_tiles, P, d_stages, d_rops, d_tops, d_mats, two_qubit_ops, s);
-  else if (rb == 4) launch_tile_pass<R, 4>(psi, n_tiles, P, d_stages, d_rops, d_tops, d_mats, two_qubit_ops, s);
+  if (rb == 5) launch_tile_pass<R, 5>(psi, n_tiles, P, d_stages, d_rops, d_tops, d_mats, forms, s);
+  else if (rb == 4) launch_tile_pass<R, 4>(psi, n_tiles, P, d_stages, d_rops, d_tops, d_mats, forms, s);
   else throw ValueError("tile pass: register bits must be 4 or 5");
 }
 
@@ -584,6 +584,8 @@ void prepare_tile_kernels() {
   prepare_tile_kernels_of<double, 4>();
   prepare_tile_kernels_of<double, 5>();
   prepare_tile_kernels_pf();
+  prepare_tile_kernels_phase_c64();
+  prepare_tile_kernels_phase_c128();
   done = true;
 }
 
@@ -747,7 +749,7 @@ template void convert_amps<float, double>(const amp_t<float> *, amp_t<double> *,
                                    uint32_t, int, const TileStage *, const RegOp *, const TileOp *,\
                                    const amp_t<R> *, bool, hipStream_t);                                \
   template void tile_pass<R>(amp_t<R> *, uint64_t, const TilePass &, int, const TileStage *,      \
-                             const RegOp *, const TileOp *, const amp_t<R> *, bool, hipStream_t); \
+                             const RegOp *, const TileOp *, const amp_t<R> *, TileForms, hipStream_t); \
   template void apply_block<R>(amp_t<R> *, uint64_t, const BitInsert &, uint64_t,                 \
                                const uint32_t *, int, const std::complex<double> *, const amp_t<R> *, hipStream_t); \
   template void norm_masked<R>(const amp_t<R> *, uint64_t, const BitInsert &, uint64_t, double *, \

@@ -67,6 +67,9 @@ struct TileStage {
 //   kind 2: 1-qubit anti-diagonal on b0    kind 5: 2-qubit diagonal on (b0, b1)
 //   kind 6: 1-qubit real 2x2 on b0         kind 7: 1-qubit Z (diag(1, -1): sign flip) on b0
 // Matrix bit 0 belongs to b0 and bit 1 to b1.
+//   kind 8: a group of phases, code = kind << 8 | mask of register bits; `rcmask` records of kind 9 follow it,
+//   their factors are the matrix elements from `mat` on.  Where the controls of such a record hold, its
+//   factor counts; the amplitudes with all bits of the mask set are multiplied by the product.
 enum : uint32_t {
   kOp1General = 0,
   kOp1Diag = 1,
@@ -75,11 +78,15 @@ enum : uint32_t {
   kOp2General = 4,
   kOp2Diag = 5,
   kOp1Real = 6,
-  kOp1Z = 7
+  kOp1Z = 7,
+  kOpPhases = 8,
+  kOpPhaseTerm = 9
 };
+// the op forms that occur in a pass: each has kernels that hold only those
+enum TileForms : uint32_t { kFormsAll = 0, kFormsOneQubit = 1, kFormsPhases = 2 };
 struct RegOp {
   uint32_t code;
-  uint32_t rcmask;  // controls among the stage's register bits (register-index mask, <= 1 bit)
+  uint32_t rcmask;  // controls among the stage's register bits (register-index mask, <= 1 bit); kind 8: records
   uint32_t lcmask;  // tile-local controls outside the stage's register bits
   uint32_t mat;     // first element of the op's matrix in the pass's matrix array
   uint64_t gcmask;  // controls outside the tile

@@ -95,6 +95,33 @@ std::vector<PGate> cnot_to_cz(const std::vector<PGate> &gates) {
   return out;
 }
 
+std::vector<PGate> diagonals_to_phases(const std::vector<PGate> &gates) {
+  using cplx = std::complex<double>;
+  std::vector<PGate> out;
+  out.reserve(gates.size());
+  auto unit = [](const cplx &z) { return std::abs(std::abs(z) - 1.0) < 1e-9; };
+  for (const PGate &g : gates) {
+    const bool diagonal = g.tpos.size() == 1 && g.m.size() == 4 && g.m[1] == cplx(0.0) && g.m[2] == cplx(0.0);
+    if (!diagonal || !unit(g.m[0]) || !unit(g.m[3]) || (g.m[0] == cplx(1.0) && g.m[3] == cplx(-1.0))) {
+      out.push_back(g);
+      continue;
+    }
+    if (g.m[0] != cplx(1.0)) {
+      PGate p;
+      p.m = {g.m[0]};
+      p.cmask = g.cmask;
+      out.push_back(std::move(p));
+    }
+    if (g.m[3] != g.m[0]) {
+      PGate p;
+      p.m = {g.m[0] == cplx(1.0) ? g.m[3] : g.m[3] / g.m[0]};
+      p.cmask = g.cmask | g.tmask();
+      out.push_back(std::move(p));
+    }
+  }
+  return out;
+}
+
 std::vector<uint32_t> choose_by_score(const std::vector<SlotCandidate> &cands, unsigned slots) {
   std::vector<SlotCandidate> c = cands;
   std::stable_sort(c.begin(), c.end(), [](const SlotCandidate &a, const SlotCandidate &b) {
@@ -189,7 +216,7 @@ std::vector<PPass> schedule_tiles(const std::vector<PGate> &gates, const TileSha
       std::vector<double> score(n, 0.0), cnt(n, 0.0), firstr(n, -1.0);
       unsigned rank = 0;
       for (int i = first; i < G && rank < lookahead; ++i) {
-        if (done[i]) continue;
+        if (done[i] || gates[i].tpos.empty()) continue;
         for (uint32_t lab : gates[i].tpos) {
           const uint32_t p = pos_of(lab);
           if (p < L0) continue;
@@ -248,7 +275,7 @@ std::vector<PPass> schedule_tiles(const std::vector<PGate> &gates, const TileSha
       std::vector<double> need(phys.size(), 1e300);
       unsigned rank = 0;
       for (int i = first; i < G && rank < lookahead; ++i) {
-        if (done[i]) continue;
+        if (done[i] || gates[i].tpos.empty()) continue;
         for (uint32_t lab : gates[i].tpos) need[pos_of(lab)] = std::min(need[pos_of(lab)], (double)rank);
         ++rank;
       }
@@ -388,6 +415,10 @@ uint32_t pad_stage_bits(uint32_t need, unsigned t, unsigned rb, bool c64) {
   return best;
 }
 
+bool diagonal_matrix(const LocalGate &g) {
+  return g.k == 1 ? (*g.m)[1] == cplx(0.0) && (*g.m)[2] == cplx(0.0) : g.k == 2 && is_diag4(*g.m);
+}
+
 void emit_reg_stage(const std::vector<LocalGate> &run, uint32_t bits, unsigned t, unsigned rb, bool c64,
                     TileProgram &prog) {
   bits = pad_stage_bits(bits, t, rb, c64);
@@ -404,7 +435,43 @@ void emit_reg_stage(const std::vector<LocalGate> &run, uint32_t bits, unsigned t
   if (nb != rb) throw std::runtime_error("tile pass: register stage width");
   dev::fill_stage_offsets(st, rb, c64);
   st.begin = (uint32_t)prog.rops.size();
+  // Phases wait, by the register bits they need set, until a gate writes one of those bits: the factors
+  // of a group are multiplied up first and reach the amplitudes once.
+  struct Factor {
+    uint32_t lc;
+    uint64_t gc;
+    cplx f;
+  };
+  std::vector<Factor> waiting[32];
+  auto apply_phases = [&](uint32_t written) {
+    for (uint32_t mask = 0; mask < (1u << rb); ++mask) {
+      if (waiting[mask].empty() || !(mask & written)) continue;
+      dev::RegOp group{};
+      group.code = dev::kOpPhases << 8 | mask;
+      group.rcmask = (uint32_t)waiting[mask].size();
+      group.mat = (uint32_t)prog.mats.size();
+      prog.rops.push_back(group);
+      for (const Factor &w : waiting[mask]) {
+        dev::RegOp term{};
+        term.code = dev::kOpPhaseTerm << 8;
+        term.lcmask = w.lc;
+        term.gcmask = w.gc;
+        prog.mats.push_back(w.f);
+        prog.rops.push_back(term);
+      }
+      waiting[mask].clear();
+    }
+  };
+  auto all_phases = [&] {
+    apply_phases(~0u);
+    if (waiting[0].empty()) return;
+    waiting[1].swap(waiting[0]);  // mask 0 is written by no gate: it goes with the rest
+    const size_t at = prog.rops.size();
+    apply_phases(1u);
+    prog.rops[at].code = dev::kOpPhases << 8;
+  };
   auto close_stage = [&]() {
+    all_phases();
     st.end = (uint32_t)prog.rops.size();
     if (st.end > st.begin) prog.stages.push_back(st);
     st.begin = st.end;
@@ -417,6 +484,14 @@ void emit_reg_stage(const std::vector<LocalGate> &run, uint32_t bits, unsigned t
       if (regbit[p] >= 0) op.rcmask |= 1u << regbit[p];
       else op.lcmask |= 1u << p;
     }
+    if (g.k == 0) {
+      std::vector<Factor> &w = waiting[op.rcmask];
+      size_t i = 0;
+      while (i < w.size() && (w[i].lc != op.lcmask || w[i].gc != op.gcmask)) ++i;
+      if (i < w.size()) w[i].f *= (*g.m)[0];
+      else w.push_back({op.lcmask, op.gcmask, (*g.m)[0]});
+      continue;
+    }
     if (popcount32(op.rcmask) > 1) {
       // the register kernels take at most one register-bit control: run this gate on the LDS
       // tile between the ops before it and the ops after it
@@ -425,6 +500,11 @@ void emit_reg_stage(const std::vector<LocalGate> &run, uint32_t bits, unsigned t
       continue;
     }
     const uint32_t cb = op.rcmask ? 1u + (uint32_t)__builtin_ctz(op.rcmask) : 0u;
+    if (!diagonal_matrix(g)) {
+      uint32_t written = 0;
+      for (uint32_t l = 0; l < g.k; ++l) written |= 1u << regbit[g.tb[l]];
+      apply_phases(written);
+    }
     op.mat = (uint32_t)prog.mats.size();
     if (g.k == 1) {
       const uint32_t b0 = (uint32_t)regbit[g.tb[0]];
@@ -492,6 +572,16 @@ void partition_stages(const std::vector<LocalGate> &lgs, const std::vector<char>
       ps.erase(std::unique(ps.begin(), ps.end()), ps.end());
     }
   }
+  // the same lists without the phases, which any stage takes: what a phase waits for in its place
+  std::vector<std::vector<int>> through(n);
+  for (int i = 0; i < n; ++i) {
+    for (int p : preds[i]) {
+      if (lgs[p].k == 0) through[i].insert(through[i].end(), through[p].begin(), through[p].end());
+      else through[i].push_back(p);
+    }
+    std::sort(through[i].begin(), through[i].end());
+    through[i].erase(std::unique(through[i].begin(), through[i].end()), through[i].end());
+  }
   std::vector<char> done(n, 0);
   auto ready = [&](int i) {
     for (int p : preds[i])
@@ -510,7 +600,7 @@ void partition_stages(const std::vector<LocalGate> &lgs, const std::vector<char>
       std::vector<int> window;
       uint32_t cand = 0;
       for (int i = f; i < n && (int)window.size() < kWindow; ++i) {
-        if (done[i] || lds_only[i]) continue;
+        if (done[i] || lds_only[i] || lgs[i].k == 0) continue;
         window.push_back(i);
         cand |= tm[i];
       }
@@ -527,7 +617,7 @@ void partition_stages(const std::vector<LocalGate> &lgs, const std::vector<char>
         for (int k = 0; k < nw; ++k) {
           const int i = window[k];
           needs[k] = 0;
-          for (int p : preds[i]) {
+          for (int p : through[i]) {
             if (p < f) continue;  // placed
             const auto it = std::lower_bound(window.begin(), window.end(), p);
             if (it == window.end() || *it != p) stuck |= uint64_t(1) << k;  // not among the gates simulated
@@ -580,7 +670,8 @@ void partition_stages(const std::vector<LocalGate> &lgs, const std::vector<char>
       for (bool progress = true; progress;) {
         progress = false;
         for (int i = f; i < n; ++i) {
-          if (done[i] || lds_only[i] || (tm[i] & ~bits) || popcount32(lgs[i].lc & bits) > 1 || !ready(i)) continue;
+          if (done[i] || lds_only[i] || (tm[i] & ~bits) || !ready(i)) continue;
+          if (lgs[i].k > 0 && popcount32(lgs[i].lc & bits) > 1) continue;
           done[i] = 1;
           run.push_back(lgs[i]);
           progress = true;
@@ -642,7 +733,7 @@ void build_tile_pass(const std::vector<PGate> &gates, const PPass &ps, unsigned 
     const PGate &g = gates[gi];
     LocalGate lg{};
     lg.k = (uint32_t)g.tpos.size();
-    if (lg.k < 1 || lg.k > 5) throw std::runtime_error("tile pass: gate width outside 1..5");
+    if (lg.k > 5 || (lg.k == 0 && (rb != 4 || t < rb))) throw std::runtime_error("tile pass: gate width outside 1..5");
     uint32_t need = 0;
     for (uint32_t l = 0; l < lg.k; ++l) {
       const uint32_t p = at(g.tpos[l]);
@@ -679,13 +770,18 @@ PassFeatures tile_pass_features(const TileProgram &prog, unsigned n, bool c64, u
   f[5] = P.h / 9.f;
   f[6] = (P.h ? P.hpos[0] : n) / 32.f;
   f[7] = rb / 5.f;
+  size_t n_ops = prog.rops.size() + prog.tops.size();
   float reg = 0, lds = 0, kinds[7] = {0, 0, 0, 0, 0, 0, 0}, rctl = 0, lctl = 0, gctl = 0, ldsflops = 0;
   for (const auto &st : prog.stages) (st.kind == dev::kStageRegisters ? reg : lds) += 1;
   for (const auto &op : prog.rops) {
     uint32_t kd = (op.code >> 8) & 15u;
-    if (kd == dev::kOp1Z) kd = dev::kOp1Diag;  // a diagonal op (cheaper than the general diagonal)
+    if (kd == dev::kOpPhaseTerm) {  // a few operations per thread, whatever its bits
+      --n_ops;
+      continue;
+    }
+    if (kd == dev::kOp1Z || kd == dev::kOpPhases) kd = dev::kOp1Diag;  // cheaper than the general diagonal
     kinds[std::min<uint32_t>(kd, 6)] += 1;
-    rctl += op.rcmask != 0;
+    rctl += op.rcmask != 0 && (op.code >> 8) != dev::kOpPhases;
     lctl += op.lcmask != 0;
     gctl += op.gcmask != 0;
   }
@@ -706,7 +802,7 @@ PassFeatures tile_pass_features(const TileProgram &prog, unsigned n, bool c64, u
   f[17] = lctl / 32.f;
   f[18] = gctl / 32.f;
   f[19] = ldsflops / 1024.f;
-  f[23] = std::log2(1.f + float(prog.rops.size() + prog.tops.size())) / 8.f;
+  f[23] = std::log2(1.f + float(n_ops)) / 8.f;
   return F;
 }
 

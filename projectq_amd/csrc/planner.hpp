@@ -17,7 +17,8 @@
 
 namespace qs {
 
-// A queued gate resolved to bit positions (matrix bit l <-> tpos[l]).
+// A queued gate resolved to bit positions (matrix bit l <-> tpos[l]).  Without targets it is a phase: the
+// amplitudes with all control bits set are multiplied by m[0].
 struct PGate {
   std::vector<std::complex<double>> m;
   std::vector<uint32_t> tpos;
@@ -68,6 +69,11 @@ using SlotChooser =
 // scheduler may move a diagonal gate past gates that only read its target.
 std::vector<PGate> cnot_to_cz(const std::vector<PGate> &gates);
 
+// Diagonal 1-qubit gates with any controls become phases: diag(a, d) is the factor a where the controls
+// are set and d / a where the target is set as well.  A phase has no target, so it fits every tile and
+// every stage (build_tile_pass).  Gates with |a| or |d| other than 1, and the sign flips diag(1, -1), stay.
+std::vector<PGate> diagonals_to_phases(const std::vector<PGate> &gates);
+
 // Merge runs of uncontrolled single-qubit gates on the same position (no other gate touching
 // that position in between) into one matrix product.
 std::vector<PGate> merge_single_qubit_runs(const std::vector<PGate> &gates);
@@ -79,7 +85,7 @@ constexpr size_t kPassUploadBudget = size_t(4) << 20;
 // Worst-case upload bytes of one gate: its complex128 matrix plus an LDS op and its own stage.
 inline size_t gate_upload_bytes(const PGate &g) {
   return sizeof(std::complex<double>) * (size_t(1) << (2 * g.tpos.size())) + sizeof(dev::TileOp) +
-         sizeof(dev::TileStage) + sizeof(dev::RegOp);
+         sizeof(dev::TileStage) + 2 * sizeof(dev::RegOp);
 }
 
 // Tile scheduling: repeatedly pick a tile (forced: the targets of the first unscheduled gate;

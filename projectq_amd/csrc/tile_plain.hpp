@@ -10,7 +10,8 @@ namespace dev {
 namespace {
 
 // TWO = false: the instantiation for passes without 2-qubit register ops (see reg_op)
-template <typename R, int RB, bool FULL, bool TWO = true>
+// PH = true: the one for passes with phase ops
+template <typename R, int RB, bool FULL, bool TWO = true, bool PH = false>
 __global__ __launch_bounds__(kBlock) void k_tile_pass(amp_t<R> *__restrict__ psi, uint64_t n_tiles,
                                                       TilePass P, const TileStage *__restrict__ stages,
                                                       const RegOp *__restrict__ rops,
@@ -23,7 +24,7 @@ __global__ __launch_bounds__(kBlock) void k_tile_pass(amp_t<R> *__restrict__ psi
   uint64_t *seg = reinterpret_cast<uint64_t *>(smem + (sizeof(amp_t<R>) << P.t));
   fill_segments(P, seg);
   for (uint64_t tix = blockIdx.x; tix < n_tiles; tix += gridDim.x)
-    tile_body<R, RB, FULL, TWO>(psi, tix, P, seg, tile, stages, rops, tops, mats);
+    tile_body<R, RB, FULL, TWO, PH>(psi, tix, P, seg, tile, stages, rops, tops, mats);
 }
 
 // Many circuits at once: workgroup b runs tile (b - job.first_block) of job block_job[b]; every
@@ -49,7 +50,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_tile_pass(amp_t<R> *__restrict
 
 template <typename R, int RB>
 void launch_tile_pass(amp_t<R> *psi, uint64_t n_tiles, const TilePass &P, const TileStage *d_stages,
-                      const RegOp *d_rops, const TileOp *d_tops, const amp_t<R> *d_mats, bool two_qubit_ops,
+                      const RegOp *d_rops, const TileOp *d_tops, const amp_t<R> *d_mats, TileForms forms,
                       hipStream_t s) {
   prepare_tile_kernels();
   const size_t lds = (sizeof(amp_t<R>) << P.t) + (sizeof(uint64_t) << P.h);
@@ -63,6 +64,12 @@ void launch_tile_pass(amp_t<R> *psi, uint64_t n_tiles, const TilePass &P, const 
   const uint64_t grid = std::min<uint64_t>(n_tiles, cap ? cap : std::max<uint64_t>(8192, n_tiles / 16));
   const uint64_t chunk = uint64_t(kStreamChunk) * kBlock * Vec16<R>::n;  // amplitudes streamed per round
   const uint64_t tsize = uint64_t(1) << P.t;
+  const bool two_qubit_ops = forms == kFormsAll;
+  if (forms == kFormsPhases) {
+    if (RB != 4 || tsize % chunk != 0) throw ValueError("tile pass: phase ops need full tiles and 4 register bits");
+    launch_tile_pass_phase(psi, n_tiles, P, d_stages, d_rops, d_tops, d_mats, (unsigned)grid, lds, s);
+    return;
+  }
   if constexpr (RB == 4 && sizeof(R) == 4) {  // the only instantiations of the pipelined kernel
     if (launch_tile_pass_pf(psi, n_tiles, P, d_stages, d_rops, d_tops, d_mats, two_qubit_ops, (unsigned)grid, lds, s))
       return;
@@ -117,7 +124,7 @@ void prepare_tile_kernels_of() {
 
 #define QS_INSTANTIATE_TILE(R, RB)                                                                              \
   template void launch_tile_pass<R, RB>(amp_t<R> *, uint64_t, const TilePass &, const TileStage *,             \
-                                        const RegOp *, const TileOp *, const amp_t<R> *, bool, hipStream_t);   \
+                                        const RegOp *, const TileOp *, const amp_t<R> *, TileForms, hipStream_t); \
   template void launch_batch_tile_pass<R, RB>(amp_t<R> *, const BatchJob *, const uint32_t *, uint32_t,        \
                                               uint32_t, const TileStage *, const RegOp *, const TileOp *,      \
                                               const amp_t<R> *, bool, hipStream_t);                            \
