@@ -53,6 +53,7 @@ SOURCES = [
     "tile_c128_rb4.hip",
     "kernels.hip",
     "math.hip",
+    "permute.hip",
     "energy.hip",
     "pauli_sum.hip",
     "measure.hip",

@@ -16,19 +16,20 @@ struct BitInsert {
   uint8_t pos[kMaxBits];
 };
 
-// One pass of an index-bit permutation through LDS tiles.  A tile holds the 2^m amplitudes whose
-// source bits outside `src_pos` are fixed; it is loaded with tile bit r at source position
-// src_pos[r] (the first bits are the source's lowest positions: contiguous reads) and stored with
-// tile bit r at destination position dst_pos[r] (the first bits are the destination's lowest
-// positions: contiguous writes), store tile bit r taking load tile bit st_from[r].  The tile id's
-// bits go to the source positions outer_src[i] and the destination positions outer_dst[i].
+// One pass of an index-bit permutation through LDS tiles (plan_permutation).  A tile holds the 2^m
+// amplitudes whose source bits outside `src_pos` are fixed.  Load bit r of a tile is at source position
+// src_pos[r] (the first bits are the source's lowest positions: contiguous reads), store bit r at
+// destination position dst_pos[r] (the destination's lowest first: contiguous writes).  The LDS slot
+// of an amplitude is linear in either: the XOR of slot_src[r] over its load bits, or of slot_dst[r] over its
+// store bits.  The tile id's bits go to the source positions outer_src[i] and the destination
+// positions outer_dst[i].
 constexpr int kPermTileMaxBits = 12;
 struct PermTile {
   uint32_t m, n_outer;
-  uint8_t src_pos[kPermTileMaxBits], dst_pos[kPermTileMaxBits], st_from[kPermTileMaxBits];
+  uint8_t src_pos[kPermTileMaxBits], dst_pos[kPermTileMaxBits];
+  uint16_t slot_src[kPermTileMaxBits], slot_dst[kPermTileMaxBits];
   uint8_t outer_src[kMaxBits], outer_dst[kMaxBits];
 };
-
 
 namespace dev {
 

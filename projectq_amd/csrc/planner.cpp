@@ -819,6 +819,84 @@ PassFeatures block_pass_features(unsigned k, unsigned n_ctrl, unsigned min_targe
   return F;
 }
 
+PermTile plan_permutation(const std::vector<unsigned> &to, bool c64) {
+  const unsigned n = (unsigned)to.size();
+  std::vector<unsigned> from(n);
+  for (unsigned p = 0; p < n; ++p) from[to[p]] = p;
+  // 32 KiB tiles (five workgroups per CU) with segments of 512 bytes at least on both sides: the lowest k
+  // positions of source and destination, then the next ones up to the full tile, so that a thread has
+  // eight 16-byte loads in flight
+  const unsigned most = c64 ? 12 : 11, k = std::min(n, most / 2), m = std::min(n, most);
+  std::vector<unsigned> tsrc;
+  auto in_tile = [&](unsigned p) { return std::find(tsrc.begin(), tsrc.end(), p) != tsrc.end(); };
+  for (unsigned p = 0; p < k; ++p) tsrc.push_back(p);
+  for (unsigned b = 0; b < k; ++b)
+    if (!in_tile(from[b])) tsrc.push_back(from[b]);
+  for (unsigned p = k; p < n && tsrc.size() < m; ++p) {
+    if (!in_tile(p)) tsrc.push_back(p);
+    if (tsrc.size() < m && !in_tile(from[p])) tsrc.push_back(from[p]);
+  }
+  std::sort(tsrc.begin(), tsrc.end());
+  std::vector<unsigned> tdst;
+  for (unsigned p : tsrc) tdst.push_back(to[p]);
+  std::sort(tdst.begin(), tdst.end());
+  PermTile P{};
+  P.m = (uint32_t)tsrc.size();
+  std::vector<unsigned> load_bit(P.m);  // of store bit r
+  for (unsigned r = 0; r < P.m; ++r) {
+    P.src_pos[r] = (uint8_t)tsrc[r];
+    P.dst_pos[r] = (uint8_t)tdst[r];
+    load_bit[r] = unsigned(std::find(tsrc.begin(), tsrc.end(), from[tdst[r]]) - tsrc.begin());
+  }
+  for (unsigned p = 0; p < n; ++p)
+    if (!in_tile(p)) {
+      P.outer_src[P.n_outer] = (uint8_t)p;
+      P.outer_dst[P.n_outer++] = (uint8_t)to[p];
+    }
+  // LDS slots: load bit r < w is slot bit r, a higher one also flips some of the low w bits (the bank of
+  // an access of 2^w lanes: 32 of 8 bytes, 16 of 16).  Two sets of bits vary over those lanes: the load
+  // bits from v on and the load bits of the store bits from v on, v = 1 where a lane moves a pair of amplitudes.
+  // Wanted: flips under which both sets reach every bank.
+  const unsigned w = std::min(c64 ? 5u : 4u, (unsigned)P.m), v = c64 ? 1 : 0;
+  std::vector<uint32_t> col(P.m);
+  auto banks = [&](auto &&bit) {
+    uint32_t basis[8] = {}, rank = 0;
+    for (unsigned i = v; i < v + w && i < P.m; ++i) {
+      uint32_t c = col[bit(i)] & ((1u << w) - 1);
+      for (unsigned b = w; b-- > 0 && c;) {
+        if (!((c >> b) & 1)) continue;
+        if (!basis[b]) {
+          basis[b] = c;
+          ++rank;
+          break;
+        }
+        c ^= basis[b];
+      }
+    }
+    return rank;
+  };
+  std::vector<uint32_t> best(P.m);
+  uint32_t best_rank = 0, seed = 1;
+  for (int attempt = 0; attempt < 256 && best_rank < 2 * w; ++attempt) {
+    for (unsigned r = 0; r < P.m; ++r) {
+      seed = seed * 1664525u + 1013904223u;
+      col[r] = 1u << r | (r >= w && attempt ? (seed >> 16) & ((1u << w) - 1) : 0u);
+    }
+    const uint32_t rank = banks([](unsigned i) { return i; }) + banks([&](unsigned i) { return load_bit[i]; });
+    if (rank > best_rank) {
+      best_rank = rank;
+      best = col;
+    }
+  }
+  if (best_rank == 0)
+    for (unsigned r = 0; r < P.m; ++r) best[r] = 1u << r;
+  for (unsigned r = 0; r < P.m; ++r) {
+    P.slot_src[r] = (uint16_t)best[r];
+    P.slot_dst[r] = (uint16_t)best[load_bit[r]];
+  }
+  return P;
+}
+
 void PauliEncoder::add(uint32_t pos, char op) {
   if (pos >= 64) throw std::invalid_argument("Pauli string position out of range");
   const uint64_t q = uint64_t(1) << pos;

@@ -114,6 +114,9 @@ struct TileProgram {
 void build_tile_pass(const std::vector<PGate> &gates, const PPass &pass, unsigned t, unsigned rb, bool c64,
                      TileProgram &prog);
 
+// The index-bit permutation that sends source position p to to[p], as one pass through LDS tiles.
+PermTile plan_permutation(const std::vector<unsigned> &to, bool c64);
+
 // A Pauli string applied left to right, ops given as (bit position, 'X'|'Y'|'Z'), equals
 // omega * X^x Z^z:  X_q: x ^= q;  Z_q: omega *= (-1)^{x_q}, z ^= q;  Y_q = i X_q Z_q:
 // omega *= i (-1)^{x_q}, x ^= q, z ^= q.  Then (P psi)_i = omega (-1)^{popcount((i^x)&z)} psi_{i^x}.
