@@ -1153,12 +1153,21 @@ void Engine::emulate_math_op(int opcode, const std::vector<int64_t> &params,
     for (unsigned q : regs[r]) at[r].push_back(pos_.at(q));
   MathGather g;
   if (plan_math_gather(opcode, (int32_t)a.a, (int32_t)a.N, at, a.cmask, n_, c64_, &g)) {
-    void *dst = scratch(0);
-    dispatch([&](auto tag) {
-      using R = decltype(tag);
-      dev::math_gather<R>((const amp_t<R> *)psi_, (amp_t<R> *)dst, amps(), g, stream_);
-    });
-    std::swap(psi_, buf_[0]);
+    // In place where the changing bits fit an LDS tile: less traffic under controls, and no scratch.
+    MathTile tile;
+    if (plan_math_tile(g, n_, c64_, &tile)) {
+      dispatch([&](auto tag) {
+        using R = decltype(tag);
+        dev::math_tile<R>((amp_t<R> *)psi_, amps(), g, tile, stream_);
+      });
+    } else {
+      void *dst = scratch(0);
+      dispatch([&](auto tag) {
+        using R = decltype(tag);
+        dev::math_gather<R>((const amp_t<R> *)psi_, (amp_t<R> *)dst, amps(), g, stream_);
+      });
+      std::swap(psi_, buf_[0]);
+    }
     norm_changed();
     subspace_unknown();
     return;

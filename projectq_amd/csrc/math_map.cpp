@@ -141,4 +141,39 @@ bool plan_math_gather(int opcode, int64_t a, int64_t N, const std::vector<std::v
   return true;
 }
 
+bool plan_math_tile(const MathGather &G, unsigned n, bool c64, MathTile *out) {
+  MathTile &T = *out;
+  T = MathTile{};
+  const unsigned most = c64 ? kMathTileBits64 : kMathTileBits128;
+  // the changing bits and 256 contiguous bytes; then the lowest positions that are no controls
+  uint64_t in = G.changed;
+  for (unsigned p = 0; p < (c64 ? 5u : 4u) && p < n; ++p) in |= uint64_t(1) << p;
+  if ((unsigned)__builtin_popcountll(in) > most) return false;
+  for (unsigned p = 0; p < n && (unsigned)__builtin_popcountll(in) < most; ++p)
+    if (!((G.cmask >> p) & 1)) in |= uint64_t(1) << p;
+  T.fixed = G.cmask & ~in;
+  std::vector<unsigned> at, rest;
+  for (unsigned p = 0; p < n; ++p) {
+    if ((in >> p) & 1) at.push_back(p);
+    else if (!((T.fixed >> p) & 1)) rest.push_back(p);
+  }
+  T.m = (uint32_t)at.size();
+  T.outside = (uint32_t)rest.size();
+  T.tile = runs_of(at);
+  T.tile_id = runs_of(rest);
+  for (int b = 0; b < kMathThreadBits; ++b) {
+    T.step[b] = 8u + b < T.m ? uint64_t(1) << at[8 + b] : 0;
+    for (int r = 0; r < G.n_regs; ++r) T.reg_step[b][r] = (uint32_t)gather_bits(T.step[b], G.reg[r]);
+  }
+  T.changed = (uint32_t)gather_bits(G.changed, T.tile);
+  for (int r = 0; r < G.n_regs; ++r) {
+    if (!G.moves[r]) continue;
+    std::vector<unsigned> local(G.width[r]);
+    for (uint32_t b = 0; b < G.width[r]; ++b)
+      local[b] = (unsigned)__builtin_ctzll(gather_bits(scatter_bits(uint64_t(1) << b, G.reg[r]), T.tile));
+    T.local[r] = runs_of(local);
+  }
+  return true;
+}
+
 }  // namespace qs

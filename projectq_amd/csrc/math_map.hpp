@@ -34,6 +34,12 @@ QS_HD inline uint64_t scatter_bits(uint64_t value, const BitRuns &r) {
   return i;
 }
 
+QS_HD inline uint32_t scatter_bits32(uint32_t value, const BitRuns &r) {  // positions below 32
+  uint32_t i = 0;
+  for (uint32_t k = 0; k < r.n; ++k) i |= ((value >> r.bit[k]) & ((1u << r.len[k]) - 1)) << r.pos[k];
+  return i;
+}
+
 // What the gather kernel computes per destination: the register values (u, v, w) of the one source,
 // or, modulo N, of the first of a few sources.
 enum MathSource : int32_t {
@@ -70,6 +76,23 @@ struct MathGather {
 // or constant outside what the rules below cover), and the general path decides.
 bool plan_math_gather(int opcode, int64_t a, int64_t N, const std::vector<std::vector<unsigned>> &regs, uint64_t cmask,
                       unsigned n, bool c64, MathGather *out);
+
+// The same call in place, where every index bit that changes fits one LDS tile (the destinations of a tile
+// then have all their sources in it).
+struct MathTile {
+  uint32_t m;         // tile bits
+  uint32_t changed;   // tile bits that change
+  uint64_t fixed;     // controls outside the tile: only the indices that have them set are visited
+  uint32_t outside;   // index bits of the tile number
+  BitRuns tile_id;    // tile number -> index bits
+  BitRuns tile;       // tile-local index <-> index bits
+  BitRuns local[3];   // register value <-> tile-local index (registers that change)
+  // index and register values of tile-local bits 8..11 (the amplitudes of one thread)
+  uint64_t step[kMathThreadBits];
+  uint32_t reg_step[kMathThreadBits][3];
+};
+constexpr unsigned kMathTileBits64 = 12, kMathTileBits128 = 11;  // 32 KiB
+bool plan_math_tile(const MathGather &G, unsigned n, bool c64, MathTile *out);
 
 // Source values (u, v, w) of one destination under the rule S = G.source; returns false where there is
 // no source (modulo N only).
@@ -112,6 +135,19 @@ QS_HD inline bool math_source(const MathGather &G, uint64_t &u, uint64_t &v, uin
       return true;
     }
   }
+}
+
+// The residue rules on registers of at most 16 bits, in 32-bit arithmetic (64-bit products are a dozen
+// quarter-rate instructions): the first source of destination u < N, magic = floor(2^32 / N).
+template <int S>
+QS_HD inline uint32_t residue_source32(uint32_t u, uint32_t a, uint32_t N, uint32_t magic) {
+  if (S == kSrcAddMod) return u >= a ? u - a : u + N - a;
+  const uint32_t p = u * a;  // below 2^32; the quotient is one or two too small at most
+  const uint32_t q = (uint32_t)(((uint64_t)p * magic) >> 32);
+  uint32_t r = p - q * N;
+  if (r >= N) r -= N;
+  if (r >= N) r -= N;
+  return r;
 }
 
 }  // namespace qs
