@@ -233,6 +233,7 @@ class Engine {
   // state in HBM); every call that hands the layout out restores it first (canonicalize).
   std::map<unsigned, unsigned> ref_pos_;
   void canonicalize();
+  void restore_layout(double scale);
   std::vector<Gate> window_;  // queued gates, both fusion modes
   // block fusion: window_ is cut into the reference's blocks as gates arrive (ends_: the end of each
   // block that is complete, open_: the qubits of the one that is not)

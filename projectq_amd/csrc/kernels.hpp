@@ -98,9 +98,9 @@ void drop_bit(const amp_t<R> *src, amp_t<R> *dst, uint64_t n_out, int p, int val
 // In place: exchange index bits a and b (a != b) of every amplitude of a 2^n state
 template <typename R>
 void swap_bits(amp_t<R> *psi, uint64_t n_amps, int a, int b, hipStream_t s);
-// dst <- src with its index bits permuted, one pass through LDS tiles (PermTile)
+// dst <- scale * src with its index bits permuted, one pass through LDS tiles (PermTile)
 template <typename R>
-void permute_tiles(const amp_t<R> *src, amp_t<R> *dst, uint64_t n_amps, const PermTile &P, hipStream_t s);
+void permute_tiles(const amp_t<R> *src, amp_t<R> *dst, uint64_t n_amps, const PermTile &P, double scale, hipStream_t s);
 
 // psi_i *= c where (i & cmask) == cmask
 template <typename R>

@@ -22,9 +22,10 @@ constexpr int kPair = sizeof(R) == 4 ? 2 : 1;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef double f64x2 __attribute__((ext_vector_type(2)));
 
-template <typename R>
+// SCALE: the amplitudes are multiplied by `scale` as well (in FP64, as k_scale_masked does)
+template <typename R, bool SCALE>
 __global__ __launch_bounds__(kBlock) void k_permute_tiles(const amp_t<R> *__restrict__ src, amp_t<R> *__restrict__ dst,
-                                                          uint64_t n_tiles, PermTile P) {
+                                                          uint64_t n_tiles, PermTile P, double scale) {
   constexpr int VN = kPair<R>, V0 = VN == 2 ? 1 : 0, JB = 3, NJ = 1 << JB;  // tile bits V0.. thread, V0 + 8.. turn
   extern __shared__ __align__(16) unsigned char smem[];
   amp_t<R> *tile = reinterpret_cast<amp_t<R> *>(smem);
@@ -56,6 +57,7 @@ __global__ __launch_bounds__(kBlock) void k_permute_tiles(const amp_t<R> *__rest
       if ((j >> b) & 1) v ^= bits[b];
     return v;
   };
+  auto scaled = [&](R v) { return SCALE ? (R)((double)v * scale) : v; };
   for (uint64_t id = blockIdx.x; id < n_tiles; id += gridDim.x) {
     uint64_t sb = src_t, db = dst_t;
     for (uint32_t i = 0; i < P.n_outer; ++i) {
@@ -83,7 +85,7 @@ __global__ __launch_bounds__(kBlock) void k_permute_tiles(const amp_t<R> *__rest
         if ((uint32_t)j * kBlock + threadIdx.x < units) {
           const uint32_t s = out_t ^ of(j, out_j);
           const amp_t<R> a = tile[s], b = tile[s ^ pair];
-          f32x4 o = {a.x, a.y, b.x, b.y};
+          f32x4 o = {scaled(a.x), scaled(a.y), scaled(b.x), scaled(b.y)};
           __builtin_nontemporal_store(o, reinterpret_cast<f32x4 *>(dst + (db ^ of(j, dst_j))));
         }
     } else {
@@ -99,9 +101,11 @@ __global__ __launch_bounds__(kBlock) void k_permute_tiles(const amp_t<R> *__rest
       __syncthreads();
 #pragma unroll
       for (int j = 0; j < NJ; ++j)
-        if ((uint32_t)j * kBlock + threadIdx.x < units)
-          __builtin_nontemporal_store(reinterpret_cast<const f64x2 *>(tile)[out_t ^ of(j, out_j)],
-                                      reinterpret_cast<f64x2 *>(dst + (db ^ of(j, dst_j))));
+        if ((uint32_t)j * kBlock + threadIdx.x < units) {
+          const f64x2 a = reinterpret_cast<const f64x2 *>(tile)[out_t ^ of(j, out_j)];
+          f64x2 o = {scaled(a.x), scaled(a.y)};
+          __builtin_nontemporal_store(o, reinterpret_cast<f64x2 *>(dst + (db ^ of(j, dst_j))));
+        }
     }
     __syncthreads();  // the tile is free for the next turn
   }
@@ -110,7 +114,7 @@ __global__ __launch_bounds__(kBlock) void k_permute_tiles(const amp_t<R> *__rest
 }  // namespace
 
 template <typename R>
-void permute_tiles(const amp_t<R> *src, amp_t<R> *dst, uint64_t n_amps, const PermTile &P, hipStream_t s) {
+void permute_tiles(const amp_t<R> *src, amp_t<R> *dst, uint64_t n_amps, const PermTile &P, double scale, hipStream_t s) {
   // a turn of 256 threads takes 2^8 units of 16 bytes, 8 turns at most; a pair needs one tile bit
   const uint32_t most = sizeof(R) == 4 ? 12 : 11;
   if (P.m > most || P.m < (sizeof(R) == 4 ? 1u : 0u) || (uint64_t(1) << P.m) > n_amps || P.m + P.n_outer > 64 ||
@@ -118,13 +122,16 @@ void permute_tiles(const amp_t<R> *src, amp_t<R> *dst, uint64_t n_amps, const Pe
     throw ValueError("permute_tiles: bad tile");
   const uint64_t n_tiles = n_amps >> P.m;
   const uint64_t grid = std::min<uint64_t>(n_tiles, 16384);
-  hipLaunchKernelGGL(k_permute_tiles<R>, dim3((unsigned)grid), dim3(kBlock), sizeof(amp_t<R>) << P.m, s, src, dst, n_tiles,
-                     P);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(kBlock), sizeof(amp_t<R>) << P.m, s, src, dst, n_tiles, P, scale);
+  };
+  if (scale == 1.0) go(k_permute_tiles<R, false>);
+  else go(k_permute_tiles<R, true>);
   QS_HIP(hipGetLastError());
 }
 
-template void permute_tiles<float>(const float2 *, float2 *, uint64_t, const PermTile &, hipStream_t);
-template void permute_tiles<double>(const double2 *, double2 *, uint64_t, const PermTile &, hipStream_t);
+template void permute_tiles<float>(const float2 *, float2 *, uint64_t, const PermTile &, double, hipStream_t);
+template void permute_tiles<double>(const double2 *, double2 *, uint64_t, const PermTile &, double, hipStream_t);
 
 }  // namespace dev
 }  // namespace qs
