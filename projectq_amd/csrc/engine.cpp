@@ -215,6 +215,14 @@ void Engine::check_known(const std::vector<unsigned> &ids, const char *what) con
     if (!pos_.count(q)) throw RuntimeError(std::string(what) + ": Unknown qubit id.");
 }
 
+// compact index -> index of the amplitudes whose bits in `fixed` are given
+BitRuns Engine::free_runs(uint64_t fixed) const {
+  std::vector<unsigned> free;
+  for (unsigned p = 0; p < n_; ++p)
+    if (!((fixed >> p) & 1)) free.push_back(p);
+  return runs_of(free);
+}
+
 uint64_t Engine::mask_of(const std::vector<unsigned> &ids) const {
   uint64_t m = 0;
   for (unsigned q : ids) m |= uint64_t(1) << pos_.at(q);
@@ -249,10 +257,10 @@ void Engine::allocate_qubit(unsigned id) {
 // Whether an amplitude above tol has the bit of qubit `id` clear (bit 0 of the answer) and set (bit 1).
 int Engine::sides(unsigned id, double tol) {
   const bool known = tol >= 0.0;  // the amplitudes known to be zero are not above it
-  const BitInsert sub = make_insert(bits_of(known ? zmask_ : 0));
+  const uint64_t fixed = known ? zmask_ : 0;
   dispatch([&](auto tag) {
     using R = decltype(tag);
-    dev::classical<R>((const amp_t<R> *)psi_, amps() >> sub.count, sub, known ? zval_ : 0, (int)pos_[id], tol, d_flags_, h_flags_,
+    dev::classical<R>((const amp_t<R> *)psi_, amps() >> __builtin_popcountll(fixed), free_runs(fixed), known ? zval_ : 0, (int)pos_[id], tol, d_flags_, h_flags_,
                       stream_);
   });
   sync();
@@ -336,8 +344,8 @@ std::vector<uint8_t> Engine::measure_qubits(const std::vector<unsigned> &ids) {
   dev::MeasureArgs a{};
   a.rnd = uni_(rng_);
   a.n_amps = amps();
-  a.sub = make_insert(bits_of(zmask_));
-  a.n_sub = a.n_amps >> a.sub.count;
+  a.free = free_runs(zmask_);
+  a.n_sub = a.n_amps >> __builtin_popcountll(zmask_);
   a.sval = zval_;
   a.zmask = zmask_;
   a.mask = mask_of(ids);

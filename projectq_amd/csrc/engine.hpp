@@ -122,6 +122,7 @@ class Engine {
   void sync();
   void check_known(const std::vector<unsigned> &ids, const char *what) const;
   uint64_t mask_of(const std::vector<unsigned> &ids) const;
+  BitRuns free_runs(uint64_t fixed) const;
   void pauli_encode(const PauliString &t, const std::vector<unsigned> &ids, uint64_t *x,
                     uint64_t *z, cplx *omega) const;
   dev::MathArgs math_args(const std::vector<std::vector<unsigned>> &regs,

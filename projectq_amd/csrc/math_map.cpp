@@ -5,8 +5,6 @@
 
 namespace qs {
 
-namespace {
-
 BitRuns runs_of(const std::vector<unsigned> &positions) {
   BitRuns r{};
   for (size_t b = 0; b < positions.size(); ++b) {
@@ -21,6 +19,8 @@ BitRuns runs_of(const std::vector<unsigned> &positions) {
   }
   return r;
 }
+
+namespace {
 
 // x with a x = 1 (mod N), 0 if there is none
 uint64_t inverse_mod(uint64_t a, uint64_t N) {

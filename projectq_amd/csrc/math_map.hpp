@@ -71,6 +71,9 @@ struct MathGather {
   uint32_t reg_step[kMathThreadBits][3];
 };
 
+// Positions in the order of the value's bits.
+BitRuns runs_of(const std::vector<unsigned> &positions);
+
 // Registers as bit positions, ascending significance.  true: `out` describes the call, whose sources
 // are found from the destination.  false: nothing is known about the map (a shared qubit, a width
 // or constant outside what the rules below cover), and the general path decides.

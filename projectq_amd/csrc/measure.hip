@@ -8,6 +8,10 @@
 // Large subspaces are read once for the chunk sums (split by the measured bit, so that the norm of
 // the outcome needs no second read) and written once by the collapse, which does not load what it
 // clears; up to 4096 amplitudes one workgroup does everything.
+// What is left between the large reads is latency, so loads go out in batches before their first use, the
+// amplitudes of a subspace are found by runs of free bits (after k measured qubits: one run, not k
+// fixed bits to insert), and chunks are short enough for a thousand workgroups.  One pick took 25 us, the
+// chunk sums of 2^19 amplitudes 28 us and a measurement of 4096 amplitudes 112 us, FIGURES now.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -19,13 +23,8 @@ namespace qs {
 namespace dev {
 namespace {
 
-__device__ __forceinline__ uint64_t insert_zeros(uint64_t g, const BitInsert &ins) {
-  for (uint32_t i = 0; i < ins.count; ++i) {
-    const uint32_t p = ins.pos[i];
-    g = ((g >> p) << (p + 1)) | (g & ((uint64_t(1) << p) - 1));
-  }
-  return g;
-}
+// index of the subspace's amplitude c
+__device__ __forceinline__ uint64_t index_of(uint64_t c, const MeasureArgs &a) { return scatter_bits(c, a.free) | a.sval; }
 template <typename A>
 __device__ __forceinline__ double norm2(const A &a) {
   const double x = a.x, y = a.y;
@@ -71,6 +70,36 @@ __device__ __forceinline__ bool contradicts(const MeasureArgs &a, uint64_t pick)
   return ((pick ^ a.sval) & a.mask & a.zmask) != 0;
 }
 
+// The first j in [lo, hi) at which run + value(lo) + ... + value(j) reaches the draw, hi if none; a batch of
+// loads at a time.
+constexpr int kBatch = 8;
+template <class I, class F>
+__device__ __forceinline__ I first_reaching(I lo, I hi, double run, double rnd, F &&value) {
+  for (I j = lo; j < hi; j += kBatch) {
+    double v[kBatch];
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) v[k] = j + k < hi ? value(j + k) : 0.0;
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) {
+      run += v[k];
+      if (run >= rnd && j + k < hi) return j + k;
+    }
+  }
+  return hi;
+}
+template <class I, class F>
+__device__ __forceinline__ double sum_range(I lo, I hi, F &&value) {
+  double sum = 0.0;
+  for (I j = lo; j < hi; j += kBatch) {
+    double v[kBatch];
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) v[k] = j + k < hi ? value(j + k) : 0.0;
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) sum += v[k];
+  }
+  return sum;
+}
+
 // The in-order scan of `len` compact indices from `start` by a workgroup of NT threads: the first index
 // at which base + running norm reaches the draw, ~0 if none.  *total: base + their norm.
 template <typename R, int NT>
@@ -79,54 +108,75 @@ __device__ __forceinline__ unsigned long long scan_pick(const amp_t<R> *psi, con
                                                         double *total) {
   const uint64_t per = (len + NT - 1) / NT;
   const uint64_t lo = min<uint64_t>(len, threadIdx.x * per), hi = min<uint64_t>(len, lo + per);
-  double mine = 0.0;
-  for (uint64_t j = lo; j < hi; ++j) mine += norm2(psi[insert_zeros(start + j, a.sub) | a.sval]);
+  auto value = [&](uint64_t j) { return norm2(psi[index_of(start + j, a)]); };
+  const double mine = sum_range(lo, hi, value);
   if (threadIdx.x == 0) *found = ~0ull;
   double sum;
-  double run = base + prefix<NT>(mine, lds, &sum);  // its barriers order *found before the scan
+  const double run = base + prefix<NT>(mine, lds, &sum);  // its barriers order *found before the scan
   *total = base + sum;
-  for (uint64_t j = lo; j < hi; ++j) {
-    run += norm2(psi[insert_zeros(start + j, a.sub) | a.sval]);
-    if (run >= a.rnd) {
-      atomicMin(found, (unsigned long long)(start + j));
-      break;
-    }
-  }
+  const uint64_t at = first_reaching(lo, hi, run, a.rnd, value);
+  if (at < hi) atomicMin(found, (unsigned long long)(start + at));
   __syncthreads();
   return *found;
 }
 
-template <typename R>
-__global__ __launch_bounds__(kBlock) void k_measure_small(amp_t<R> *__restrict__ psi, MeasureArgs a,
-                                                          unsigned long long *__restrict__ host_pick) {
-  __shared__ double lds[kBlock / 64];
+// The subspace in registers: kMeasureSmall / NT consecutive amplitudes per thread, read once.
+template <typename R, int NT>
+__global__ __launch_bounds__(NT) void k_measure_small(amp_t<R> *__restrict__ psi, MeasureArgs a,
+                                                      unsigned long long *__restrict__ host_pick) {
+  constexpr int PER = kMeasureSmall / 1024;
+  __shared__ double lds[NT / 64];
   __shared__ unsigned long long found;
+  uint64_t at[PER];
+  amp_t<R> v[PER];
+  double norm[PER], mine = 0.0;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const uint64_t c = (uint64_t)threadIdx.x * PER + k;
+    at[k] = index_of(c, a);
+    v[k].x = v[k].y = 0;
+    if (c < a.n_sub) v[k] = psi[at[k]];
+  }
+#pragma unroll
+  for (int k = 0; k < PER; ++k) mine += norm[k] = norm2(v[k]);
   uint64_t pick = ~uint64_t(0);
   if (a.rnd > 0.0) {
+    if (threadIdx.x == 0) found = ~0ull;
     double total;
-    const unsigned long long c = scan_pick<R, kBlock>(psi, a, 0, a.n_sub, 0.0, lds, &found, &total);
-    if (c != ~0ull) pick = insert_zeros(c, a.sub) | a.sval;
-    else pick = total >= a.rnd ? insert_zeros(a.n_sub - 1, a.sub) | a.sval : a.n_amps - 1;
+    double run = prefix<NT>(mine, lds, &total);  // its barriers order `found` before the scan
+    unsigned long long mine_at = ~0ull;
+#pragma unroll
+    for (int k = PER - 1; k >= 0; --k) {  // the first that reaches the draw is kept
+      double r = run;
+#pragma unroll
+      for (int i = 0; i <= k; ++i) r += norm[i];
+      if (r >= a.rnd && (uint64_t)threadIdx.x * PER + k < a.n_sub) mine_at = (uint64_t)threadIdx.x * PER + k;
+    }
+    if (mine_at != ~0ull) atomicMin(&found, mine_at);
+    __syncthreads();
+    const unsigned long long c = found;
+    if (c != ~0ull) pick = index_of(c, a);
+    else pick = total >= a.rnd ? index_of(a.n_sub - 1, a) : a.n_amps - 1;
   }
   if (threadIdx.x == 0) *host_pick = pick;
   const uint64_t val = pick & a.mask;
   double kept = 0.0;
-  if (!contradicts(a, pick))
-    for (uint64_t c = threadIdx.x; c < a.n_sub; c += kBlock) {
-      const uint64_t i = insert_zeros(c, a.sub) | a.sval;
-      if ((i & a.mask) == val) kept += norm2(psi[i]);
+  if (!contradicts(a, pick)) {
+#pragma unroll
+    for (int k = 0; k < PER; ++k)
+      if ((at[k] & a.mask) == val) kept += norm[k];  // 0 beyond the subspace
+  }
+  const double scale = 1.0 / sqrt(sum_all<NT>(kept, lds));
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    if ((uint64_t)threadIdx.x * PER + k >= a.n_sub) continue;
+    amp_t<R> w;
+    w.x = w.y = 0;
+    if ((at[k] & a.mask) == val) {
+      w.x = (R)((double)v[k].x * scale);
+      w.y = (R)((double)v[k].y * scale);
     }
-  const double scale = 1.0 / sqrt(sum_all<kBlock>(kept, lds));
-  for (uint64_t c = threadIdx.x; c < a.n_sub; c += kBlock) {
-    const uint64_t i = insert_zeros(c, a.sub) | a.sval;
-    amp_t<R> v;
-    v.x = v.y = 0;
-    if ((i & a.mask) == val) {
-      v = psi[i];
-      v.x = (R)((double)v.x * scale);
-      v.y = (R)((double)v.y * scale);
-    }
-    psi[i] = v;
+    psi[at[k]] = w;
   }
 }
 
@@ -139,7 +189,7 @@ __global__ __launch_bounds__(kBlock) void k_measure_chunks(const amp_t<R> *__res
   const uint64_t base = (uint64_t)blockIdx.x << lg, len = uint64_t(1) << lg;
   double clear = 0.0, set = 0.0;
   for (uint64_t j = threadIdx.x; j < len; j += kBlock) {
-    const uint64_t i = insert_zeros(base + j, a.sub) | a.sval;
+    const uint64_t i = index_of(base + j, a);
     const double v = norm2(psi[i]);
     if ((i & a.mask) == a.mask) set += v;
     else clear += v;
@@ -167,39 +217,32 @@ __global__ __launch_bounds__(kPickThreads) void k_measure_pick(const amp_t<R> *_
   if (a.rnd > 0.0) {
     const uint32_t per = (chunks + kPickThreads - 1) / kPickThreads;
     const uint32_t lo = min(chunks, threadIdx.x * per), hi = min(chunks, lo + per);
-    double mine = 0.0;
-    for (uint32_t c = lo; c < hi; ++c) mine += sums[2 * c] + sums[2 * c + 1];
+    auto value = [&](uint32_t c) { return sums[2 * c] + sums[2 * c + 1]; };
+    const double mine = sum_range(lo, hi, value);
     if (threadIdx.x == 0) found = ~0ull;
     double total;
     const double start = prefix<kPickThreads>(mine, lds, &total);
-    double run = start;
-    for (uint32_t c = lo; c < hi; ++c) {
-      run += sums[2 * c] + sums[2 * c + 1];
-      if (run >= a.rnd) {
-        atomicMin(&found, (unsigned long long)c);
-        break;
-      }
-    }
+    const uint32_t at = first_reaching(lo, hi, start, a.rnd, value);
+    if (at < hi) atomicMin(&found, (unsigned long long)at);
     __syncthreads();
     const unsigned long long chunk = found;
     if (chunk == ~0ull) {
       pick = a.n_amps - 1;  // the draw exceeds the total norm: the scan runs off the end
     } else {
       if (chunk >= lo && chunk < hi) {
-        double r = start;
-        for (uint32_t c = lo; c < chunk; ++c) r += sums[2 * c] + sums[2 * c + 1];
-        before = r;
+        before = start + sum_range(lo, (uint32_t)chunk, value);
       }
       __syncthreads();
       const uint64_t len = uint64_t(1) << lg;
       const unsigned long long c =
           scan_pick<R, kPickThreads>(psi, a, chunk * len, len, before, lds, &found, &total);
-      pick = insert_zeros(c != ~0ull ? (uint64_t)c : (chunk + 1) * len - 1, a.sub) | a.sval;
+      pick = index_of(c != ~0ull ? (uint64_t)c : (chunk + 1) * len - 1, a);
     }
   }
   double kept = 0.0;
   if (single && !contradicts(a, pick)) {
     const uint32_t set = (pick & a.mask) ? 1 : 0;
+#pragma unroll 8
     for (uint32_t c = threadIdx.x; c < chunks; c += kPickThreads) kept += sums[2 * c + set];
   }
   kept = sum_all<kPickThreads>(kept, lds);
@@ -219,7 +262,7 @@ __global__ __launch_bounds__(kBlock) void k_measure_kept(const amp_t<R> *__restr
   double kept = 0.0;
   if (!contradicts(a, pick))
     for (uint64_t c = (uint64_t)blockIdx.x * kBlock + threadIdx.x; c < a.n_sub; c += (uint64_t)gridDim.x * kBlock) {
-      const uint64_t i = insert_zeros(c, a.sub) | a.sval;
+      const uint64_t i = index_of(c, a);
       if ((i & a.mask) == val) kept += norm2(psi[i]);
     }
   kept = sum_all<kBlock>(kept, lds);
@@ -239,7 +282,7 @@ __global__ __launch_bounds__(kBlock) void k_measure_collapse(amp_t<R> *__restric
   const uint64_t val = m->pick & a.mask;
   const double scale = m->scale;
   for (uint64_t c = (uint64_t)blockIdx.x * kBlock + threadIdx.x; c < a.n_sub; c += (uint64_t)gridDim.x * kBlock) {
-    const uint64_t i = insert_zeros(c, a.sub) | a.sval;
+    const uint64_t i = index_of(c, a);
     amp_t<R> v;
     v.x = v.y = 0;
     if ((i & a.mask) == val) {
@@ -253,12 +296,12 @@ __global__ __launch_bounds__(kBlock) void k_measure_collapse(amp_t<R> *__restric
 
 // SMALL: one workgroup, which writes the answer itself.
 template <typename R, bool SMALL>
-__global__ __launch_bounds__(kBlock) void k_classical(const amp_t<R> *__restrict__ psi, uint64_t n_sub, BitInsert sub,
+__global__ __launch_bounds__(kBlock) void k_classical(const amp_t<R> *__restrict__ psi, uint64_t n_sub, BitRuns free,
                                                       uint64_t sval, int p, double tol, int *__restrict__ count,
                                                       int *__restrict__ flags) {
   int lo = 0, hi = 0;
   for (uint64_t c = (uint64_t)blockIdx.x * kBlock + threadIdx.x; c < n_sub; c += (uint64_t)gridDim.x * kBlock) {
-    const uint64_t i = insert_zeros(c, sub) | sval;
+    const uint64_t i = scatter_bits(c, free) | sval;
     const amp_t<R> v = psi[i];
     const double x = v.x, y = v.y;
     const int big = (x * x + y * y) > tol;
@@ -289,12 +332,16 @@ template <typename R>
 void measure(amp_t<R> *psi, const MeasureArgs &a, Measurement *m, unsigned long long *pick, double *sums, double *partials,
              hipEvent_t picked, hipStream_t s) {
   if (a.n_sub <= kMeasureSmall) {
-    hipLaunchKernelGGL(k_measure_small<R>, dim3(1), dim3(kBlock), 0, s, psi, a, pick);
+    // as few waves as hold the subspace: their barriers are most of the time on 10 qubits and fewer
+    if (a.n_sub <= 64 * 4) hipLaunchKernelGGL((k_measure_small<R, 64>), dim3(1), dim3(64), 0, s, psi, a, pick);
+    else if (a.n_sub <= 256 * 4) hipLaunchKernelGGL((k_measure_small<R, 256>), dim3(1), dim3(256), 0, s, psi, a, pick);
+    else hipLaunchKernelGGL((k_measure_small<R, 1024>), dim3(1), dim3(1024), 0, s, psi, a, pick);
     QS_HIP(hipGetLastError());
     QS_HIP(hipEventRecord(picked, s));
     return;
   }
-  int lg = 12;
+  int lg = 8;  // about a thousand chunks, from 2^8 amplitudes to 2^12, then as many as fit the sums
+  while (lg < 12 && (a.n_sub >> lg) > 1024) ++lg;
   while ((a.n_sub >> lg) > kMeasureChunks) ++lg;
   const uint32_t chunks = (uint32_t)(a.n_sub >> lg);
   const int single = a.mask != 0 && (a.mask & (a.mask - 1)) == 0;
@@ -314,16 +361,16 @@ void measure(amp_t<R> *psi, const MeasureArgs &a, Measurement *m, unsigned long 
 }
 
 template <typename R>
-void classical(const amp_t<R> *psi, uint64_t n_sub, const BitInsert &sub, uint64_t sval, int p, double tol, int *count,
+void classical(const amp_t<R> *psi, uint64_t n_sub, const BitRuns &free, uint64_t sval, int p, double tol, int *count,
                int *flags, hipStream_t s) {
   if (n_sub <= 4 * kMeasureSmall) {
-    hipLaunchKernelGGL((k_classical<R, true>), dim3(1), dim3(kBlock), 0, s, psi, n_sub, sub, sval, p, tol, count, flags);
+    hipLaunchKernelGGL((k_classical<R, true>), dim3(1), dim3(kBlock), 0, s, psi, n_sub, free, sval, p, tol, count, flags);
     QS_HIP(hipGetLastError());
     return;
   }
   hipLaunchKernelGGL(k_classical_clear, dim3(1), dim3(2), 0, s, count);
   QS_HIP(hipGetLastError());
-  hipLaunchKernelGGL((k_classical<R, false>), dim3(grid_of(n_sub)), dim3(kBlock), 0, s, psi, n_sub, sub, sval, p, tol, count, flags);
+  hipLaunchKernelGGL((k_classical<R, false>), dim3(grid_of(n_sub)), dim3(kBlock), 0, s, psi, n_sub, free, sval, p, tol, count, flags);
   QS_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_classical_flags, dim3(1), dim3(1), 0, s, count, flags);
   QS_HIP(hipGetLastError());
@@ -332,7 +379,7 @@ void classical(const amp_t<R> *psi, uint64_t n_sub, const BitInsert &sub, uint64
 #define QS_INSTANTIATE_MEASURE(R)                                                                                       \
   template void measure<R>(amp_t<R> *, const MeasureArgs &, Measurement *, unsigned long long *, double *, double *,   \
                            hipEvent_t, hipStream_t);                                                                    \
-  template void classical<R>(const amp_t<R> *, uint64_t, const BitInsert &, uint64_t, int, double, int *, int *, hipStream_t);
+  template void classical<R>(const amp_t<R> *, uint64_t, const BitRuns &, uint64_t, int, double, int *, int *, hipStream_t);
 QS_INSTANTIATE_MEASURE(double)
 QS_INSTANTIATE_MEASURE(float)
 

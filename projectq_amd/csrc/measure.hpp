@@ -2,6 +2,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "math_map.hpp"
 
 namespace qs {
 namespace dev {
@@ -20,8 +21,8 @@ constexpr uint64_t kMeasureSmall = 4096;
 
 struct MeasureArgs {
   uint64_t n_amps, n_sub;  // amplitudes of the state, and of the subspace outside which they are zero
-  BitInsert sub;           // the subspace's fixed bits
-  uint64_t sval, zmask;    // their values, and their mask
+  BitRuns free;            // the subspace's free bits: compact index -> index
+  uint64_t sval, zmask;    // the values of the fixed bits, and their mask
   uint64_t mask;           // index bits of the measured qubits
   double rnd;              // the draw; 0: the reference's loop never runs and the pick is all ones
 };
@@ -36,7 +37,7 @@ void measure(amp_t<R> *psi, const MeasureArgs &a, Measurement *m, unsigned long 
 // *flags (pinned) <- bit 0: an amplitude > tol with index bit p clear, bit 1: one with it set, over the
 // subspace.  count: two ints of device memory.
 template <typename R>
-void classical(const amp_t<R> *psi, uint64_t n_sub, const BitInsert &sub, uint64_t sval, int p, double tol, int *count,
+void classical(const amp_t<R> *psi, uint64_t n_sub, const BitRuns &free, uint64_t sval, int p, double tol, int *count,
                int *flags, hipStream_t s);
 
 }  // namespace dev
