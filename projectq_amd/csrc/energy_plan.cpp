@@ -78,6 +78,14 @@ void complete(Span &span, uint64_t *gen, uint32_t L, uint32_t h, uint8_t *pivot)
 
 void plan_energy(const EnergyTerm *terms, int count, unsigned n, bool c64, uint64_t workgroups, EnergyPlan &plan) {
   tile_of(n, c64, c64 ? 12u : 11u, &plan.t, &plan.L, &plan.h);
+  // One generator more for segments of 128 bytes: an eighth string per read of the state.  It pays where
+  // the state is beyond the caches (from 128 MiB on) and the strings need a second read: 27 qubits complex128,
+  // 30 random strings 2.00 -> 1.82 ms, 28 qubits complex64, 40 random strings 3.09 -> 2.91 ms (6 -> 5
+  // reads); six strings, one read either way, 0.54 and 0.56 ms; 22 qubits the same.
+  if (n >= (c64 ? 24u : 23u) && count > (int)plan.h) {
+    --plan.L;
+    ++plan.h;
+  }
   // 32 KiB of LDS, 256 threads with 16 (complex64) or 8 (complex128) amplitudes each
   plan.n_passes = plan.n_groups = plan.n_strings = 0;
 
