@@ -1,25 +1,23 @@
-"""Energies of states beyond the caches, where the tiles have shorter segments: against torch in 64 bits.
+"""Energies of states beyond the caches, where the tiles have shorter segments: against numpy in 64 bits.
 
 The products and sums are FP64 on the stored amplitudes: 2^24 terms of a normalised state, each string within
 2^24 * 2^-53 of exact in the worst case, far less pairwise."""
 
+import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n,precision,terms", [(23, "c64", 12), (24, "c64", 7), (24, "c64", 8), (24, "c64", 30), (23, "c128", 20)])
-def test_energy_against_torch(n, precision, terms):
-    import numpy as np
-    import torch
-
+@pytest.mark.parametrize("n,precision,terms", [(24, "c64", 7), (24, "c64", 8), (23, "c128", 9)])
+def test_energy_against_numpy(n, precision, terms):
     from projectq_amd import Simulator
 
-    gen = torch.Generator(device="cuda").manual_seed(n + terms)
-    real = torch.float32 if precision == "c64" else torch.float64
-    psi = torch.randn(1 << n, 2, generator=gen, device="cuda", dtype=real)
-    psi = torch.view_as_complex(psi.div_(float(psi.double().square().sum()) ** 0.5))
-    rng = np.random.default_rng(n)
+    rng = np.random.default_rng(n + terms)
+    psi = rng.normal(size=1 << n) + 1j * rng.normal(size=1 << n)
+    psi /= np.linalg.norm(psi)
+    if precision == "c64":
+        psi = psi.astype(np.complex64).astype(np.complex128)
     ham = []
     for _ in range(terms):
         ops = rng.integers(0, 4, size=n)
@@ -27,16 +25,17 @@ def test_energy_against_torch(n, precision, terms):
     sim = Simulator(1, precision=precision, capacity_qubits=n)
     for q in range(n):
         sim.allocate_qubit(q)
-    sim.set_wavefunction_device(psi, list(range(n)))
+    sim.set_wavefunction(psi, list(range(n)))
     got = sim.get_expectation_value(ham, list(range(n)))
-    wide, index, want = psi.to(torch.complex128), torch.arange(1 << n, device="cuda"), 0.0
+    index, want = np.arange(1 << n, dtype=np.uint32), 0.0
     for ops, c in ham:
-        x = sum(1 << q for q, p in ops if p in "XY")
-        z = sum(1 << q for q, p in ops if p in "YZ")
+        x = np.uint32(sum(1 << q for q, p in ops if p in "XY"))
+        z = np.uint32(sum(1 << q for q, p in ops if p in "YZ"))
         source = index ^ x
-        sign = source & z
-        for shift in (32, 16, 8, 4, 2, 1):
-            sign = sign ^ (sign >> shift)
-        image = wide[source] * (1.0 - 2.0 * (sign & 1).double()) * (1j ** sum(p == "Y" for _, p in ops))
-        want += c * float((wide.conj() * image).real.sum())
+        odd = source & z
+        for shift in (16, 8, 4, 2, 1):
+            odd ^= odd >> np.uint32(shift)
+        image = psi[source]
+        image[(odd & 1) == 1] *= -1.0
+        want += c * (np.vdot(psi, image) * 1j ** sum(p == "Y" for _, p in ops)).real
     assert abs(got - want) <= 2.0 ** 24 * 2.0 ** -53 * sum(abs(c) for _, c in ham)
