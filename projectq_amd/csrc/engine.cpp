@@ -465,7 +465,9 @@ void Engine::exec_blocks() {
   }
   if (tiles) {
     unsigned t;
-    exec_programs(plan_tiles(resolve(gates, c64_ && cnot_cz_), tile_tmax_, tile_rb_, tile_lmin_, kSlotEarliest, false, &t),
+    const Resolved pg = resolve(gates, c64_ && cnot_cz_);
+    if (!pg.phases.empty()) queued_drift_ *= 2.0;  // a diagonal gate in two phases rounds two factors
+    exec_programs(plan_tiles(pg, tile_tmax_, tile_rb_, tile_lmin_, kSlotEarliest, false, &t),
                   tile_rb_);
   } else {
     size_t i = 0;
@@ -714,6 +716,7 @@ void Engine::plan_window(const std::vector<Gate> &gates, std::vector<Block> *blo
     return;
   }
   const Resolved pg = resolve(gates, cnot_cz_);
+  if (!pg.phases.empty()) queued_drift_ *= 2.0;  // a diagonal gate in two phases rounds two factors
   if (planner_kind_ == 2) {
     unsigned t;
     *progs_out = plan_tiles(pg, tile_tmax_, tile_rb_, tile_lmin_, slot_rule_, relabel_mode_ == 1, &t);

@@ -114,7 +114,8 @@ std::vector<PGate> diagonals_to_phases(const std::vector<PGate> &gates) {
     }
     if (g.m[3] != g.m[0]) {
       PGate p;
-      p.m = {g.m[0] == cplx(1.0) ? g.m[3] : g.m[3] / g.m[0]};
+      using wide = std::complex<long double>;  // the quotient to half an ulp: its length is the norm's error
+      p.m = {g.m[0] == cplx(1.0) ? g.m[3] : cplx(wide(g.m[3]) / wide(g.m[0]))};
       p.cmask = g.cmask | g.tmask();
       out.push_back(std::move(p));
     }
