@@ -405,7 +405,7 @@ void Engine::apply_controlled_gate(Gate g) {
     window_.push_back(std::move(g));
     return;
   }
-  if (nonunitary) exec_blocks();  // the norm guard judges what is complete without it
+  if (nonunitary) exec_blocks();  // the norm guard looks at what is complete without it
   const unsigned before = open_.num_qubits();
   BlockQubits trial = open_;
   trial.insert(g);
