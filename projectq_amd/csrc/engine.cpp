@@ -405,7 +405,6 @@ void Engine::apply_controlled_gate(Gate g) {
     window_.push_back(std::move(g));
     return;
   }
-  if (nonunitary) exec_blocks();  // the norm guard looks at what is complete without it
   const unsigned before = open_.num_qubits();
   BlockQubits trial = open_;
   trial.insert(g);
@@ -417,6 +416,7 @@ void Engine::apply_controlled_gate(Gate g) {
   } else {
     open_ = std::move(trial);
   }
+  if (nonunitary) exec_blocks();  // the norm guard looks at what is complete without it
   queued();
   window_.push_back(std::move(g));
   if (full) close_block();
@@ -425,14 +425,17 @@ void Engine::apply_controlled_gate(Gate g) {
 // The open block is complete.  It runs with the ones before it at the next run() (every call that looks
 // at the state makes one): at once behind a gate that is not unitary, where the norm guard stops.
 void Engine::close_block() {
-  if (window_.size() == (ends_.empty() ? 0 : ends_.back())) return;
+  if (window_.size() == (ends_.empty() ? 0 : ends_.back().end)) return;
   if (open_.num_qubits() < 1 || open_.num_qubits() > 5) {  // the block stays queued, like the reference's
     exec_blocks();
     throw ValueError("Gates with more than 5 qubits are not supported!");
   }
-  ends_.push_back(window_.size());
+  const bool nonunitary = queued_nonunitary_;
+  ends_.push_back({window_.size(), queued_drift_, nonunitary});
   open_.clear();
-  if (queued_nonunitary_ || window_.size() >= kMaxPending) exec_blocks();
+  queued_drift_ = 0.0;
+  queued_nonunitary_ = false;
+  if (nonunitary || window_.size() >= kMaxPending) exec_blocks();
 }
 
 // simulator.hpp:487-527: the state after the queued gates.
@@ -453,11 +456,17 @@ void Engine::run() {
 // meaning outside their block's matrix.
 void Engine::exec_blocks() {
   if (ends_.empty()) return;
-  const std::vector<size_t> ends = std::move(ends_);
-  std::vector<Gate> gates(std::make_move_iterator(window_.begin()), std::make_move_iterator(window_.begin() + ends.back()));
-  window_.erase(window_.begin(), window_.begin() + ends.back());
+  const std::vector<BlockEnd> ends = std::move(ends_);
+  std::vector<Gate> gates(std::make_move_iterator(window_.begin()), std::make_move_iterator(window_.begin() + ends.back().end));
+  window_.erase(window_.begin(), window_.begin() + ends.back().end);
   ends_.clear();
-  before_unitary_passes();
+  double drift = 0.0;  // of these blocks: what is queued behind them keeps its own
+  bool nonunitary = false;
+  for (const BlockEnd &b : ends) {
+    drift += b.drift;
+    nonunitary |= b.nonunitary;
+  }
+  before_unitary_passes(nonunitary);
   bool tiles = ends.size() > 2;
   for (const Gate &g : gates) {
     uint64_t seen = mask_of(g.ids);
@@ -466,18 +475,18 @@ void Engine::exec_blocks() {
   if (tiles) {
     unsigned t;
     const Resolved pg = resolve(gates, c64_ && cnot_cz_);
-    if (!pg.phases.empty()) queued_drift_ *= 2.0;  // a diagonal gate in two phases rounds two factors
+    if (!pg.phases.empty()) drift *= 2.0;  // a diagonal gate in two phases rounds two factors
     exec_programs(plan_tiles(pg, tile_tmax_, tile_rb_, tile_lmin_, kSlotEarliest, false, &t),
                   tile_rb_);
   } else {
     size_t i = 0;
-    for (size_t end : ends) {
+    for (const BlockEnd &b : ends) {
       GateQueue queue;
-      for (; i < end; ++i) queue.insert(gates[i]);
+      for (; i < b.end; ++i) queue.insert(gates[i]);
       exec_block(queue.fuse());
     }
   }
-  after_passes();
+  after_passes(drift, nonunitary);
 }
 
 void Engine::exec_programs(const std::vector<TileProgram> &progs, unsigned rb) {
@@ -491,19 +500,16 @@ void Engine::exec_programs(const std::vector<TileProgram> &progs, unsigned rb) {
   }
 }
 
-void Engine::before_unitary_passes() {
-  if (!c64_ || queued_nonunitary_ || norm_known_) return;
+void Engine::before_unitary_passes(bool nonunitary) {
+  if (!c64_ || nonunitary || norm_known_) return;
   norm_ref_ = masked_norm(0, 0);
   norm_known_ = true;
   drift_bound_ = 0.0;
 }
 
-void Engine::after_passes() {
+void Engine::after_passes(double drift, bool nonunitary) {
   if (!c64_) return;
-  const double drift = queued_drift_;
-  queued_drift_ = 0.0;
-  if (queued_nonunitary_) {
-    queued_nonunitary_ = false;
+  if (nonunitary) {
     norm_changed();
     return;
   }
@@ -612,15 +618,19 @@ void Engine::flush_window() {
   PlanInfo info;
   plan_window(window_, &blocks, &progs, &rb, &info);
   window_.clear();
+  const double drift = queued_drift_;
+  const bool nonunitary = queued_nonunitary_;
+  queued_drift_ = 0.0;
+  queued_nonunitary_ = false;
   for (const TileProgram &p : progs) info.relabels += p.swaps.empty() ? 0u : 1u;
   last_plan_ = info;
-  before_unitary_passes();
+  before_unitary_passes(nonunitary);
   if (info.kind == 0) {
     for (const Block &b : blocks) exec_block(b);
   } else {
     exec_programs(progs, rb);
   }
-  after_passes();
+  after_passes(drift, nonunitary);
 }
 
 // The state moves to the reference's layout, in buf_[0], and is multiplied by `scale` on the way.

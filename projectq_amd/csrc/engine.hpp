@@ -142,14 +142,15 @@ class Engine {
   double norm_ref_ = 1.0;      // norm^2 of the state before the unitary gates since the last check
   bool norm_known_ = true;     // norm_ref_ is valid (the empty state |> has norm 1)
   double drift_bound_ = 0.0;   // bound on the relative norm change of the gates since the check
-  bool queued_nonunitary_ = false;  // a gate queued since the last execution is not unitary
-  double queued_drift_ = 0.0;       // drift bound of the gates queued since the last execution
+  // of the queued gates that no complete block holds: one is not unitary, and their drift bound
+  bool queued_nonunitary_ = false;
+  double queued_drift_ = 0.0;
   void norm_changed() {
     norm_known_ = false;
     drift_bound_ = 0.0;
   }
-  void before_unitary_passes();
-  void after_passes();
+  void before_unitary_passes(bool nonunitary);
+  void after_passes(double drift, bool nonunitary);
   // Known-zero amplitudes: every amplitude i with (i & zmask_) != zval_ is exactly zero (qubits
   // fixed by a measurement or a collapse, or freshly allocated and not touched by a non-diagonal
   // gate since).  Measurements then read and write only that subspace: after All(Measure) the k-th
@@ -237,8 +238,13 @@ class Engine {
   void restore_layout(double scale);
   std::vector<Gate> window_;  // queued gates, both fusion modes
   // block fusion: window_ is cut into the reference's blocks as gates arrive (ends_: the end of each
-  // block that is complete, open_: the qubits of the one that is not)
-  std::vector<size_t> ends_;
+  // block that is complete, and what the norm guard has to know of it; open_: the qubits of the one that is not)
+  struct BlockEnd {
+    size_t end;
+    double drift;
+    bool nonunitary;
+  };
+  std::vector<BlockEnd> ends_;
   BlockQubits open_;
   static constexpr size_t kMaxPending = 4096;  // gates of complete blocks that may wait
   void close_block();

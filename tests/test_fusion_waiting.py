@@ -1,0 +1,55 @@
+"""Complete blocks that wait under the reference's fusion rule (GPU): what runs them, and what of the queue is
+left when it does.
+
+The reference values come from the oracle or the mathematics.  8 roundings of half an ulp per gate bound the
+error: 8 * gates * 2^-24 (complex64) or 2^-53 (complex128) on amplitudes of at most 1.
+"""
+
+import numpy as np
+import pytest
+
+from oracle.cpu_sim import OracleSimulator
+
+pytestmark = pytest.mark.gpu
+
+EPS = {"c64": 2.0 ** -24, "c128": 2.0 ** -53}
+H = np.array([[1, 1], [1, -1]], dtype=complex) / np.sqrt(2.0)
+X = np.array([[0, 1], [1, 0]], dtype=complex)
+SQUEEZE = np.diag([1.0, 0.5]).astype(complex)
+
+BREAKS = {
+    "allocate": lambda sim: sim.allocate_qubit(3),
+    "synchronize": lambda sim: sim.synchronize(),
+    "stats": lambda sim: sim.stats(),
+    "reset_stats": lambda sim: sim.reset_stats(),
+    "set_profiling": lambda sim: sim.set_profiling(True),
+}
+
+
+def _amplitudes(sim):
+    return np.array(sim.cheat_numpy()[1])
+
+
+@pytest.mark.parametrize("what", list(BREAKS))
+def test_norm_guard_keeps_a_waiting_gate(what):
+    """A gate that is not unitary waits in the open block while the block before it runs: the norm guard
+    still stops at it, and the gates behind it do not scale its norm away."""
+    from projectq_amd import Simulator
+
+    sim, ref = Simulator(3, precision="c64"), OracleSimulator(3)
+    for s in (sim, ref):
+        for q in range(3):
+            s.allocate_qubit(q)
+            s.apply_controlled_gate(H, [q], [])
+        s.run()
+        s.apply_controlled_gate(H, [0], [])
+        s.apply_controlled_gate(SQUEEZE, [2], [1])  # does not fit the block of the H: closes it, opens its own
+        if s is sim or what == "allocate":
+            BREAKS[what](s)
+        s.run()
+        for _ in range(40):  # more drift than the guard's budget
+            s.apply_controlled_gate(H, [0], [])
+            s.run()
+    got, want = _amplitudes(sim), _amplitudes(ref)
+    assert np.linalg.norm(want) < 0.95
+    assert np.max(np.abs(got - want)) <= 8 * 45 * EPS["c64"]
