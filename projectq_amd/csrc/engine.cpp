@@ -452,8 +452,8 @@ void Engine::run() {
 // matrix product); several go through tile passes, which read the state once for the gates of many
 // blocks.  That is the faster way for every size measured, 5 layers of the random-layer circuit in
 // complex128: 6 qubits 427 us in blocks, 238 in tiles; 21 qubits 1210 and 860; 25 qubits 20.2 and 3.5 ms.
-// A pair of blocks is about even, so it stays with the blocks.  Gates that name a qubit twice have no
-// meaning outside their block's matrix.
+// A pair of blocks is about even, so it stays with the blocks.  Gates that name a qubit twice or have no
+// target have no meaning outside their block's matrix (a gate without targets is a phase to the planner).
 void Engine::exec_blocks() {
   if (ends_.empty()) return;
   const std::vector<BlockEnd> ends = std::move(ends_);
@@ -470,7 +470,7 @@ void Engine::exec_blocks() {
   bool tiles = ends.size() > 2;
   for (const Gate &g : gates) {
     uint64_t seen = mask_of(g.ids);
-    tiles = tiles && (size_t)__builtin_popcountll(seen) == g.ids.size() && !(seen & mask_of(g.ctrl));
+    tiles = tiles && !g.ids.empty() && (size_t)__builtin_popcountll(seen) == g.ids.size() && !(seen & mask_of(g.ctrl));
   }
   if (tiles) {
     unsigned t;

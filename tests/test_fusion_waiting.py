@@ -53,3 +53,29 @@ def test_norm_guard_keeps_a_waiting_gate(what):
     got, want = _amplitudes(sim), _amplitudes(ref)
     assert np.linalg.norm(want) < 0.95
     assert np.max(np.abs(got - want)) <= 8 * 45 * EPS["c64"]
+
+
+@pytest.mark.parametrize("n,precision", [(4, "c64"), (4, "c128"), (13, "c64"), (13, "c128"), (19, "c128"), (20, "c64")])
+def test_gates_without_targets(n, precision):
+    """A 1x1 matrix without targets, with and without controls, inside blocks of other gates.  19 qubits
+    complex128 and 20 complex64 have full tiles."""
+    from projectq_amd import Simulator
+
+    swap = np.eye(4, dtype=complex)[[0, 2, 1, 3]]
+    sim, ref = Simulator(3, precision=precision, capacity_qubits=n), OracleSimulator(3)
+    rng = np.random.default_rng(n)
+    gates = 0
+    for q in range(n):
+        sim.allocate_qubit(q)
+        ref.allocate_qubit(q)
+    for _ in range(4):
+        a, b, c, d = (int(q) for q in rng.permutation(n)[:4])
+        block = [(H, [a], []), (np.array([[np.exp(0.3j)]]), [], []), (H, [b], []), (np.array([[1j]]), [], [a]),
+                 (swap, [a, b], []), (H, [c], []), (X, [d], [a])]
+        for s in (sim, ref):
+            for m, t, k in block:
+                s.apply_controlled_gate(np.asarray(m, dtype=complex), t, k)
+        gates += len(block)
+    sim.run()
+    ref.run()
+    assert np.max(np.abs(_amplitudes(sim) - _amplitudes(ref))) <= 8 * gates * EPS[precision]
