@@ -75,9 +75,9 @@ Engine::Engine(uint32_t seed, int precision, int fusion_mode, int planner, unsig
   // tile shape: 2^t amplitudes of LDS per workgroup and rb register bits per thread in register
   // stages.  complex64: t = 12 (32 KiB, four workgroups per CU at 123 VGPRs), rb = 4;
   // complex128: t = 12 (64 KiB, two workgroups per CU), rb = 4.
-  tile_tmax_ = 12u;
-  tile_rb_ = 4u;
-  tile_lmin_ = c64_ ? 5u : 4u;
+  tile_tmax_ = kDefaultTile;
+  tile_rb_ = kDefaultRegBits;
+  tile_lmin_ = default_low_bits();
   if (const char *env = std::getenv("PROJECTQ_AMD_MFMA")) {
     if (!std::strcmp(env, "0")) mfma_mode_ = 0;
     else if (!std::strcmp(env, "all")) mfma_mode_ = 2;
@@ -454,30 +454,36 @@ void Engine::run() {
 // complex128: 6 qubits 427 us in blocks, 238 in tiles; 21 qubits 1210 and 860; 25 qubits 20.2 and 3.5 ms.
 // A pair of blocks is about even, so it stays with the blocks.  Gates that name a qubit twice or have no
 // target have no meaning outside their block's matrix (a gate without targets is a phase to the planner).
+// The tiles are the default ones, wide enough for five targets: the tile planner's settings are for windows.
 void Engine::exec_blocks() {
   if (ends_.empty()) return;
-  const std::vector<BlockEnd> ends = std::move(ends_);
-  std::vector<Gate> gates(std::make_move_iterator(window_.begin()), std::make_move_iterator(window_.begin() + ends.back().end));
-  window_.erase(window_.begin(), window_.begin() + ends.back().end);
-  ends_.clear();
+  const size_t count = ends_.back().end;
   double drift = 0.0;  // of these blocks: what is queued behind them keeps its own
   bool nonunitary = false;
-  for (const BlockEnd &b : ends) {
+  for (const BlockEnd &b : ends_) {
     drift += b.drift;
     nonunitary |= b.nonunitary;
   }
-  before_unitary_passes(nonunitary);
-  bool tiles = ends.size() > 2;
-  for (const Gate &g : gates) {
-    uint64_t seen = mask_of(g.ids);
-    tiles = tiles && !g.ids.empty() && (size_t)__builtin_popcountll(seen) == g.ids.size() && !(seen & mask_of(g.ctrl));
+  bool tiles = ends_.size() > 2;
+  for (size_t i = 0; i < count && tiles; ++i) {
+    const Gate &g = window_[i];
+    const uint64_t seen = mask_of(g.ids);
+    tiles = !g.ids.empty() && (size_t)__builtin_popcountll(seen) == g.ids.size() && !(seen & mask_of(g.ctrl));
   }
-  if (tiles) {
+  std::vector<TileProgram> progs;
+  if (tiles) {  // planned before the queue is touched: where planning fails, nothing has run and nothing is lost
     unsigned t;
-    const Resolved pg = resolve(gates, c64_ && cnot_cz_);
+    const Resolved pg = resolve(window_.data(), count, c64_ && cnot_cz_);
     if (!pg.phases.empty()) drift *= 2.0;  // a diagonal gate in two phases rounds two factors
-    exec_programs(plan_tiles(pg, tile_tmax_, tile_rb_, tile_lmin_, kSlotEarliest, false, &t),
-                  tile_rb_);
+    progs = plan_tiles(pg, kDefaultTile, kDefaultRegBits, default_low_bits(), kSlotEarliest, false, &t);
+  }
+  const std::vector<BlockEnd> ends = std::move(ends_);
+  const std::vector<Gate> gates(std::make_move_iterator(window_.begin()), std::make_move_iterator(window_.begin() + count));
+  window_.erase(window_.begin(), window_.begin() + count);
+  ends_.clear();
+  before_unitary_passes(nonunitary);
+  if (tiles) {
+    exec_programs(progs, kDefaultRegBits);
   } else {
     size_t i = 0;
     for (const BlockEnd &b : ends) {
@@ -554,10 +560,11 @@ std::vector<Block> Engine::greedy_blocks(const std::vector<Gate> &gates) const {
   return out;
 }
 
-Engine::Resolved Engine::resolve(const std::vector<Gate> &gates, bool cnot_cz) const {
+Engine::Resolved Engine::resolve(const Gate *gates, size_t count, bool cnot_cz) const {
   std::vector<PGate> pg;
-  pg.reserve(gates.size());
-  for (const Gate &g : gates) {
+  pg.reserve(count);
+  for (size_t i = 0; i < count; ++i) {
+    const Gate &g = gates[i];
     PGate p;
     p.m = g.m;
     for (unsigned id : g.ids) p.tpos.push_back(pos_.at(id));
@@ -725,7 +732,7 @@ void Engine::plan_window(const std::vector<Gate> &gates, std::vector<Block> *blo
     info->passes = (unsigned)blocks_out->size();
     return;
   }
-  const Resolved pg = resolve(gates, cnot_cz_);
+  const Resolved pg = resolve(gates.data(), gates.size(), cnot_cz_);
   if (!pg.phases.empty()) queued_drift_ *= 2.0;  // a diagonal gate in two phases rounds two factors
   if (planner_kind_ == 2) {
     unsigned t;

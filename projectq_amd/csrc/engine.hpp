@@ -167,14 +167,17 @@ class Engine {
   }
   void plan_window(const std::vector<Gate> &gates, std::vector<Block> *blocks, std::vector<TileProgram> *progs,
                    unsigned *rb, PlanInfo *info);
-  unsigned tile_tmax_ = 13, tile_rb_ = 5;  // tile shape limits (PROJECTQ_AMD_TILE="t:rb" overrides)
+  static constexpr unsigned kDefaultTile = 12, kDefaultRegBits = 4;
+  unsigned default_low_bits() const { return c64_ ? 5u : 4u; }
+  // tile shape limits of the tile planner (PROJECTQ_AMD_TILE="t:rb" overrides)
+  unsigned tile_tmax_ = kDefaultTile, tile_rb_ = kDefaultRegBits;
   unsigned tile_bits(unsigned tmax) const;
   std::vector<Block> greedy_blocks(const std::vector<Gate> &gates) const;
   struct Resolved {
     std::vector<PGate> gates;
     std::vector<PGate> phases;  // the same with phases for the diagonal gates; empty where that is no gain
   };
-  Resolved resolve(const std::vector<Gate> &gates, bool cnot_cz) const;
+  Resolved resolve(const Gate *gates, size_t count, bool cnot_cz) const;
   std::vector<TileProgram> plan_tiles(const Resolved &pg, unsigned tmax, unsigned rb, unsigned lmin,
                                       int rule, bool relabel, unsigned *t_used) const;
   int slot_rule_ = kSlotLookahead;  // rule of QS_PLANNER_TILE

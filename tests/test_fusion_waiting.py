@@ -79,3 +79,32 @@ def test_gates_without_targets(n, precision):
     sim.run()
     ref.run()
     assert np.max(np.abs(_amplitudes(sim) - _amplitudes(ref))) <= 8 * gates * EPS[precision]
+
+
+@pytest.mark.parametrize("shape", ["env", (10, 4, 8), (6, 4, 5)])
+@pytest.mark.parametrize("precision", ["c64", "c128"])
+def test_tile_planner_settings_leave_fusion_alone(precision, shape, monkeypatch):
+    """The tile planner's shape, here too narrow for three targets, has no say in what gate fusion runs."""
+    from projectq_amd import Simulator
+
+    n = 12
+    rng = np.random.default_rng(7)
+    q, _ = np.linalg.qr(rng.normal(size=(8, 8)) + 1j * rng.normal(size=(8, 8)))
+    if shape == "env":
+        monkeypatch.setenv("PROJECTQ_AMD_TILE", "6:4")
+    sim, ref = Simulator(3, precision=precision), OracleSimulator(3)
+    if shape != "env":
+        sim.set_tile_params(*shape)
+    gates = 0
+    for s in (sim, ref):
+        for k in range(n):
+            s.allocate_qubit(k)
+    for k in range(6):
+        picks = [int(v) for v in np.random.default_rng(k).permutation(n)[:3]]
+        for s in (sim, ref):
+            s.apply_controlled_gate(np.ascontiguousarray(q), picks, [])
+            s.apply_controlled_gate(H, [picks[0]], [])
+        gates += 2
+    sim.run()
+    ref.run()
+    assert np.max(np.abs(_amplitudes(sim) - _amplitudes(ref))) <= 8 * 8 * gates * EPS[precision]
