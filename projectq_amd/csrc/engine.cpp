@@ -431,7 +431,7 @@ void Engine::close_block() {
     throw ValueError("Gates with more than 5 qubits are not supported!");
   }
   const bool nonunitary = queued_nonunitary_;
-  ends_.push_back({window_.size(), queued_drift_, nonunitary});
+  ends_.push_back({window_.size(), open_.num_qubits(), queued_drift_, nonunitary});
   open_.clear();
   queued_drift_ = 0.0;
   queued_nonunitary_ = false;
@@ -450,11 +450,13 @@ void Engine::run() {
 
 // Runs the complete blocks.  One block is one pass over the state (and 8 to 13 us of host time for its
 // matrix product); several go through tile passes, which read the state once for the gates of many
-// blocks.  That is the faster way for every size measured, 5 layers of the random-layer circuit in
-// complex128: 6 qubits 427 us in blocks, 238 in tiles; 21 qubits 1210 and 860; 25 qubits 20.2 and 3.5 ms.
-// A pair of blocks is about even, so it stays with the blocks.  Gates that name a qubit twice or have no
-// target have no meaning outside their block's matrix (a gate without targets is a phase to the planner).
-// The tiles are the default ones, wide enough for five targets: the tile planner's settings are for windows.
+// blocks.  With gates of up to 3 targets that is the faster way for every size measured.  5 layers of the
+// random-layer circuit in complex128: 6 qubits 427 us in blocks, 238 in tiles; 21 qubits 1210 and 860; 25 qubits
+// 20.2 and 3.5 ms.  30 gates of 3 targets: 6 qubits 715 and 381 us, 24 qubits 2.1 and 1.7 ms.  With wider
+// gates blocks_faster decides.  A pair of blocks is about even, so it stays with the blocks.  Gates that name
+// a qubit twice or have no target have no meaning outside their block's matrix (a gate without targets is a phase
+// to the planner).  The tiles are the default ones, wide enough for five targets: the tile planner's settings
+// are for windows.
 void Engine::exec_blocks() {
   if (ends_.empty()) return;
   const size_t count = ends_.back().end;
@@ -470,6 +472,7 @@ void Engine::exec_blocks() {
     const uint64_t seen = mask_of(g.ids);
     tiles = !g.ids.empty() && (size_t)__builtin_popcountll(seen) == g.ids.size() && !(seen & mask_of(g.ctrl));
   }
+  tiles = tiles && !blocks_faster(count);
   std::vector<TileProgram> progs;
   if (tiles) {  // planned before the queue is touched: where planning fails, nothing has run and nothing is lost
     unsigned t;
@@ -493,6 +496,38 @@ void Engine::exec_blocks() {
     }
   }
   after_passes(drift, nonunitary);
+}
+
+// Whether the first `count` gates run faster in their blocks than in tile passes, a question only where
+// gates of 4 or 5 targets are among them.  Such a gate fills a block alone, so fusing saves nothing, and in a tile
+// pass it is an LDS stage of its own.  With 5 targets that stage loses to a pass of the dense kernel over a
+// large state (matrix cores for complex64), and wins where the host's matrix product for the block is the
+// longer part.  30 gates of 5 targets, complex128, in blocks and in tiles: 20 qubits 2.79 and 1.31 ms, 24 qubits
+// 3.9 and 6.8; of 4 targets: 22 qubits 0.83 and 0.94, 26 qubits 12.4 and 9.9.
+// Both ways in microseconds, before anything is planned.  A pass streams the state (a block's pass in 2/3 of the
+// time where it fits the Infinity Cache) or waits for its launch; about three wide gates share a tile pass; an LDS
+// stage has a time per amplitude and a least one; a block's matrix costs 2.4 ns per complex product.  The constants
+// are fitted to 384 circuits (6 to 27 qubits, both precisions, 6 to 40 gates, 10% to all of them with 3 to 5
+// targets): the choice is 0.1% slower than the better way on average and 11% at most, tiles always 4.4% and 85%.
+bool Engine::blocks_faster(size_t count) const {
+  size_t wide[6] = {};
+  for (size_t i = 0; i < count; ++i) ++wide[std::min<size_t>(window_[i].ids.size(), 5)];
+  if (wide[4] + wide[5] == 0) return false;
+  const double n = (double)amps(), bytes = (double)amp_bytes() * n, stream = 2.0 * bytes / 3.3e6;
+  const double in_cache = bytes <= (double)(256u << 20) ? 0.67 : 1.0;
+  double blocks = 0.0;
+  size_t i = 0;
+  for (const BlockEnd &b : ends_) {
+    double products = 0.0;
+    for (; i < b.end; ++i) products += std::ldexp(1.0, 2 * (int)b.qubits + (int)window_[i].ids.size());
+    blocks += std::max(in_cache * stream, 10.0 + 2.4e-3 * products);
+  }
+  const double least[6] = {0, 0, 0, 0.7, 8.5, 53.0};
+  const double per_amp[2][6] = {{0, 0, 0, 1.4e-6, 3.1e-6, 14.0e-6}, {0, 0, 0, 2.2e-6, 2.2e-6, 8.9e-6}};
+  const double passes = 1.0 + (n_ > 10 ? 0.35 * (double)(wide[4] + wide[5]) : 0.0);
+  double tiles = 5.3 + 3.7 * (double)count + passes * std::max(26.0, stream);
+  for (int k = 3; k <= 5; ++k) tiles += (double)wide[k] * std::max(least[k], per_amp[c64_][k] * n);
+  return blocks <= tiles;
 }
 
 void Engine::exec_programs(const std::vector<TileProgram> &progs, unsigned rb) {

@@ -244,6 +244,7 @@ class Engine {
   // block that is complete, and what the norm guard has to know of it; open_: the qubits of the one that is not)
   struct BlockEnd {
     size_t end;
+    unsigned qubits;
     double drift;
     bool nonunitary;
   };
@@ -252,6 +253,7 @@ class Engine {
   static constexpr size_t kMaxPending = 4096;  // gates of complete blocks that may wait
   void close_block();
   void exec_blocks();
+  bool blocks_faster(size_t count) const;
   std::mt19937 rng_;
   std::uniform_real_distribution<double> uni_{0.0, 1.0};
   hipStream_t stream_ = nullptr;

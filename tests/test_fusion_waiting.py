@@ -108,3 +108,32 @@ def test_tile_planner_settings_leave_fusion_alone(precision, shape, monkeypatch)
     sim.run()
     ref.run()
     assert np.max(np.abs(_amplitudes(sim) - _amplitudes(ref))) <= 8 * 8 * gates * EPS[precision]
+
+
+@pytest.mark.parametrize("n,k,precision,blocks", [
+    (12, 5, "c64", False), (12, 5, "c128", False), (21, 3, "c128", False), (21, 3, "c64", False),
+    (23, 5, "c128", True), (24, 5, "c64", True),
+])
+def test_wide_gates_take_the_faster_way(n, k, precision, blocks):
+    """Gates of 5 targets on large states run one per block (as many passes as gates), else the waiting
+    blocks share passes.  A row of a gate adds 2^k products."""
+    from projectq_amd import Simulator
+
+    sim, ref = Simulator(3, precision=precision, capacity_qubits=n), OracleSimulator(3)
+    rng = np.random.default_rng(n + k)
+    for q in range(n):
+        sim.allocate_qubit(q)
+        ref.allocate_qubit(q)
+    sim.run()
+    sim.reset_stats()
+    count = 6
+    for _ in range(count):
+        u, _ = np.linalg.qr(rng.normal(size=(1 << k, 1 << k)) + 1j * rng.normal(size=(1 << k, 1 << k)))
+        targets = [int(q) for q in rng.permutation(n)[:k]]
+        for s in (sim, ref):
+            s.apply_controlled_gate(np.ascontiguousarray(u), targets, [])
+    sim.run()
+    ref.run()
+    passes = sim.stats()["passes"]
+    assert passes == count if blocks else passes < count
+    assert np.max(np.abs(_amplitudes(sim) - _amplitudes(ref))) <= 8 * (1 << k) * count * EPS[precision]
