@@ -349,6 +349,8 @@ std::vector<uint8_t> Engine::measure_qubits(const std::vector<unsigned> &ids) {
   a.sval = zval_;
   a.zmask = zmask_;
   a.mask = mask_of(ids);
+  a.kept = free_runs(zmask_ | a.mask);
+  a.n_kept = a.n_amps >> __builtin_popcountll(zmask_ | a.mask);
   if (a.n_sub > dev::kMeasureSmall && !d_sums_) QS_HIP(hipMalloc(&d_sums_, 2 * dev::kMeasureChunks * sizeof(double)));
   dispatch([&](auto tag) {
     using R = decltype(tag);
