@@ -1230,7 +1230,24 @@ void Engine::emulate_math_op(int opcode, const std::vector<int64_t> &params,
   if (plan_math_gather(opcode, (int32_t)a.a, (int32_t)a.N, at, a.cmask, n_, c64_, &g)) {
     // In place where the changing bits fit an LDS tile: less traffic under controls, and no scratch.
     MathTile tile;
-    if (plan_math_tile(g, n_, c64_, &tile)) {
+    MathAdd add;
+    bool in_tiles = plan_math_tile(g, n_, c64_, &tile);
+    const bool adds = plan_math_add(g, &add);
+    if (opcode == 0) {
+      // An addition of a constant needs no pass for collisions on any path, so the others have to beat the general
+      // one.  On registers in order the gather from memory order does (complex64, all qubits in one register: 16
+      // qubits 30 and 24 us, 27 qubits 3.4 and 0.42 ms), and in turn loses to tiles where controls spare them
+      // traffic, from 32 MiB on (3 low qubits, 2 controls, 27 qubits: 0.40 and 0.14 ms).  On registers in another
+      // order a loop over the bits per amplitude is left, on all paths: from 11 to 21 qubits the general one is the
+      // fastest (18 qubits 34 us against 58), above it loses (27 qubits 3.4 ms against 2.4).
+      if (!adds && n_ > 10 && n_ <= 21) {
+        math_apply(a, nullptr, true);
+        return;
+      }
+      if (adds) in_tiles = in_tiles && amps() * amp_bytes() >= (uint64_t(32) << 20) && (tile.fixed || (c64_ && g.cmask));
+      else in_tiles = in_tiles && (c64_ || tile.fixed);
+    }
+    if (in_tiles) {
       dispatch([&](auto tag) {
         using R = decltype(tag);
         dev::math_tile<R>((amp_t<R> *)psi_, amps(), g, tile, stream_);
@@ -1239,7 +1256,8 @@ void Engine::emulate_math_op(int opcode, const std::vector<int64_t> &params,
       void *dst = scratch(0);
       dispatch([&](auto tag) {
         using R = decltype(tag);
-        dev::math_gather<R>((const amp_t<R> *)psi_, (amp_t<R> *)dst, amps(), g, stream_);
+        if (adds) dev::math_add<R>((const amp_t<R> *)psi_, (amp_t<R> *)dst, amps(), add, stream_);
+        else dev::math_gather<R>((const amp_t<R> *)psi_, (amp_t<R> *)dst, amps(), g, stream_);
       });
       std::swap(psi_, buf_[0]);
     }

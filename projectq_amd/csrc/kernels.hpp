@@ -116,6 +116,9 @@ void math_permute(const amp_t<R> *src, amp_t<R> *dst, uint64_t n_amps, const Mat
 // the same for the calls plan_math_gather covers (math_map.hpp): every destination reads its sources
 template <typename R>
 void math_gather(const amp_t<R> *src, amp_t<R> *dst, uint64_t n_amps, const MathGather &G, hipStream_t s);
+// additions of a constant on registers in ascending or descending order (plan_math_add)
+template <typename R>
+void math_add(const amp_t<R> *src, amp_t<R> *dst, uint64_t n_amps, const MathAdd &A, hipStream_t s);
 // in place, where the changing bits fit an LDS tile (plan_math_tile)
 template <typename R>
 void math_tile(amp_t<R> *psi, uint64_t n_amps, const MathGather &G, const MathTile &T, hipStream_t s);

@@ -10,6 +10,7 @@
 // which share the edges, run on one XCD and meet in its L2.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "kernels.hpp"
@@ -88,6 +89,30 @@ __global__ __launch_bounds__(kBlock) void k_math_gather(const amp_t<R> *__restri
     a.x = (R)0 + out[j].x;  // newvec starts at 0 (simulator.hpp:239-240): -0 becomes +0
     a.y = (R)0 + out[j].y;
     dst[it | part(j, step)] = a;
+  }
+}
+
+// Additions of a constant (MathAdd): a source costs a few operations however its bits lie, so the destinations
+// go in memory order with eight loads in flight per thread.
+template <typename R>
+__global__ __launch_bounds__(kBlock) void k_math_add(const amp_t<R> *__restrict__ src, amp_t<R> *__restrict__ dst,
+                                                     uint64_t n_amps, MathAdd A) {
+  constexpr int NJ = 8;
+  for (uint64_t first = (uint64_t)blockIdx.x * kBlock * NJ + threadIdx.x; first < n_amps; first += (uint64_t)gridDim.x * kBlock * NJ) {
+    amp_t<R> v[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      v[j].x = v[j].y = 0;
+      if (first + j * kBlock < n_amps) v[j] = src[add_source(A, first + j * kBlock)];
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      if (first + j * kBlock >= n_amps) continue;
+      amp_t<R> a;
+      a.x = (R)0 + v[j].x;  // newvec starts at 0 (simulator.hpp:239-240): -0 becomes +0
+      a.y = (R)0 + v[j].y;
+      dst[first + j * kBlock] = a;
+    }
   }
 }
 
@@ -199,6 +224,13 @@ void math_gather(const amp_t<R> *src, amp_t<R> *dst, uint64_t n_amps, const Math
 }
 
 template <typename R>
+void math_add(const amp_t<R> *src, amp_t<R> *dst, uint64_t n_amps, const MathAdd &A, hipStream_t s) {
+  const uint64_t grid = std::min<uint64_t>(16384, (n_amps + 8 * kBlock - 1) / (8 * kBlock));
+  hipLaunchKernelGGL(k_math_add<R>, dim3((unsigned)grid), dim3(kBlock), 0, s, src, dst, n_amps, A);
+  QS_HIP(hipGetLastError());
+}
+
+template <typename R>
 void math_tile(amp_t<R> *psi, uint64_t n_amps, const MathGather &G, const MathTile &T, hipStream_t s) {
   const uint64_t n_tiles = uint64_t(1) << T.outside;
   if (T.m > (sizeof(R) == 4 ? kMathTileBits64 : kMathTileBits128) || (n_tiles << T.m) > n_amps)
@@ -211,6 +243,8 @@ void math_tile(amp_t<R> *psi, uint64_t n_amps, const MathGather &G, const MathTi
 
 template void math_gather<float>(const float2 *, float2 *, uint64_t, const MathGather &, hipStream_t);
 template void math_gather<double>(const double2 *, double2 *, uint64_t, const MathGather &, hipStream_t);
+template void math_add<float>(const float2 *, float2 *, uint64_t, const MathAdd &, hipStream_t);
+template void math_add<double>(const double2 *, double2 *, uint64_t, const MathAdd &, hipStream_t);
 template void math_tile<float>(float2 *, uint64_t, const MathGather &, const MathTile &, hipStream_t);
 template void math_tile<double>(double2 *, uint64_t, const MathGather &, const MathTile &, hipStream_t);
 

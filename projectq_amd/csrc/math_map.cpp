@@ -141,6 +141,27 @@ bool plan_math_gather(int opcode, int64_t a, int64_t N, const std::vector<std::v
   return true;
 }
 
+bool plan_math_add(const MathGather &G, MathAdd *out) {
+  MathAdd &A = *out;
+  A = MathAdd{};
+  if (G.source != kSrcAddConstant) return false;
+  A.n_regs = G.n_regs;
+  A.cmask = G.cmask;
+  for (int r = 0; r < G.n_regs; ++r) {
+    std::vector<unsigned> at(G.width[r]);
+    for (uint32_t b = 0; b < G.width[r]; ++b) at[b] = (unsigned)__builtin_ctzll(scatter_bits(uint64_t(1) << b, G.reg[r]));
+    const bool up = std::is_sorted(at.begin(), at.end()), down = std::is_sorted(at.rbegin(), at.rend());
+    if (!up && !down) return false;
+    if (!up) A.reversed |= 1u << r;
+    for (uint32_t b = 0; b < G.width[r]; ++b) {
+      const uint64_t bit = uint64_t(1) << (up ? at[b] : 63 - at[b]);
+      A.mask[r] |= bit;
+      if ((G.a >> b) & 1) A.sub[r] |= bit;
+    }
+  }
+  return true;
+}
+
 bool plan_math_tile(const MathGather &G, unsigned n, bool c64, MathTile *out) {
   MathTile &T = *out;
   T = MathTile{};

@@ -97,6 +97,39 @@ struct MathTile {
 constexpr unsigned kMathTileBits64 = 12, kMathTileBits128 = 11;  // 32 KiB
 bool plan_math_tile(const MathGather &G, unsigned n, bool c64, MathTile *out);
 
+// x -> x + a on registers whose qubits ascend or descend in position.  The subtraction that finds the source runs on
+// the register's bits where they are: with zeros between them a borrow passes through the gaps.  A descending
+// register ascends in the index read backwards.
+struct MathAdd {
+  int32_t n_regs;
+  uint32_t reversed;  // bit r: register r descends
+  uint64_t cmask;
+  uint64_t mask[3], sub[3];  // the register's bits, and a on them (of the index read backwards where reversed)
+};
+bool plan_math_add(const MathGather &G, MathAdd *out);
+
+QS_HD inline uint64_t reverse_bits(uint64_t v) {
+#ifdef __HIPCC__
+  return __builtin_bitreverse64(v);
+#else
+  uint64_t r = 0;
+  for (int b = 0; b < 64; ++b) r |= ((v >> b) & 1) << (63 - b);
+  return r;
+#endif
+}
+QS_HD inline uint64_t add_source(const MathAdd &A, uint64_t i) {
+  if ((i & A.cmask) != A.cmask) return i;
+  uint64_t s = i;
+  for (int r = 0; r < 3; ++r) {
+    if (r >= A.n_regs) break;
+    const bool back = (A.reversed >> r) & 1;
+    uint64_t t = back ? reverse_bits(s) : s;
+    t = (t & ~A.mask[r]) | (((t & A.mask[r]) - A.sub[r]) & A.mask[r]);
+    s = back ? reverse_bits(t) : t;
+  }
+  return s;
+}
+
 // Source values (u, v, w) of one destination under the rule S = G.source; returns false where there is
 // no source (modulo N only).
 template <int S>
