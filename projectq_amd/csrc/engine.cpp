@@ -1367,16 +1367,23 @@ struct Engine::SumUpload {
   void *own = nullptr;
   SumUpload(Engine &engine, const SumPlan &plan) : e(engine) {
     const size_t groups = plan.groups.size() * sizeof(SumGroup), strings = plan.strings.size() * sizeof(EnergyString);
-    if (groups + strings == 0) return;
-    std::vector<char> host(groups + strings);
-    std::memcpy(host.data(), plan.groups.data(), groups);
-    std::memcpy(host.data() + groups, plan.strings.data(), strings);
+    const size_t bytes = groups + strings;
+    if (bytes == 0) return;
+    auto fill = [&](char *to) {
+      std::memcpy(to, plan.groups.data(), groups);
+      if (strings) std::memcpy(to + groups, plan.strings.data(), strings);
+    };
     const char *d;
-    if (host.size() <= kArenaBytes / 4) {
-      d = (const char *)e.upload(host.data(), host.size());
+    if (bytes <= kArenaBytes / 4) {
+      char *host;
+      d = e.reserve(bytes, &host);
+      fill(host);
+      QS_HIP(hipMemcpyAsync((void *)d, host, bytes, hipMemcpyHostToDevice, e.stream_));
     } else {
-      QS_HIP(hipMalloc(&own, host.size()));
-      const hipError_t err = hipMemcpy(own, host.data(), host.size(), hipMemcpyHostToDevice);
+      std::vector<char> host(bytes);
+      fill(host.data());
+      QS_HIP(hipMalloc(&own, bytes));
+      const hipError_t err = hipMemcpy(own, host.data(), bytes, hipMemcpyHostToDevice);
       if (err != hipSuccess) (void)hipFree(own);
       QS_HIP(err);
       d = (const char *)own;
@@ -1403,15 +1410,22 @@ void Engine::apply_qubit_operator(const std::vector<PauliString> &terms, const s
     pauli_encode(terms[t], ids, &st[t].x, &st[t].z, &w);
     st[t].c = coeffs[t] * w;
   }
-  SumPlan plan;
-  plan_sum(st, n_, c64_, plan);
-  SumUpload up(*this, plan);
   void *dst = scratch(0);
-  dispatch([&](auto tag) {
-    using R = decltype(tag);
-    dev::pauli_sum<R>((const amp_t<R> *)psi_, (amp_t<R> *)dst, nullptr, n_, plan, up.rec, 1.0, false, 1.0, 0, nullptr,
-                      d_partials_, stream_);
-  });
+  if (dev::pauli_few(st, n_)) {
+    dispatch([&](auto tag) {
+      using R = decltype(tag);
+      dev::pauli_map<R>((const amp_t<R> *)psi_, (amp_t<R> *)dst, amps(), st, stream_);
+    });
+  } else {
+    SumPlan plan;
+    plan_sum(st, n_, c64_, plan);
+    SumUpload up(*this, plan);
+    dispatch([&](auto tag) {
+      using R = decltype(tag);
+      dev::pauli_sum<R>((const amp_t<R> *)psi_, (amp_t<R> *)dst, nullptr, n_, plan, up.rec, 1.0, false, 1.0, 0, nullptr,
+                        d_partials_, stream_);
+    });
+  }
   std::swap(psi_, buf_[0]);
   norm_changed();
   subspace_unknown();

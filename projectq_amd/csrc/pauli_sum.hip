@@ -179,6 +179,51 @@ __global__ __launch_bounds__(kBlock) void k_pauli_sum(const amp_t<R> *__restrict
   }
 }
 
+// Operators that need no tile (pauli_few): every amplitude reads its partners, from memory once where there is
+// one x, from the caches on small states.  The tiles above cost them their upload, two barriers and a second read:
+// 20 strings on 14 qubits 68 us through a tile, 55 here (62 with the same loop behind an upload); one string on 24 qubits
+// complex64 90 and 67.  NJ amplitudes per thread: 1 on small states and for complex64 (4: 25 qubits 114 -> 132 us),
+// 4 for complex128 (26 qubits 486 -> 406).
+constexpr int kFewTerms = 64, kFewBits = 18;
+struct FewTerms {
+  uint64_t x[kFewTerms], z[kFewTerms];
+  double re[kFewTerms], im[kFewTerms];
+  uint32_t n;
+};
+template <typename R, int NJ>
+__global__ __launch_bounds__(kBlock) void k_pauli_map(const amp_t<R> *__restrict__ src, amp_t<R> *__restrict__ dst,
+                                                      uint64_t n_amps, FewTerms t) {
+  for (uint64_t first = (uint64_t)blockIdx.x * kBlock * NJ + threadIdx.x; first < n_amps; first += (uint64_t)gridDim.x * kBlock * NJ) {
+    double ur[NJ], ui[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) ur[j] = ui[j] = 0.0;
+#pragma unroll 4
+    for (uint32_t k = 0; k < t.n; ++k) {
+      amp_t<R> b[NJ];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        b[j].x = b[j].y = 0;
+        if (first + j * kBlock < n_amps) b[j] = src[(first + j * kBlock) ^ t.x[k]];
+      }
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const uint32_t odd = (uint32_t)__popcll(((first + j * kBlock) ^ t.x[k]) & t.z[k]) & 1u;
+        const double br = flip(b[j].x, odd), bi = flip(b[j].y, odd);
+        ur[j] += br * t.re[k] - bi * t.im[k];
+        ui[j] += br * t.im[k] + bi * t.re[k];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      if (first + j * kBlock >= n_amps) continue;
+      amp_t<R> d;
+      d.x = (R)ur[j];
+      d.y = (R)ui[j];
+      dst[first + j * kBlock] = d;
+    }
+  }
+}
+
 // A launch of its own (5 us): the last workgroup of the term doing this behind an agent-scope counter
 // made every workgroup write back and invalidate its L2, and the term twice as long.
 __global__ __launch_bounds__(kBlock) void k_evolve_check(const double *__restrict__ partials, uint32_t n,
@@ -255,6 +300,32 @@ void pauli_sum(const amp_t<R> *src, amp_t<R> *dst, amp_t<R> *out, unsigned n, co
   QS_HIP(hipGetLastError());
 }
 
+bool pauli_few(const std::vector<SumTerm> &terms, unsigned n) {
+  if (terms.empty() || terms.size() > (size_t)kFewTerms) return false;
+  if (n <= (unsigned)kFewBits) return true;
+  return terms.size() == 1 || (terms.size() == 2 && (n <= kFewBits + 2 || terms[0].x == terms[1].x));
+}
+
+template <typename R>
+void pauli_map(const amp_t<R> *src, amp_t<R> *dst, uint64_t n_amps, const std::vector<SumTerm> &terms, hipStream_t s) {
+  FewTerms t;
+  t.n = (uint32_t)terms.size();
+  for (uint32_t k = 0; k < t.n; ++k) {
+    t.x[k] = terms[k].x;
+    t.z[k] = terms[k].z;
+    t.re[k] = terms[k].c.real();
+    t.im[k] = terms[k].c.imag();
+  }
+  auto go = [&](auto nj) {
+    constexpr int NJ = decltype(nj)::value;
+    const uint64_t grid = std::min<uint64_t>(16384, (n_amps + NJ * kBlock - 1) / (NJ * kBlock));
+    hipLaunchKernelGGL((k_pauli_map<R, NJ>), dim3((unsigned)grid), dim3(kBlock), 0, s, src, dst, n_amps, t);
+    QS_HIP(hipGetLastError());
+  };
+  if (sizeof(R) == 8 && n_amps > (uint64_t(1) << (kFewBits + 2))) go(std::integral_constant<int, 4>{});
+  else go(std::integral_constant<int, 1>{});
+}
+
 void evolve_check(const double *partials, unsigned n, const SumPlan &plan, EvolveState *state, EvolveState *host, hipStream_t s) {
   hipLaunchKernelGGL(k_evolve_check, dim3(1), dim3(kBlock), 0, s, partials, workgroups(n, plan), state, host);
   QS_HIP(hipGetLastError());
@@ -265,6 +336,8 @@ void evolve_reset(EvolveState *state, hipStream_t s) {
   QS_HIP(hipGetLastError());
 }
 
+template void pauli_map<float>(const float2 *, float2 *, uint64_t, const std::vector<SumTerm> &, hipStream_t);
+template void pauli_map<double>(const double2 *, double2 *, uint64_t, const std::vector<SumTerm> &, hipStream_t);
 template void pauli_sum<float>(const float2 *, float2 *, float2 *, unsigned, const SumPlan &, const SumRecords &,
                                std::complex<double>, bool, std::complex<double>, uint64_t, const EvolveState *, double *,
                                hipStream_t);

@@ -28,6 +28,11 @@ template <typename R>
 void pauli_sum(const amp_t<R> *src, amp_t<R> *dst, amp_t<R> *out, unsigned n, const SumPlan &plan, const SumRecords &rec,
                std::complex<double> f, bool first, std::complex<double> g, uint64_t cmask, const EvolveState *evolve,
                double *partials, hipStream_t s);
+// Operators that need no tile: a few strings on a small state, one or two strings with one x on any.  The terms
+// travel in the kernel arguments.
+bool pauli_few(const std::vector<SumTerm> &terms, unsigned n);
+template <typename R>
+void pauli_map(const amp_t<R> *src, amp_t<R> *dst, uint64_t n_amps, const std::vector<SumTerm> &terms, hipStream_t s);
 // state->terms += 1, state->done <- the norm of the last term is at most 1e-12; mirrored to `host`
 // (pinned).  Does nothing once done.
 void evolve_check(const double *partials, unsigned n, const SumPlan &plan, EvolveState *state, EvolveState *host, hipStream_t s);

@@ -97,3 +97,24 @@ def test_gpu_operator_too_large_for_the_arena():
     for sim in sims:
         sim.apply_qubit_operator(terms, [0, 1, 2, 3])
     assert np.max(np.abs(sims[0].cheat_numpy()[1] - sims[1].cheat_numpy()[1])) <= 1e-12
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", ["c128", "c64"])
+@pytest.mark.parametrize("n,count,one_x", [(1, 1, False), (7, 64, False), (7, 65, False), (18, 20, False), (18, 65, False),
+                                           (19, 3, False), (20, 2, False), (21, 1, False), (21, 2, True), (21, 2, False)])
+def test_gpu_operator_routes(precision, n, count, one_x):
+    """With and without tiles, at the edges of both: strings 64 and 65, qubits 18 to 21, one x and two.  The
+    coefficients add up to 1, so amplitudes stay below 1 and a string rounds each a few times."""
+    sims = simulators(n, precision, n + count)
+    rng = np.random.default_rng(n * count)
+    terms = []
+    for t in range(count):
+        ops = [(int(q), "XYZ"[int(o)]) for q, o in zip(range(n), rng.integers(0, 3, size=n))]
+        if one_x:
+            ops = [(q, "X") for q in range(0, n, 2)] + [(q, "Z") for q in range(1, n, 2) if t or q % 4 == 1]
+        terms.append((ops, complex(np.exp(1j * t)) / count))
+    for sim in sims:
+        sim.apply_qubit_operator(terms, list(range(n)))
+    eps = 2.0 ** -53 if precision == "c128" else 2.0 ** -24
+    assert np.max(np.abs(sims[0].cheat_numpy()[1] - sims[1].cheat_numpy()[1])) <= 8 * (count * 2.0 ** -53 + eps)
