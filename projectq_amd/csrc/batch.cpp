@@ -205,6 +205,7 @@ void Batch::build(const BatchShape &shape) {
   constexpr int kXcds = 8;
   constexpr uint64_t kBatchWorkgroups = 8;  // per circuit at least: 100 strings in one workgroup take 40 us
   constexpr uint32_t kSmallest = 8, kSizes = 5;  // tiles of 2^8 .. 2^12 amplitudes
+  constexpr size_t kOwnLaunch = 1024;            // workgroups, four per CU
   // Workgroup w runs on XCD w mod 8.  Every circuit goes whole to one XCD (largest first, to the
   // least loaded), so the later passes over its state hit that XCD's L2; the XCDs' workgroup lists are
   // interleaved and padded with idle workgroups to equal length.
@@ -271,14 +272,29 @@ void Batch::build(const BatchShape &shape) {
     list.insert(list.end(), of_circuit[c].begin(), of_circuit[c].end());
   }
   std::vector<dev::BatchEnergyBlock> eblock;
-  for (uint32_t s = kSizes; s-- > 0;) {  // the largest first
+  auto launch = [&](uint32_t t, const std::vector<std::vector<dev::BatchEnergyBlock>> &lists) {
     size_t longest = 0;
-    for (auto &v : per_xcd[s]) longest = std::max(longest, v.size());
-    if (longest == 0) continue;
-    energy_launches_.push_back({kSmallest + s, (uint32_t)eblock.size(), (uint32_t)(longest * kXcds)});
+    for (auto &v : lists) longest = std::max(longest, v.size());
+    if (longest == 0) return;
+    energy_launches_.push_back({t, (uint32_t)eblock.size(), (uint32_t)(longest * kXcds)});
     for (size_t k = 0; k < longest; ++k)
-      for (int x = 0; x < kXcds; ++x)
-        eblock.push_back(k < per_xcd[s][x].size() ? per_xcd[s][x][k] : dev::BatchEnergyBlock{dev::kNoPass, 0, 0, 0});
+      for (int x = 0; x < kXcds; ++x) eblock.push_back(k < lists[x].size() ? lists[x][k] : dev::BatchEnergyBlock{dev::kNoPass, 0, 0, 0});
+  };
+  // the largest first; sizes that do not fill the chip go together
+  std::vector<uint32_t> small;
+  for (uint32_t s = kSizes; s-- > 0;) {
+    size_t count = 0;
+    for (auto &v : per_xcd[s]) count += v.size();
+    if (count >= kOwnLaunch) launch(kSmallest + s, per_xcd[s]);
+    else if (count > 0) small.push_back(s);
+  }
+  if (small.size() == 1) {
+    launch(kSmallest + small[0], per_xcd[small[0]]);
+  } else {
+    std::vector<std::vector<dev::BatchEnergyBlock>> mixed(kXcds);
+    for (uint32_t s : small)
+      for (int x = 0; x < kXcds; ++x) mixed[x].insert(mixed[x].end(), per_xcd[s][x].begin(), per_xcd[s][x].end());
+    launch(dev::kMixedTiles, mixed);
   }
   // ---- device buffers
   const size_t ab = c64_ ? 8 : 16;

@@ -31,7 +31,8 @@ constexpr uint32_t kNoPass = 0xffffffffu;
 struct BatchEnergyBlock {
   uint32_t pass, tile, tiles, slot;
 };
-// partials of the workgroups, all of whose passes have tiles of 2^t amplitudes
+// partials of the workgroups, all of whose passes have tiles of 2^t amplitudes, or of any size (kMixedTiles)
+constexpr uint32_t kMixedTiles = 0;
 template <typename R>
 void batch_energy(const amp_t<R> *psi, uint32_t t, const BatchEnergyPass *passes, const BatchEnergyBlock *blocks,
                   uint32_t n_blocks, const EnergyGroup *groups, const EnergyString *strings, double *partials, hipStream_t s);

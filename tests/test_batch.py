@@ -94,3 +94,18 @@ def test_batch_shapes_agree():
         finally:
             del os.environ["PROJECTQ_AMD_BATCH_SHAPE"]
     assert relabelled >= 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", ["c64", "c128"])
+@pytest.mark.parametrize("sizes,strings", [([1, 4, 8], 2), ([8, 9, 10, 11, 12, 13], 1), ([12] * 20 + [15, 16, 9, 10, 3], 40)])
+def test_energies_of_every_tile_size(sizes, strings, precision):
+    """Tiles of 2^8 to 2^12 amplitudes in one launch (few workgroups), and one size filling a launch of its own."""
+    from projectq_amd.batch import BatchExpectation
+
+    circ, ops = make_batch(sizes, 51)
+    ops = [circuits.random_pauli_operator(n, strings, 70 + i) for i, n in enumerate(sizes)]
+    want, _ = OracleBatch(circ, ops).run()
+    scale = np.array([sum(abs(c) for _, c in terms) for terms in ops])
+    got, _ = BatchExpectation(circ, ops, precision=precision, autotune=False).run()
+    assert np.max(np.abs(got - want) / scale) <= (1e-12 if precision == "c128" else 2e-5)
