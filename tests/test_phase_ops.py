@@ -113,3 +113,24 @@ def test_kernels_run_phases(n, precision, kind, mode):
     eps = 2.0 ** -24 if precision == "c64" else 2.0 ** -53
     # rounding is relative to an amplitude, the largest about 5 times 2^(-n/2)
     assert np.max(np.abs(np.array(sim.cheat_numpy()[1]) - _oracle(n, gates, psi))) <= 8 * len(gates) * eps * 5 * 2.0 ** (-n / 2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["qft", "diagonal"])
+@pytest.mark.parametrize("lmin", [4, 5])
+def test_kernel_of_512_threads_runs_phases(lmin, kind):
+    """complex64 tiles of 2^13 amplitudes, which take 21 qubits: the tolerance as above."""
+    from projectq_amd import Simulator
+
+    n = 21
+    gates = _circuit(n, kind, n + lmin)
+    psi = _state(n, 7)
+    sim = Simulator(1, precision="c64", capacity_qubits=n, fusion="window", planner="tile")
+    sim.set_tile_params(13, 4, lmin)
+    for q in range(n):
+        sim.allocate_qubit(q)
+    sim.set_wavefunction(psi, list(range(n)))
+    commands.execute(sim, [("gate", m, tuple(t), tuple(c)) for m, t, c in gates], gate_fusion=True)
+    sim.run()
+    assert sim.last_plan()["tile_bits"] == 13
+    assert np.max(np.abs(np.array(sim.cheat_numpy()[1]) - _oracle(n, gates, psi))) <= 8 * len(gates) * 2.0 ** -24 * 5 * 2.0 ** (-n / 2)
