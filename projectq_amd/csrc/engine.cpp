@@ -30,14 +30,6 @@ BitInsert make_insert(std::vector<uint32_t> positions) {
   return ins;
 }
 
-uint64_t insert_zeros_host(uint64_t g, const BitInsert &ins) {
-  for (uint32_t i = 0; i < ins.count; ++i) {
-    const uint32_t p = ins.pos[i];
-    g = ((g >> p) << (p + 1)) | (g & ((uint64_t(1) << p) - 1));
-  }
-  return g;
-}
-
 std::vector<uint32_t> bits_of(uint64_t mask) {
   std::vector<uint32_t> out;
   for (uint32_t p = 0; p < 64; ++p)
@@ -1624,7 +1616,7 @@ void Engine::cheat(uint32_t *ids, uint32_t *positions, double *state) {
 
 
 // The state stays where it is: the pointer is valid until the next call on this simulator that
-// applies gates, allocates or frees qubits (those may move the state to the other buffer).
+// applies gates, allocates or frees qubits (those may move the state to the other buffer), or measures.
 void Engine::device_state(void **ptr, uint64_t *n_amps, int *precision) {
   canonicalize();
   sync();

@@ -578,26 +578,12 @@ __device__ __forceinline__ void tile_put16(uint32_t addr, const typename Vec16<R
     lds_store<typename Vec16<R>::type>(addr, v);
   }
 }
-// The same read when the stored tile relabels qubits: the pair (l, l + 1) of the stored tile comes
+// The read of a 16-byte vector for the store, which may relabel qubits: the pair (l, l + 1) of the stored tile comes
 // from computed-tile slots addr and addr ^ pair (pair = the slot bytes of the partner's bit).
 template <typename R>
 __device__ __forceinline__ typename Vec16<R>::type tile_get16p(uint32_t addr, uint32_t pair) {
   if constexpr (sizeof(R) == 4) {
     const re2_t<float> a = lds_load<re2_t<float>>(addr), b = lds_load<re2_t<float>>(addr ^ pair);
-    typename Vec16<R>::type v;
-    v.x = a.x;
-    v.y = a.y;
-    v.z = b.x;
-    v.w = b.y;
-    return v;
-  } else {
-    return lds_load<typename Vec16<R>::type>(addr);
-  }
-}
-template <typename R>
-__device__ __forceinline__ typename Vec16<R>::type tile_get16(uint32_t addr) {
-  if constexpr (sizeof(R) == 4) {
-    const re2_t<float> a = lds_load<re2_t<float>>(addr), b = lds_load<re2_t<float>>(addr ^ 8u);
     typename Vec16<R>::type v;
     v.x = a.x;
     v.y = a.y;
