@@ -341,8 +341,10 @@ std::vector<uint8_t> Engine::measure_qubits(const std::vector<unsigned> &ids) {
   a.sval = zval_;
   a.zmask = zmask_;
   a.mask = mask_of(ids);
-  a.kept = free_runs(zmask_ | a.mask);
-  a.n_kept = a.n_amps >> __builtin_popcountll(zmask_ | a.mask);
+  if (a.n_sub > dev::kMeasureSmall && ids.size() != 1) {  // one qubit: the chunk sums hold its norms
+    a.kept = free_runs(zmask_ | a.mask);
+    a.n_kept = a.n_amps >> __builtin_popcountll(zmask_ | a.mask);
+  }
   if (a.n_sub > dev::kMeasureSmall && !d_sums_) QS_HIP(hipMalloc(&d_sums_, 2 * dev::kMeasureChunks * sizeof(double)));
   dispatch([&](auto tag) {
     using R = decltype(tag);
@@ -460,13 +462,14 @@ void Engine::exec_blocks() {
     drift += b.drift;
     nonunitary |= b.nonunitary;
   }
-  bool tiles = ends_.size() > 2;
+  bool tiles = ends_.size() > 2, wide = false;
   for (size_t i = 0; i < count && tiles; ++i) {
     const Gate &g = window_[i];
     const uint64_t seen = mask_of(g.ids);
+    wide |= g.ids.size() > 3;
     tiles = !g.ids.empty() && (size_t)__builtin_popcountll(seen) == g.ids.size() && !(seen & mask_of(g.ctrl));
   }
-  tiles = tiles && !blocks_faster(count);
+  tiles = tiles && !(wide && blocks_faster(count));
   std::vector<TileProgram> progs;
   if (tiles) {  // planned before the queue is touched: where planning fails, nothing has run and nothing is lost
     unsigned t;
@@ -506,7 +509,6 @@ void Engine::exec_blocks() {
 bool Engine::blocks_faster(size_t count) const {
   size_t wide[6] = {};
   for (size_t i = 0; i < count; ++i) ++wide[std::min<size_t>(window_[i].ids.size(), 5)];
-  if (wide[4] + wide[5] == 0) return false;
   const double n = (double)amps(), bytes = (double)amp_bytes() * n, stream = 2.0 * bytes / 3.3e6;
   const double in_cache = bytes <= (double)(256u << 20) ? 0.67 : 1.0;
   double blocks = 0.0;

@@ -24,7 +24,7 @@ struct MeasureArgs {
   BitRuns free;            // the subspace's free bits: compact index -> index
   uint64_t sval, zmask;    // the values of the fixed bits, and their mask
   uint64_t mask;           // index bits of the measured qubits
-  uint64_t n_kept;         // amplitudes of the subspace with one outcome of them
+  uint64_t n_kept;         // of another number of qubits than one: amplitudes of the subspace with one outcome of them
   BitRuns kept;            // their free bits
   double rnd;              // the draw; 0: the reference's loop never runs and the pick is all ones
 };
