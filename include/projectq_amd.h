@@ -231,7 +231,7 @@ int qs_take_records(qs_simulator *sim, float *features, float *ms, size_t cap, s
  * uses; without a model the learned planner falls back to greedy max-5 blocks. */
 int qs_set_planner_model(qs_simulator *sim, const float *weights, size_t n_weights);
 /* The last window's plan: kind (0 greedy blocks, 1 tile passes), tile shape, passes, number of
- * candidate plans compared and the model's predicted time (ms). */
+ * candidate plans compared and the model's predicted time (ms; 0 where no plan was scored). */
 int qs_last_plan(qs_simulator *sim, int *kind, uint32_t *tile_bits, uint32_t *reg_bits,
                  uint32_t *low_bits, uint32_t *passes, uint32_t *candidates, double *predicted_ms);
 /* The MLP (24 -> 64 -> 64 -> 1, ReLU, fp32) on the GPU: weight count, inference, loss and
