@@ -406,13 +406,11 @@ void Engine::apply_controlled_gate(Gate g) {
   trial.insert(g);
   const unsigned now = trial.num_qubits();
   const bool full = now >= 4 && now <= 5;
-  if (!full && (now > 5 || (size_t)(now - g.ids.size()) > (size_t)before)) {
-    close_block();
-    open_.insert(g);
-  } else {
-    open_ = std::move(trial);
-  }
+  const bool next = !full && (now > 5 || (size_t)(now - g.ids.size()) > (size_t)before);
+  if (next) close_block();
   if (nonunitary) exec_blocks();  // the norm guard looks at what is complete without it
+  if (next) open_.insert(g);
+  else open_ = std::move(trial);
   queued();
   window_.push_back(std::move(g));
   if (full) close_block();
