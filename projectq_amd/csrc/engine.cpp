@@ -170,6 +170,15 @@ void *Engine::scratch(int which) {
   return buf_[which];
 }
 
+// Scratch buffer 0, null where it cannot be allocated.
+void *Engine::try_scratch() {
+  if (!buf_[0] && hipMalloc(&buf_[0], cap_ * amp_bytes()) != hipSuccess) {
+    (void)hipGetLastError();  // clear the failed allocation's error state
+    buf_[0] = nullptr;
+  }
+  return buf_[0];
+}
+
 // Space for `bytes` in the arena: the device address, and the pinned address to fill and copy from.
 char *Engine::reserve(size_t bytes, char **host) {
   const size_t need = (bytes + 255) & ~size_t(255);
@@ -697,13 +706,7 @@ void Engine::restore_layout(double scale) {
 void Engine::canonicalize() {
   run();
   if (pos_ == ref_pos_) return;
-  void *dst = buf_[0];
-  if (!dst && hipMalloc(&dst, cap_ * amp_bytes()) != hipSuccess) {
-    (void)hipGetLastError();  // clear the failed allocation's error state
-    dst = nullptr;
-  }
-  if (dst) {
-    buf_[0] = dst;
+  if (try_scratch()) {
     restore_layout(1.0);
     sync();
     return;
@@ -1223,7 +1226,8 @@ void Engine::emulate_math_op(int opcode, const std::vector<int64_t> &params,
     // In place where the changing bits fit an LDS tile: less traffic under controls, and no scratch.
     MathTile tile;
     MathAdd add;
-    bool in_tiles = plan_math_tile(g, n_, c64_, &tile);
+    const bool fits = plan_math_tile(g, n_, c64_, &tile);
+    bool in_tiles = fits;
     const bool adds = plan_math_add(g, &add);
     if (opcode == 0) {
       // An addition of a constant needs no pass for collisions on any path, so the others have to beat the general
@@ -1238,6 +1242,7 @@ void Engine::emulate_math_op(int opcode, const std::vector<int64_t> &params,
       }
       if (adds) in_tiles = in_tiles && amps() * amp_bytes() >= (uint64_t(32) << 20) && (tile.fixed || (c64_ && g.cmask));
       else in_tiles = in_tiles && (c64_ || tile.fixed);
+      in_tiles = in_tiles || (fits && !try_scratch());
     }
     if (in_tiles) {
       dispatch([&](auto tag) {

@@ -115,6 +115,7 @@ class Engine {
   uint64_t amps() const { return uint64_t(1) << n_; }
   void ensure_capacity(uint64_t need_amps);
   void *scratch(int which);  // full-capacity scratch buffer 0 or 1 (lazy)
+  void *try_scratch();
   void release_scratch();
   char *reserve(size_t bytes, char **host);
   const void *upload(const void *host, size_t bytes);
