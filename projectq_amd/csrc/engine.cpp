@@ -579,22 +579,25 @@ void Engine::after_passes(double drift, bool nonunitary) {
 std::vector<Block> Engine::greedy_blocks(const std::vector<Gate> &gates) const {
   std::vector<Block> out;
   GateQueue q;
+  BlockQubits open;  // decides without the matrices: trying a gate of many controls on them would widen all of them
+  auto close = [&] {
+    if (!q.empty()) out.push_back(q.fuse());
+    q.clear();
+    open.clear();
+  };
   for (const Gate &g : gates) {
-    GateQueue trial = q;
+    BlockQubits trial = open;
     trial.insert(g);
-    const unsigned now = trial.num_qubits(), before = q.num_qubits();
-    if (now >= 4 && now <= 5) {
-      out.push_back(trial.fuse());
-      q.clear();
-    } else if (now > 5 || (size_t)(now - g.ids.size()) > (size_t)before) {
-      if (!q.empty()) out.push_back(q.fuse());
-      q.clear();
-      q.insert(g);
-    } else {
-      q = std::move(trial);
-    }
+    const unsigned now = trial.num_qubits(), before = open.num_qubits();
+    const bool full = now >= 4 && now <= 5;
+    const bool next = !full && (now > 5 || (size_t)(now - g.ids.size()) > (size_t)before);
+    if (next) close();
+    q.insert(g);
+    if (next) open.insert(g);
+    else open = std::move(trial);
+    if (full) close();
   }
-  if (!q.empty()) out.push_back(q.fuse());
+  close();
   return out;
 }
 

@@ -137,3 +137,24 @@ def test_wide_gates_take_the_faster_way(n, k, precision, blocks):
     passes = sim.stats()["passes"]
     assert passes == count if blocks else passes < count
     assert np.max(np.abs(_amplitudes(sim) - _amplitudes(ref))) <= 8 * (1 << k) * count * EPS[precision]
+
+
+@pytest.mark.parametrize("precision", ["c64", "c128"])
+def test_greedy_window_with_many_controls(precision):
+    """A gate of 19 controls behind others: the block it does not fit is closed without building the matrix of
+    both."""
+    from projectq_amd import Simulator
+
+    n = 20
+    z = np.diag([1, -1]).astype(complex)
+    sim, ref = Simulator(3, precision=precision, capacity_qubits=n, fusion="window", planner="greedy"), OracleSimulator(3)
+    gates = [(H, [q], []) for q in range(n)] + [(z, [0], list(range(1, n)))] + [(H, [q], []) for q in range(n)]
+    for s in (sim, ref):
+        for q in range(n):
+            s.allocate_qubit(q)
+    for m, t, c in gates:
+        sim.apply_controlled_gate(m, t, c)
+        ref.apply_controlled_gate(m, t, c)
+        ref.run()
+    sim.run()
+    assert np.max(np.abs(_amplitudes(sim) - _amplitudes(ref))) <= 8 * len(gates) * EPS[precision]
