@@ -93,7 +93,9 @@ __global__ __launch_bounds__(kBlock) void k_math_gather(const amp_t<R> *__restri
 }
 
 // Additions of a constant (MathAdd): a source costs a few operations however its bits lie, so the destinations
-// go in memory order with eight loads in flight per thread.
+// go in memory order with eight loads in flight per thread.  Bound by HBM on large states: 27 qubits complex64, all in
+// one register, 0.42 ms (5.1 TB/s; 0.58 by k_math_gather); by the launch on small ones: 16 qubits in descending
+// order 24 us (55 by the gather's loop over 16 runs of bits).
 template <typename R>
 __global__ __launch_bounds__(kBlock) void k_math_add(const amp_t<R> *__restrict__ src, amp_t<R> *__restrict__ dst,
                                                      uint64_t n_amps, MathAdd A) {
